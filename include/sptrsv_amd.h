@@ -277,12 +277,19 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * in-degree walk (SIMPLE/ORDER, one right-hand side): each row waits on a
  * counter of its unsolved dependencies, which solved rows decrement through
  * the column pattern, then folds its entries exactly as variant 1 does (same
- * results, bit for bit); cu_waves caps the waves
+ * results, bit for bit); 4 is the level walk (ORDER/MULTIROW, one right-hand
+ * side): one workgroup solves level by level with the results exchanged in
+ * LDS, from a plan that is made on first use for the matrix and analysis (20
+ * bytes for each of 64 * 5 slots per group of up to 64 rows of a level,
+ * released with either; the lean path runs instead while a stream is captured
+ * before the plan exists, while a trace is taken, and where no plan can be
+ * made); cu_waves caps the waves
  * resident per CU (0 = hardware limit): every resident wave polls, and past a
  * few thousand polling waves the dependency hand-off latency grows several
  * fold, so deep dependency chains run fastest with a small cap.  With lanes
  * = 0 the lanes (and, when variant is 0, the variant) come from the tuned
- * shape of the kernel, else from the default shape; MULTIROW takes its lanes
+ * shape of the kernel, else from the default shape (the level walk where a
+ * level's share of the matrix is small, else the lean path); MULTIROW takes its lanes
  * per row from the analysis and ignores a nonzero lanes. */
 typedef struct {
     int kernel;
@@ -363,9 +370,9 @@ int csr_L_solve_mixed(sp_mat_t* mat, dfr_analysis_info_t* info, const double* b,
  * (allocate_memory_upper, or the transpose of a lower-triangular handle), the
  * in-degree walk (variant 3) and a named level-ordered copy (reorder = 1).
  * An automatic call (cfg NULL or kernel AUTO) takes the tuned shape, with
- * two substitutions: a tuned JACOBI choice becomes the default sync-free
- * shape, and a tuned level-ordered copy walks the matrix as given (same
- * bits).
+ * three substitutions: a tuned JACOBI choice becomes the default sync-free
+ * shape, a tuned level-ordered copy walks the matrix as given (same bits), and
+ * the level walk (whose plan is a workspace) becomes the lean path.
  * Each call re-initialises the scratch it uses.  Every call on one GPU
  * shares that GPU's scratch, so calls that overlap in time on one GPU (two
  * streams, two threads) race and must be serialised by the caller. */

@@ -410,6 +410,7 @@ void free_info_arrays(dfr_analysis_info_t* info) {
         std::lock_guard<std::mutex> g(g_info_mu);
         g_infos.erase(ip);
     }
+    analysis_freed(ip->id);
     free_segments(ip->seg);
     int* arrays[] = {info->lev_size, info->warp_lev, info->inv_iorder, info->iorder,
                      info->ibase_row, info->ivect_size_warp, info->row_ctr, info->level,

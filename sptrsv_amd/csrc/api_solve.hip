@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "syncfree.hpp"
@@ -76,6 +77,11 @@ int jacobi_solve(sp_mat_t* m, const sptrsv_config_t& c, int k, const double* b, 
 int jacobi_tune(sp_mat_t* m, int k, int reps, sptrsv_config_t* best, float* best_ms);
 int jacobi_margin(sp_mat_t* m, double* delta);
 int reserve_jacobi(sp_mat_t* m, int k);
+// level_walk.hip: *done stays false where the walk cannot be taken
+int level_walk_f64(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed, bool* done);
+int level_walk_f32(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed, bool* done);
+int level_walk_mixed(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed,
+                     bool* done);
 
 // ---- configuration --------------------------------------------------------------
 
@@ -134,14 +140,30 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
     return c;
 }
 
+// The same with the analysis at hand: ORDER and MULTIROW solves with one
+// right-hand side take the level walk where it fits.
+static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
+    sptrsv_config_t c = shape_for(m, kernel, k);
+    if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1 && level_walk_fits(m, info))
+        c.variant = 4;
+    return c;
+}
+
 int default_config(const sp_mat_t* m, const dfr_analysis_info_t* info, int precision, int k,
                    sptrsv_config_t* out) {
     (void)precision;
     int kernel = SPTRSV_KERNEL_SIMPLE;
     if (info && info->mode == ORDER && has_order(info)) kernel = SPTRSV_KERNEL_ORDER;
     if (info && info->mode == MULTIROW && has_waves(info)) kernel = SPTRSV_KERNEL_MULTIROW;
-    *out = shape_for(m, kernel, k);
+    *out = analysed_shape_for(m, info, kernel, k);
     return SPTRSV_OK;
+}
+
+// Whether a call that names a kernel without lanes leaves the rest of the
+// shape open too.
+static bool shape_open(const sptrsv_config_t& c) {
+    return c.variant == 0 && c.wg <= 0 && c.cu_waves <= 0 && c.window == 0 && c.claim_rounds == 0 && c.split_rows == 0 &&
+           c.reorder == 0;
 }
 
 static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision, int k,
@@ -154,7 +176,9 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
             // of the default shape; so is the variant unless one is named
             const sptrsv_config_t& t = pv->tuned_cfg[precision];
             sptrsv_config_t d = (pv->tuned[precision] && pv->tuned_k[precision] == k && t.kernel == cfg->kernel)
-                                    ? t : shape_for(m, cfg->kernel, k);
+                                    ? t
+                                    : shape_open(*cfg) ? analysed_shape_for(m, info, cfg->kernel, k)
+                                                       : shape_for(m, cfg->kernel, k);
             out->lanes = d.lanes;
             if (cfg->variant == 0) out->variant = d.variant;
             if (cfg->wg <= 0) out->wg = d.wg;
@@ -194,7 +218,8 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
     if (K > 1) {
         // several RHS: the general engine, ticketed (256 threads) or
         // persistent (256 or 1024 threads)
-        if (out->kernel != SPTRSV_KERNEL_JACOBI && out->variant != 2 && out->variant != 3) out->variant = 0;
+        if (out->kernel != SPTRSV_KERNEL_JACOBI && out->variant != 2 && out->variant != 3 && out->variant != 4)
+            out->variant = 0;
         if (!(out->variant == 2 && out->wg == 1024)) out->wg = 256;
     }
     if (out->cu_waves < 0) out->cu_waves = 0;
@@ -217,8 +242,12 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
         return fail(SPTRSV_E_INVALID_ARG, "unknown kernel");
     if (out->kernel == SPTRSV_KERNEL_JACOBI && precision != SPTRSV_PREC_MIXED)
         return fail(SPTRSV_E_INVALID_ARG, "JACOBI is the bulk solver of the MIXED path only");
-    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 3))
-        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..3");
+    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 4))
+        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..4");
+    if (out->variant == 4 && out->kernel != SPTRSV_KERNEL_JACOBI &&
+        (K > 1 || out->kernel == SPTRSV_KERNEL_SIMPLE || out->reorder == 1))
+        return fail(SPTRSV_E_INVALID_ARG, "the level walk (variant 4) takes ORDER or MULTIROW, one right-hand side and "
+                                          "the matrix as given");
     if (out->variant == 3 && out->kernel != SPTRSV_KERNEL_JACOBI &&
         (K > 1 || out->kernel == SPTRSV_KERNEL_MULTIROW))
         return fail(SPTRSV_E_INVALID_ARG, "the in-degree walk (variant 3) takes SIMPLE or ORDER and one right-hand side");
@@ -518,10 +547,21 @@ struct LevelView {
 // when given, names a level-ordered copy whose arrays are walked (with the
 // analysis `info` of the copy) while b and x stay in the caller's order.
 template <class P>
-static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_t& c, int k,
+static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_t& cfg, int k,
                     const void* b, void* pub, double* x_out, hipStream_t s, bool timed = true,
                     uint64_t* part_ext = nullptr, const LevelView* lv = nullptr) {
     MatPriv* pv = priv_of(m);
+    sptrsv_config_t c = cfg;
+    if (c.variant == 4) {
+        bool done = false;
+        if (!pv->trace) {  // a trace is written by the walks through memory
+            if constexpr (std::is_same<P, PolF64>::value) SPT_TRY(level_walk_f64(m, info, b, pub, s, timed, &done));
+            if constexpr (std::is_same<P, PolF32>::value) SPT_TRY(level_walk_f32(m, info, b, pub, s, timed, &done));
+            if constexpr (std::is_same<P, PolMixed>::value) SPT_TRY(level_walk_mixed(m, info, b, x_out, s, timed, &done));
+        }
+        if (done) return SPTRSV_OK;
+        c = shape_for(m, c.kernel, k);
+    }
     const sp_mat_t* sm = lv ? lv->mat : m;
     const int K = pow2_ceil(k);
     SolveArgs A{};
@@ -890,6 +930,7 @@ int sptrsv_solve_mixed_noalloc(sp_mat_t* mat, dfr_analysis_info_t* info, const s
         SPT_TRY(default_config(mat, info, SPTRSV_PREC_MIXED, k, &c));
     }
     c.fused = 1;
+    if (c.variant == 4) c = shape_for(mat, c.kernel, k);  // its plan is a per-analysis workspace
     if (c.variant == 3)
         return fail(SPTRSV_E_INVALID_ARG, "the allocation-free solve does not run the in-degree walk (its "
                                           "counters are a per-matrix workspace)");
@@ -1075,6 +1116,9 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
         }
     }
 
+    // level by level in one workgroup, where a level is small
+    if (K == 1 && has_order(info) && level_walk_fits(mat, info)) shapes.push_back({SPTRSV_KERNEL_ORDER, ref, 256, 1, 4, 0});
+
     hipEvent_t e0, e1;
     SPT_HIP(hipEventCreate(&e0));
     SPT_HIP(hipEventCreate(&e1));
@@ -1095,7 +1139,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     // Stage 1: every shape without and with a tight residency cap.
     std::vector<std::pair<float, sptrsv_config_t>> ranked;
     for (auto c : shapes) {
-        for (int cw : (c.variant == 2 ? std::vector<int>{2, 8} : std::vector<int>{0, 4})) {
+        for (int cw : (c.variant == 2 ? std::vector<int>{2, 8} : c.variant == 4 ? std::vector<int>{0} : std::vector<int>{0, 4})) {
             c.cu_waves = cw;
             float t = time_cfg(c);
             if (status != SPTRSV_OK) break;
@@ -1121,6 +1165,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
             }
             if (dup) continue;
             ++taken;
+            if (c.variant == 4) continue;  // one workgroup: nothing to cap
             for (int cw : (c.variant == 2 ? std::vector<int>{1, 3, 4, 6, 12, 16}
                                           : std::vector<int>{32, 16, 8, 2})) {
                 c.cu_waves = cw;
@@ -1135,7 +1180,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     }
     // Stage 3 (long rows): the best shape of each kernel with 16 entries per
     // lane in flight instead of 4, which shortens the load chain of a long row.
-    if (status == SPTRSV_OK && K == 1 && pv->max_row > 64) {
+    if (status == SPTRSV_OK && K == 1 && pv->max_row > 64 && bc.variant != 4) {
         for (int kern : {SPTRSV_KERNEL_SIMPLE, SPTRSV_KERNEL_ORDER, SPTRSV_KERNEL_MULTIROW}) {
             auto it = std::find_if(ranked.begin(), ranked.end(),
                                    [&](const auto& r) { return r.second.kernel == kern; });
@@ -1177,7 +1222,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     }
     // Stage 6 (level-ordered copy): the best ORDER / MULTIROW shape walked on
     // the copy; the copy is released again when it loses.
-    if (status == SPTRSV_OK && precision != SPTRSV_PREC_F32 && bc.variant != 3 &&
+    if (status == SPTRSV_OK && precision != SPTRSV_PREC_F32 && bc.variant != 3 && bc.variant != 4 &&
         (bc.kernel == SPTRSV_KERNEL_ORDER || bc.kernel == SPTRSV_KERNEL_MULTIROW)) {
         sptrsv_config_t c = bc;
         c.reorder = 1;

@@ -57,6 +57,31 @@ struct TileTable {
     int cbits = 0;
 };
 
+// Plan of the level walk (level_walk.hip) for one analysis: steps and slices,
+// their slots (dependency, and the entry the value comes from), and the records
+// of the kinds used so far (0 FP64, 1 FP32, 2 mixed).
+struct LevelPlan {
+    bool bad = false;            // the walk is not taken for this analysis
+    bool far = false;            // entries beyond the LDS ring
+    bool permuted = false;       // b and x pass through position order (L.b, L.x)
+    bool ready[3] = {false, false, false};
+    int nw = 0, nsteps = 0, n_steps_all = 0, n_slices = 0, n_over = 0;
+    void* slice = nullptr;
+    void* step = nullptr;
+    unsigned *col = nullptr, *fcol = nullptr, *ocol = nullptr;  // slots, far slots, overflow slots
+    int *from = nullptr, *ffrom = nullptr, *ofrom = nullptr;
+    int* over = nullptr;         // first overflow unit of each slice
+    int* diag_from = nullptr;    // entry of each position's diagonal
+    int* order = nullptr;        // row of each position
+    unsigned *rec[2] = {}, *frec[2] = {}, *orec[2] = {};
+    void* rows[3] = {};
+    float* piv32 = nullptr;
+    uint64_t* pub = nullptr;     // published words (mixed, far entries)
+    void *b[3] = {}, *x[3] = {};
+    // the allocations that hold the arrays above
+    void *structure = nullptr, *shared = nullptr, *kind[3] = {};
+};
+
 struct MatPriv {
     int* counters = nullptr;     // [0] ticket, [1] watchdog word, [2..] spare (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
@@ -71,6 +96,7 @@ struct MatPriv {
     dfr_analysis_info_t* lc_info = nullptr;
     int* lc_rows = nullptr;
     unsigned long long lc_src = 0;
+    std::map<unsigned long long, LevelPlan> lw;  // level walk: plan per analysis (by its id)
     // in-degree walk: per-row counters and the off-diagonal pattern by column
     // (built on first use; structure only, so new values keep them)
     int* indeg = nullptr;
@@ -168,6 +194,14 @@ void drop_graphs(MatPriv* pv);
 void free_mat(sp_mat_t* m);  // device arrays and private state; zeroes *m
 // Releases a matrix's level-ordered copy (if any).
 void drop_level_copy(MatPriv* pv);
+// Level walk: whether it is the default shape of an analysed solve, its plan's
+// release and the plan's values after the matrix's changed.
+bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info);
+void drop_level_plans(MatPriv* pv);
+void drop_level_plan(MatPriv* pv, unsigned long long id);
+int level_plan_values_changed(sp_mat_t* m);
+// Releases what the live matrices keep for the analysis with this id.
+void analysis_freed(unsigned long long id);
 void free_info_arrays(dfr_analysis_info_t* info);
 // The analysis of `copy`, the level-ordered copy made for analysis `src`,
 // derived from `src` (levels permuted, iorder the identity, the rest shared).

@@ -46,6 +46,11 @@ void drop_graphs(MatPriv* pv) {
     pv->graphs.clear();
 }
 
+void analysis_freed(unsigned long long id) {
+    std::lock_guard<std::mutex> g(g_live_mu);
+    for (MatPriv* pv : g_live) drop_level_plan(pv, id);
+}
+
 int convert_values_to_f32(sp_mat_t* m);
 void free_info_arrays(dfr_analysis_info_t* info);
 int jacobi_values_changed(sp_mat_t* m);
@@ -102,7 +107,13 @@ void free_mat(sp_mat_t* m) {
     if (m->a32) (void)hipFree(m->a32);
     MatPriv* pv = priv_of(m);
     if (pv) {
+        {
+            // first, so that no freed analysis looks at this matrix any more
+            std::lock_guard<std::mutex> g(g_live_mu);
+            g_live.erase(pv);
+        }
         drop_level_copy(pv);
+        drop_level_plans(pv);
         if (pv->counters) (void)hipFree(pv->counters);
         if (pv->pub) (void)hipFree(pv->pub);
         if (pv->part) (void)hipFree(pv->part);
@@ -121,10 +132,6 @@ void free_mat(sp_mat_t* m) {
         if (pv->jac_norms) (void)hipFree(pv->jac_norms);
         for (auto& g : pv->graphs) (void)hipGraphExecDestroy(g.second);
         if (pv->cap_stream) (void)hipStreamDestroy(pv->cap_stream);
-        {
-            std::lock_guard<std::mutex> g(g_live_mu);
-            g_live.erase(pv);
-        }
         for (TileTable& t : pv->jac_tt) {
             if (t.tiles) (void)hipFree(t.tiles);
             if (t.member) (void)hipFree(t.member);
@@ -446,6 +453,7 @@ int sptrsv_update_values(sp_mat_t* mat, const double* vals, long long count, int
     // the margin into their launches, so they are dropped; a tuned Jacobi
     // choice may no longer apply (dominance can be lost)
     if (mat->a) SPT_TRY(jacobi_values_changed(mat));
+    SPT_TRY(level_plan_values_changed(mat));
     drop_level_copy(pv);  // holds the old values; rebuilt on its next use
     drop_graphs(pv);
     for (int p = 0; p < 3; ++p)
