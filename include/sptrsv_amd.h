@@ -283,13 +283,18 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * bytes for each of 64 * 5 slots per group of up to 64 rows of a level,
  * released with either; the lean path runs instead while a stream is captured
  * before the plan exists, while a trace is taken, and where no plan can be
- * made); cu_waves caps the waves
+ * made); 5 is the block walk (one right-hand side, natural order whatever the
+ * kernel): 64 consecutive rows per wave, results of the block's own rows
+ * exchanged in registers, for columns at most 63 rows back or rows of at most
+ * 8 off-diagonals (other matrices, and a traced solve, take the lean path);
+ * cu_waves caps the waves
  * resident per CU (0 = hardware limit): every resident wave polls, and past a
  * few thousand polling waves the dependency hand-off latency grows several
  * fold, so deep dependency chains run fastest with a small cap.  With lanes
  * = 0 the lanes (and, when variant is 0, the variant) come from the tuned
- * shape of the kernel, else from the default shape (the level walk where a
- * level's share of the matrix is small, else the lean path); MULTIROW takes its lanes
+ * shape of the kernel, else from the default shape (SIMPLE: the block walk for
+ * banded matrices and grid-like ones; ORDER and MULTIROW: the level walk where
+ * a level's share of the matrix is small; else the lean path); MULTIROW takes its lanes
  * per row from the analysis and ignores a nonzero lanes. */
 typedef struct {
     int kernel;

@@ -39,7 +39,7 @@ HIP_FLAGS = [
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", f"-I{INCLUDE}", f"-I{CSRC}",
              f"-I{ROCM / 'include'}", "-D__HIP_PLATFORM_AMD__"]
 
-HIP_SOURCES = ["inst_f64.hip", "inst_f32.hip", "inst_mixed.hip", "inst_level.hip", "level_walk.hip",
+HIP_SOURCES = ["inst_f64.hip", "inst_f32.hip", "inst_mixed.hip", "inst_level.hip", "level_walk.hip", "block_rows.hip",
                "api_solve.hip", "analysis.hip", "interface.hip", "batch.hip", "iterative.hip",
                "transpose.hip", "ingest.hip", "spsv.hip"]
 HOST_HIP_SOURCES = ["power.cpp", "rocsparse_baseline.cpp"]   # need HIP headers, no kernels

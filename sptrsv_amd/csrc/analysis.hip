@@ -594,7 +594,9 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     // entries) take one lane per row on the general engine: 64 consecutive
     // rows per wave keep many more rows in flight, which a natural-order walk
     // of a grid-like matrix needs to find ready rows.  Other matrices keep
-    // the reference's tile rule.
+    // the reference's tile rule.  Before all these, the block walk where it is
+    // the natural-order solve's default.
+    const bool blocks = block_walk_fits(m);
     int kind = KK_SIMPLE;
     unsigned dyn_lds = 0;
     const int avg = n > 0 ? m->nnz / n : 0;
@@ -621,13 +623,14 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         A.ticket = pv->counters;
         A.err = pv->counters + 1;
         A.wd_ticks = pv->watchdog_ticks;
-        A.dyn_lds = dyn_lds;
+        A.dyn_lds = blocks ? 0 : dyn_lds;
         hipLaunchKernelGGL((k_prepare<uint32_t>), dim3(grid_for(n)), dim3(256), 0, s,
                            reinterpret_cast<uint32_t*>(info->level), (size_t)n, 0u, pv->counters, nullptr,
                            (size_t)0, nullptr, nullptr, 0);
         SPT_HIP(hipGetLastError());
         int u = (pv->max_row > 2 * lanes) ? 4 : 1;
-        hipError_t e = launch_solve<PolLevel, 1>(kind, 1, wg, u, A, s);
+        const hipError_t e = blocks ? launch_block_rows<PolLevel>(A, block_walk_in_order(m), pv->max_row - 1, s)
+                                                : launch_solve<PolLevel, 1>(kind, 1, wg, u, A, s);
         if (e != hipSuccess) return hip_fail(e, "level pass", __FILE__, __LINE__);
     }
     // 2. nlevs
@@ -648,6 +651,7 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         return fail(SPTRSV_E_WATCHDOG, "level analysis: a dependency wait exceeded its bound");
     }
     const int nlevs = h_max[0];
+    if (pv->banded && !pv->band_levels) pv->band_levels = nlevs;
     if (nlevs <= 0 || (long long)nlevs * 7 > (1LL << 30))
         return fail(SPTRSV_E_INVALID_CSR, "level analysis produced an invalid level count");
     info->nlevs = nlevs;

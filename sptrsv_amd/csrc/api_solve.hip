@@ -131,6 +131,7 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
         c.variant = 1;
         int avg = m->nr > 0 ? m->nnz / m->nr : 1;
         c.lanes = std::min(kWave, std::max(4, pow2_ceil(avg)));
+        if (kernel == SPTRSV_KERNEL_SIMPLE && block_walk_fits(m)) c.variant = 5;
     } else {
         c.variant = 0;
         int lanes = reference_lanes(m);
@@ -140,12 +141,46 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
     return c;
 }
 
+// The block walk is the default of a natural-order solve
+//  * of a banded matrix with few rows per level, its rows in order: bandwidth
+//    17, n = 5000 0.21 ms against 4.0; bandwidth 60, 2 entries per row, n =
+//    300000 18.0 against 20.3;
+//  * of a matrix where at least half of the rows depend on one of the 8 rows
+//    before them, if it is banded or of short rows: grids, 1.1 (64^2) to 15
+//    times (101^3) faster than a row per wave.
+// Where fewer do (4 random entries of the last 1000, n = 300000: 5.2 ms against
+// 3.2; only the row 32 before, n = 4000: 178 us against 112) a dependency costs
+// a hand-off through memory either way, and a row per wave hands over sooner,
+// until there are so many rows per level that it is the rows in flight that
+// count (diagonal, n = 10^6: 0.19 ms against 2.8).
+// Rows are taken in order (banded kernel) unless a level has 16 rows or more
+// and they are short (2D grid of 50^2: 81 us against 118).
+constexpr long long kBandRows = 16, kWideRows = 1024;
+bool block_walk_in_order(const sp_mat_t* m) {
+    const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
+    if (!pv->banded) return false;
+    const bool parallel = pv->band_levels > 0 && m->nr >= kBandRows * pv->band_levels;
+    return !parallel || pv->max_row > kBlockRow + 1;
+}
+
+bool block_walk_fits(const sp_mat_t* m) {
+    const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
+    if (!pv->banded) return pv->near_rows && pv->max_row <= kBlockRow + 1;
+    return pv->near_rows || m->nr < kBandRows * std::max(pv->band_levels, 1) || m->nr >= kWideRows * pv->band_levels;
+}
+
 // The same with the analysis at hand: ORDER and MULTIROW solves with one
-// right-hand side take the level walk where it fits.
+// right-hand side take the level walk where it fits, or, for banded matrices
+// with less than four rows per level, the block walk: it takes about 40 ns a
+// row, the level walk 170 to 200 ns a level (bandwidth 9, n = 5000: 0.21 ms
+// against 1.00).
+constexpr long long kChainRows = 4;
 static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
     sptrsv_config_t c = shape_for(m, kernel, k);
-    if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1 && level_walk_fits(m, info))
-        c.variant = 4;
+    if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1) {
+        if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;
+        else if (level_walk_fits(m, info)) c.variant = 4;
+    }
     return c;
 }
 
@@ -218,7 +253,7 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
     if (K > 1) {
         // several RHS: the general engine, ticketed (256 threads) or
         // persistent (256 or 1024 threads)
-        if (out->kernel != SPTRSV_KERNEL_JACOBI && out->variant != 2 && out->variant != 3 && out->variant != 4)
+        if (out->kernel != SPTRSV_KERNEL_JACOBI && out->variant != 2 && out->variant != 3 && out->variant < 4)
             out->variant = 0;
         if (!(out->variant == 2 && out->wg == 1024)) out->wg = 256;
     }
@@ -242,8 +277,10 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
         return fail(SPTRSV_E_INVALID_ARG, "unknown kernel");
     if (out->kernel == SPTRSV_KERNEL_JACOBI && precision != SPTRSV_PREC_MIXED)
         return fail(SPTRSV_E_INVALID_ARG, "JACOBI is the bulk solver of the MIXED path only");
-    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 4))
-        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..4");
+    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 5))
+        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..5");
+    if (out->variant == 5 && out->kernel != SPTRSV_KERNEL_JACOBI && (K > 1 || out->reorder == 1))
+        return fail(SPTRSV_E_INVALID_ARG, "the block walk (variant 5) takes one right-hand side and the matrix as given");
     if (out->variant == 4 && out->kernel != SPTRSV_KERNEL_JACOBI &&
         (K > 1 || out->kernel == SPTRSV_KERNEL_SIMPLE || out->reorder == 1))
         return fail(SPTRSV_E_INVALID_ARG, "the level walk (variant 4) takes ORDER or MULTIROW, one right-hand side and "
@@ -562,6 +599,11 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         if (done) return SPTRSV_OK;
         c = shape_for(m, c.kernel, k);
     }
+    // a trace is written by the walks row by row
+    if (c.variant == 5 && (pv->trace || !(pv->banded || pv->max_row <= kBlockRow + 1))) {
+        c = shape_for(m, c.kernel, k);
+        if (c.variant == 5) c.variant = 1;
+    }
     const sp_mat_t* sm = lv ? lv->mat : m;
     const int K = pow2_ceil(k);
     SolveArgs A{};
@@ -628,7 +670,7 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
     int u = c.window > 0 ? c.window : window_for(pv, (kind == KK_MULTIROW || kind == KK_FAST_MULTIROW) ? 32 : c.lanes);
     const KtPair ev = timed ? kernel_timer_pair(s) : KtPair{};
     if (ev) SPT_HIP(hipEventRecord(ev[0], s));
-    hipError_t e = launch_solve<P, 64>(kind, K, c.wg, u, A, s);
+    const hipError_t e = c.variant == 5 ? launch_block_rows<P>(A, block_walk_in_order(m), pv->max_row - 1, s) : launch_solve<P, 64>(kind, K, c.wg, u, A, s);
     if (e != hipSuccess) return hip_fail(e, "sync-free solve launch", __FILE__, __LINE__);
     if (ev) SPT_HIP(hipEventRecord(ev[1], s));
     return SPTRSV_OK;
@@ -1118,6 +1160,8 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
 
     // level by level in one workgroup, where a level is small
     if (K == 1 && has_order(info) && level_walk_fits(mat, info)) shapes.push_back({SPTRSV_KERNEL_ORDER, ref, 256, 1, 4, 0});
+    // blocks of 64 rows in natural order
+    if (K == 1 && block_walk_fits(mat)) shapes.push_back({SPTRSV_KERNEL_SIMPLE, ref, 256, 1, 5, 0});
 
     hipEvent_t e0, e1;
     SPT_HIP(hipEventCreate(&e0));
@@ -1139,7 +1183,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     // Stage 1: every shape without and with a tight residency cap.
     std::vector<std::pair<float, sptrsv_config_t>> ranked;
     for (auto c : shapes) {
-        for (int cw : (c.variant == 2 ? std::vector<int>{2, 8} : c.variant == 4 ? std::vector<int>{0} : std::vector<int>{0, 4})) {
+        for (int cw : (c.variant == 2 ? std::vector<int>{2, 8} : c.variant >= 4 ? std::vector<int>{0} : std::vector<int>{0, 4})) {
             c.cu_waves = cw;
             float t = time_cfg(c);
             if (status != SPTRSV_OK) break;
@@ -1165,7 +1209,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
             }
             if (dup) continue;
             ++taken;
-            if (c.variant == 4) continue;  // one workgroup: nothing to cap
+            if (c.variant >= 4) continue;  // nothing to cap
             for (int cw : (c.variant == 2 ? std::vector<int>{1, 3, 4, 6, 12, 16}
                                           : std::vector<int>{32, 16, 8, 2})) {
                 c.cu_waves = cw;
@@ -1180,7 +1224,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     }
     // Stage 3 (long rows): the best shape of each kernel with 16 entries per
     // lane in flight instead of 4, which shortens the load chain of a long row.
-    if (status == SPTRSV_OK && K == 1 && pv->max_row > 64 && bc.variant != 4) {
+    if (status == SPTRSV_OK && K == 1 && pv->max_row > 64 && bc.variant < 4) {
         for (int kern : {SPTRSV_KERNEL_SIMPLE, SPTRSV_KERNEL_ORDER, SPTRSV_KERNEL_MULTIROW}) {
             auto it = std::find_if(ranked.begin(), ranked.end(),
                                    [&](const auto& r) { return r.second.kernel == kern; });
@@ -1222,7 +1266,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     }
     // Stage 6 (level-ordered copy): the best ORDER / MULTIROW shape walked on
     // the copy; the copy is released again when it loses.
-    if (status == SPTRSV_OK && precision != SPTRSV_PREC_F32 && bc.variant != 3 && bc.variant != 4 &&
+    if (status == SPTRSV_OK && precision != SPTRSV_PREC_F32 && bc.variant < 3 &&
         (bc.kernel == SPTRSV_KERNEL_ORDER || bc.kernel == SPTRSV_KERNEL_MULTIROW)) {
         sptrsv_config_t c = bc;
         c.reorder = 1;

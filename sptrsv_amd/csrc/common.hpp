@@ -83,7 +83,7 @@ struct LevelPlan {
 };
 
 struct MatPriv {
-    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [2..] spare (device)
+    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4], [5] row shape, others spare (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
     size_t pub_words = 0;
     uint64_t* part = nullptr;    // published partial sums of long-row segments, 2 per segment (device)
@@ -110,6 +110,9 @@ struct MatPriv {
     double wall_rate_khz = 100000.0;
     int device = 0;
     int max_row = 0;             // longest row (entries incl. diagonal)
+    bool banded = false;         // no column more than 63 rows back
+    int band_levels = 0;         // banded: number of levels (0: not known)
+    bool near_rows = false;      // at least half of the rows depend on one of the kNear rows before them
     long long* trace = nullptr;  // per-row timeline (profiling), 3*n*k
     size_t trace_len = 0;
     int backoff = 0;
@@ -202,6 +205,27 @@ void drop_level_plan(MatPriv* pv, unsigned long long id);
 int level_plan_values_changed(sp_mat_t* m);
 // Releases what the live matrices keep for the analysis with this id.
 void analysis_freed(unsigned long long id);
+// What the rows of a matrix look like, for the choice of a walk.
+constexpr int kNear = 8;
+struct RowShape {
+    int longest = 0;        // entries, with the diagonal
+    bool wide = false;      // a column 64 or more rows back
+    int levels = 0;         // while !wide; 0: not counted
+    long long near = 0;     // rows whose last off-diagonal is at most kNear rows back
+    // of the `seen` rows that near was counted over
+    void install(MatPriv* pv, long long rows, long long seen) const {
+        pv->max_row = longest;
+        pv->banded = !wide && rows > 0;
+        pv->band_levels = wide ? 0 : levels;
+        pv->near_rows = seen > 0 && 2 * near >= seen;
+    }
+};
+// The same of a matrix made on the device (its longest row given; waits).
+int install_row_shape(sp_mat_t* m, int longest);
+// Whether the block walk is the default of a natural-order solve, and whether
+// it takes its rows in order (banded kernel).
+bool block_walk_fits(const sp_mat_t* m);
+bool block_walk_in_order(const sp_mat_t* m);
 void free_info_arrays(dfr_analysis_info_t* info);
 // The analysis of `copy`, the level-ordered copy made for analysis `src`,
 // derived from `src` (levels permuted, iorder the identity, the rest shared).

@@ -239,7 +239,7 @@ int sptrsv_coo_to_lower(const int* row, const int* col, const double* val, int n
     if (st == SPTRSV_OK) {
         int mr = 0;
         for (int i = 0; i < n; ++i) mr = std::max(mr, ia_h[i + 1] - ia_h[i]);
-        pv->max_row = mr;
+        st = install_row_shape(gpu_L, mr);
         chk(hipDeviceSynchronize(), "ingest sync");
     }
     if (st == SPTRSV_OK) st = convert_values_to_f32(gpu_L);

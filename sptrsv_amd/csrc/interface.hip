@@ -87,12 +87,12 @@ int ensure_priv(sp_mat_t* m) {
         rate > 0)
         pv->wall_rate_khz = rate;
     pv->watchdog_ticks = (long long)(watchdog_ms_default() * pv->wall_rate_khz);
-    hipError_t e = hipMalloc(&pv->counters, 4 * sizeof(int));
+    hipError_t e = hipMalloc(&pv->counters, 8 * sizeof(int));
     if (e != hipSuccess) {
         delete pv;
         return hip_fail(e, "hipMalloc counters", __FILE__, __LINE__);
     }
-    SPT_HIP(hipMemset(pv->counters, 0, 4 * sizeof(int)));
+    SPT_HIP(hipMemset(pv->counters, 0, 8 * sizeof(int)));
     m->priv = pv;
     std::lock_guard<std::mutex> g(g_live_mu);
     g_live.insert(pv);
@@ -144,45 +144,91 @@ void free_mat(sp_mat_t* m) {
     memset(m, 0, sizeof(*m));
 }
 
+// out[0]: a column 64 or more rows back; out[1]: rows whose last off-diagonal
+// is nearer.  A thread leaves a row at its first far column, so long rows of
+// wide matrices cost one load.
+__global__ __launch_bounds__(256) void k_row_shape(const int* __restrict__ ia, const int* __restrict__ ja, int n,
+                                                   int* __restrict__ out) {
+    __shared__ int s_near, s_wide;
+    if (threadIdx.x == 0) s_near = s_wide = 0;
+    __syncthreads();
+    int near = 0, wide = 0;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+        const int lo = ia[i], hi = ia[i + 1] - 1;
+        if (lo < hi) near += (int)i - ja[hi - 1] <= kNear;
+        for (int p = lo; p < hi && !wide; ++p) wide = (int)i - ja[p] >= kWave;
+    }
+    if (near) atomicAdd(&s_near, near);
+    if (wide) s_wide = 1;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_wide) out[0] = 1;
+        if (s_near) atomicAdd(&out[1], s_near);
+    }
+}
+
+int install_row_shape(sp_mat_t* m, int longest) {
+    RowShape shape;
+    shape.longest = longest;
+    const int n = m->nr;
+    if (n > 0) {
+        int h[2] = {0, 0}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
+        hipLaunchKernelGGL(k_row_shape, dim3(std::min<unsigned>(ceil_div(n, 256), 512)), dim3(256), 0, nullptr, m->ia,
+                           m->ja, n, d);
+        SPT_HIP(hipGetLastError());
+        SPT_HIP(hipMemcpy(h, d, sizeof(h), hipMemcpyDeviceToHost));
+        shape.wide = h[0] != 0;
+        shape.near = h[1];
+    }
+    shape.install(priv_of(m), n, n);
+    return SPTRSV_OK;
+}
+
 // Validates a host CSR lower triangle: every row non-empty, diagonal last,
-// off-diagonal columns in [0, i).  Returns the longest row or a status < 0.
-static int validate_host_csr(const int* ia, const int* ja, int n, int* max_row) {
+// off-diagonal columns in [0, i).  Adds its rows to *shape.
+static int validate_host_csr(const int* ia, const int* ja, int n, RowShape* shape) {
     if (n < 0) return fail(SPTRSV_E_INVALID_ARG, "n < 0");
-    if (n == 0) { *max_row = 0; return SPTRSV_OK; }
+    if (n == 0) return SPTRSV_OK;
     if (!ia || !ja) return fail(SPTRSV_E_INVALID_ARG, "null CSR arrays");
     const int base = ia[0];
     if (base < 0) return fail(SPTRSV_E_INVALID_CSR, "negative row pointer");
     ja += base;  // rows index ja relative to ia[0]
-    int mr = 0;
+    int lev[kWave] = {};  // levels of the last 64 rows, while they are all that is needed
     for (int i = 0; i < n; ++i) {
+        int level = 1;
         long long s = (long long)ia[i] - base, e = (long long)ia[i + 1] - base;
         if (e <= s)
             return fail(SPTRSV_E_INVALID_CSR, "row " + std::to_string(i) + " has no diagonal entry");
         if (ja[e - 1] != i)
             return fail(SPTRSV_E_INVALID_CSR,
                         "row " + std::to_string(i) + ": last entry is not the diagonal");
-        for (long long p = s; p < e - 1; ++p)
+        for (long long p = s; p < e - 1; ++p) {
             if (ja[p] < 0 || ja[p] >= i)
                 return fail(SPTRSV_E_INVALID_CSR, "row " + std::to_string(i) + ": column " +
                                                       std::to_string(ja[p]) +
                                                       " outside the strict lower triangle");
-        mr = std::max<int>(mr, (int)(e - s));
+            shape->wide |= i - ja[p] >= kWave;
+            if (!shape->wide) level = std::max(level, lev[ja[p] % kWave] + 1);
+        }
+        lev[i % kWave] = level;
+        shape->levels = std::max(shape->levels, level);
+        shape->near += e - s > 1 && i - ja[e - 2] <= kNear;
+        shape->longest = std::max<int>(shape->longest, (int)(e - s));
     }
-    *max_row = mr;
     return SPTRSV_OK;
 }
 
 template <class V>
 static int upload(const int* ia, const int* ja, const V* val, int n, sp_mat_t* m) {
     if (!m) return fail(SPTRSV_E_INVALID_ARG, "null sp_mat_t");
-    int max_row = 0;
+    RowShape shape;
     memset(m, 0, sizeof(*m));
-    SPT_TRY(validate_host_csr(ia, ja, n, &max_row));
+    SPT_TRY(validate_host_csr(ia, ja, n, &shape));
     if (n > 0 && !val) return fail(SPTRSV_E_INVALID_ARG, "null values");
     long long nnz = n > 0 ? (long long)ia[n] - ia[0] : 0;
     if (nnz > 0x7fffffffLL) return fail(SPTRSV_E_CAPACITY, "nnz exceeds int32");
     SPT_TRY(ensure_priv(m));
-    priv_of(m)->max_row = max_row;
+    shape.install(priv_of(m), n, n);
     m->nr = n;
     m->nc = n;
     m->nnz = (int)nnz;
@@ -251,20 +297,18 @@ int upload_concat(const int* n, const int* const* ia, const int* const* ja, cons
     memset(m, 0, sizeof(*m));
     row_off.assign(nmat + 1, 0);
     std::vector<long long> nnz_off(nmat + 1, 0);
-    int max_row = 0;
+    RowShape shape;
     for (int q = 0; q < nmat; ++q) {
-        int mr = 0;
         if (n[q] < 0) return fail(SPTRSV_E_INVALID_ARG, "negative size");
-        int st = validate_host_csr(ia[q], ja[q], n[q], &mr);
+        int st = validate_host_csr(ia[q], ja[q], n[q], &shape);
         if (st != SPTRSV_OK) return fail(st, "matrix " + std::to_string(q) + ": " + g_last_error);
-        max_row = std::max(max_row, mr);
         row_off[q + 1] = row_off[q] + n[q];
         nnz_off[q + 1] = nnz_off[q] + (n[q] > 0 ? (long long)ia[q][n[q]] - ia[q][0] : 0);
     }
     const long long rows = row_off[nmat], nnz = nnz_off[nmat];
     if (rows > 0x7ffffffeLL || nnz > 0x7fffffffLL) return fail(SPTRSV_E_CAPACITY, "batch exceeds int32 indexing");
     SPT_TRY(ensure_priv(m));
-    priv_of(m)->max_row = max_row;
+    shape.install(priv_of(m), rows, rows);
     m->nr = m->nc = (int)rows;
     m->nnz = (int)nnz;
     int st = SPTRSV_OK;

@@ -34,24 +34,46 @@ unsigned row_grid(long long count) {
 
 // Stored-row lengths: kept off-diagonals + 1 (the diagonal) at the stored
 // row (i, or n-1-i for an upper triangle); dpos[i] = the diagonal entry used
-// (-1 for a unit diagonal); bad bit 1 = column outside [0, n), bit 2 = a
-// missing diagonal.
-__global__ void k_tri_count(const int* __restrict__ ia, const int* __restrict__ ja, int n, int upper, int unit,
-                            int* __restrict__ len, int* __restrict__ dpos, int* __restrict__ bad) {
+// (-1 for a unit diagonal); out[0] bit 1 = column outside [0, n), bit 2 = a
+// missing diagonal; out[1] = a kept column 64 or more rows away; out[2] of the
+// out[3] rows of every eighth workgroup have their last kept one within kNear.
+__global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, const int* __restrict__ ja, int n,
+                                                   int upper, int unit, int* __restrict__ len, int* __restrict__ dpos,
+                                                   int* __restrict__ out) {
+    int wide = 0, near = 0, rows = 0;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
          t += (long long)gridDim.x * blockDim.x) {
         const int i = (int)t;
-        int kept = 0, d = -1, flags = 0;
+        int kept = 0, d = -1, flags = 0, last = kWave;
         for (int p = ia[i]; p < ia[i + 1]; ++p) {
             const int j = ja[p];
             if (j < 0 || j >= n) flags |= 1;
             else if (j == i) { if (d < 0) d = p; }
-            else if (upper ? j > i : j < i) ++kept;
+            else if (upper ? j > i : j < i) {
+                ++kept;
+                last = abs(i - j);
+                wide |= last >= kWave;
+            }
         }
         if (!unit && d < 0) flags |= 2;
-        if (flags) atomicOr(bad, flags);
+        if (flags) atomicOr(out, flags);
         len[upper ? n - 1 - i : i] = kept + 1;
         dpos[i] = unit ? -1 : d;
+        near += last <= kNear;
+        ++rows;
+    }
+    if (wide) out[1] = 1;
+    if ((blockIdx.x & 7) == 0) {
+        __shared__ int s_near, s_rows;
+        if (threadIdx.x == 0) s_near = s_rows = 0;
+        __syncthreads();
+        if (near) atomicAdd(&s_near, near);
+        atomicAdd(&s_rows, rows);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            atomicAdd(&out[2], s_near);
+            atomicAdd(&out[3], s_rows);
+        }
     }
 }
 
@@ -100,17 +122,18 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     int *len = nullptr, *dpos = nullptr, *bad = nullptr;
     chk(hipMalloc(&len, 4 * ((size_t)n + 1)), "hipMalloc lengths");
     chk(hipMalloc(&dpos, 4 * (size_t)std::max(n, 1)), "hipMalloc diagonal positions");
-    chk(hipMalloc(&bad, 4), "hipMalloc flag");
+    chk(hipMalloc(&bad, 16), "hipMalloc flag");
     chk(hipMalloc(&m->ia, 4 * ((size_t)n + 1)), "hipMalloc ia");
     if (st == SPTRSV_OK) chk(hipMemset(len, 0, 4 * ((size_t)n + 1)), "clear lengths");
-    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 4), "clear flag");
+    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 16), "clear flag");
     if (st == SPTRSV_OK && n > 0) {
         hipLaunchKernelGGL(k_tri_count, dim3(row_grid(n)), dim3(256), 0, nullptr, ia, ja, n, upper ? 1 : 0,
                            unit ? 1 : 0, len, dpos, bad);
         chk(hipGetLastError(), "triangle count");
     }
-    int h_bad = 0;
-    if (st == SPTRSV_OK) chk(hipMemcpy(&h_bad, bad, 4, hipMemcpyDeviceToHost), "read flag");
+    int h_out[4] = {};
+    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 16, hipMemcpyDeviceToHost), "read flag");
+    const int h_bad = h_out[0];
     if (st == SPTRSV_OK && (h_bad & 1)) st = fail(SPTRSV_E_INVALID_CSR, "column index outside [0, n)");
     if (st == SPTRSV_OK && (h_bad & 2)) st = fail(SPTRSV_E_INVALID_CSR, "a row has no diagonal entry (non-unit diagonal)");
     if (st == SPTRSV_OK) st = exclusive_scan(len, m->ia, (long long)n + 1, nullptr);
@@ -129,9 +152,11 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
         chk(hipGetLastError(), "triangle fill");
     }
     if (st == SPTRSV_OK) {
-        int mr = 0;
-        for (int r = 0; r < n; ++r) mr = std::max(mr, ia_h[r + 1] - ia_h[r]);
-        priv_of(m)->max_row = mr;
+        RowShape shape;
+        for (int r = 0; r < n; ++r) shape.longest = std::max(shape.longest, ia_h[r + 1] - ia_h[r]);
+        shape.wide = h_out[1] != 0;
+        shape.near = h_out[2];
+        shape.install(priv_of(m), n, h_out[3]);
         chk(hipDeviceSynchronize(), "triangle sync");
     }
     if (st == SPTRSV_OK) st = convert_values_to_f32(m);

@@ -1322,4 +1322,10 @@ extern template hipError_t launch_solve<PolF32, 64>(int, int, int, int, const So
 extern template hipError_t launch_solve<PolMixed, 64>(int, int, int, int, const SolveArgs&, hipStream_t);
 extern template hipError_t launch_solve<PolLevel, 1>(int, int, int, int, const SolveArgs&, hipStream_t);
 
+// The block walk (block_rows.hip): natural order, one right-hand side, columns
+// at most 63 rows back (banded) or rows of at most kBlockRow off-diagonals.
+constexpr int kBlockRow = 8;
+template <class P>
+hipError_t launch_block_rows(const SolveArgs& A, bool banded, int longest, hipStream_t s);
+
 }  // namespace sptrsv

@@ -122,7 +122,13 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
         int mr = 0;
         for (int r = 0; r < n && st == SPTRSV_OK; ++r) mr = std::max(mr, ia[r + 1] - ia[r]);
         if (st == SPTRSV_OK && ia[n] != nnz) st = fail(SPTRSV_E_INVALID_CSR, "transpose row pointers do not sum to nnz");
-        priv_of(dst)->max_row = mr;
+        MatPriv* dp = priv_of(dst);
+        const MatPriv* from = priv_of(src);
+        dp->max_row = mr;
+        // distances and levels are those of the source; near rows as there
+        dp->banded = from->banded;
+        dp->band_levels = from->band_levels;
+        dp->near_rows = from->near_rows;
     }
     // the sorted payload is the value map of the new handle
     MatPriv* sp = priv_of(src);
