@@ -367,6 +367,9 @@ static unsigned grid_for(long long count) {
 // pointer not being registered, so its garbage pointers are never freed.
 struct InfoPriv {
     SegTable seg;              // long-row segments of the multirow walks (derived data)
+    // wave64 layout of an ORDER analysis, for the packed walk (derived data;
+    // MULTIROW and ALL analyses have it in info)
+    int *wbase = nullptr, *wsize = nullptr, n_waves = 0;
     unsigned long long id = 0;  // unique per analysis built, loaded or copied
 };
 static std::mutex g_info_mu;
@@ -403,6 +406,13 @@ const SegTable* segments_of(const dfr_analysis_info_t* info) {
     return t.items ? &t : nullptr;
 }
 
+PackedWaves packed_waves(const dfr_analysis_info_t* info) {
+    if (!info || !owns_info(info)) return {};
+    if (info->ibase_row64) return {info->ibase_row64, info->ivect_size_wave, info->n_waves};
+    const InfoPriv* ip = static_cast<const InfoPriv*>(info->priv);
+    return {ip->wbase, ip->wsize, ip->n_waves};
+}
+
 void free_info_arrays(dfr_analysis_info_t* info) {
     if (!info || !owns_info(info)) return;
     InfoPriv* ip = static_cast<InfoPriv*>(info->priv);
@@ -412,7 +422,7 @@ void free_info_arrays(dfr_analysis_info_t* info) {
     }
     analysis_freed(ip->id);
     free_segments(ip->seg);
-    int* arrays[] = {info->lev_size, info->warp_lev, info->inv_iorder, info->iorder,
+    int* arrays[] = {ip->wbase, ip->wsize, info->lev_size, info->warp_lev, info->inv_iorder, info->iorder,
                      info->ibase_row, info->ivect_size_warp, info->row_ctr, info->level,
                      info->bucket_off, info->ibase_row64, info->ivect_size_wave};
     for (int* p : arrays)
@@ -516,15 +526,15 @@ int build_segments(dfr_analysis_info_t* info, sp_mat_t* m) {
     if (!owns_info(info)) return SPTRSV_OK;
     SegTable& t = static_cast<InfoPriv*>(info->priv)->seg;
     free_segments(t);
-    if (!info->ibase_row64 || info->n_waves == 0 || m->nr == 0) return SPTRSV_OK;
+    const PackedWaves pw = packed_waves(info);
+    if (!pw.base || pw.n == 0 || m->nr == 0) return SPTRSV_OK;
     const MatPriv* pv = priv_of(m);
     if (pv && pv->max_row <= kSegMin + 1) return SPTRSV_OK;  // no row long enough to split
-    const int nw = info->n_waves, n = m->nr;
+    const int nw = pw.n, n = m->nr;
     hipStream_t s = nullptr;
     int* cnt = nullptr;
     SPT_HIP(hipMalloc(&cnt, sizeof(int) * (size_t)(nw + 1)));
-    hipLaunchKernelGGL(k_seg_count, dim3(grid_for(nw + 1)), dim3(256), 0, s, m->ia, info->iorder, info->ibase_row64,
-                       info->ivect_size_wave, nw, cnt);
+    hipLaunchKernelGGL(k_seg_count, dim3(grid_for(nw + 1)), dim3(256), 0, s, m->ia, info->iorder, pw.base, pw.size, nw, cnt);
     int st = hipGetLastError() == hipSuccess ? SPTRSV_OK : fail(SPTRSV_E_HIP, "segment count");
     if (st == SPTRSV_OK) st = exclusive_scan(cnt, cnt, nw + 1, s);
     int total = 0;
@@ -544,7 +554,7 @@ int build_segments(dfr_analysis_info_t* info, sp_mat_t* m) {
         if (st == SPTRSV_OK) {
             hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n)), dim3(256), 0, s, t.row_seg, (long long)n, -1);
             hipLaunchKernelGGL(k_seg_fill, dim3(grid_for(nw)), dim3(256), 0, s, m->ia, info->iorder,
-                               info->ibase_row64, info->ivect_size_wave, nw, cnt, t.items, t.seg_lo, t.seg_hi,
+                               pw.base, pw.size, nw, cnt, t.items, t.seg_lo, t.seg_hi,
                                t.row_seg);
             if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
                 st = fail(SPTRSV_E_HIP, "segment fill");
@@ -567,6 +577,30 @@ int build_segments(dfr_analysis_info_t* info, sp_mat_t* m) {
     }
     (void)hipFree(cnt);
     return st;
+}
+
+__global__ void k_bucket_counts(const int* __restrict__ bucket_off, int nb, int* __restrict__ cnt) {
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x)
+        cnt[b] = bucket_off[b + 1] - bucket_off[b];
+}
+
+// What solves derive from an analysis: the long-row segments of the wave64
+// layout, and that layout itself where the mode leaves it out.
+static int build_derived(dfr_analysis_info_t* info, sp_mat_t* m) {
+    if (info->mode == ORDER && info->n > 0 && owns_info(info)) {
+        InfoPriv* ip = static_cast<InfoPriv*>(info->priv);
+        const int nb = 7 * info->nlevs;
+        int* cnt = nullptr;
+        SPT_HIP(hipMalloc(&cnt, sizeof(int) * (size_t)(nb + 1)));
+        hipLaunchKernelGGL(k_bucket_counts, dim3(grid_for(nb)), dim3(256), 0, nullptr, info->bucket_off, nb, cnt);
+        int st = hipGetLastError() == hipSuccess ? SPTRSV_OK : fail(SPTRSV_E_HIP, "bucket counts");
+        if (st == SPTRSV_OK)
+            st = build_warps(cnt, info->bucket_off, nb, 64, info->n, &ip->wbase, &ip->wsize, &ip->n_waves, nullptr, nullptr);
+        if (st == SPTRSV_OK && hipStreamSynchronize(nullptr) != hipSuccess) st = fail(SPTRSV_E_HIP, "wave layout");
+        (void)hipFree(cnt);
+        if (st != SPTRSV_OK) return st;
+    }
+    return build_segments(info, m);
 }
 
 static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
@@ -726,7 +760,7 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     (void)hipFree(bucket_cnt);
     if (st != SPTRSV_OK) return st;
     SPT_HIP(hipStreamSynchronize(s));
-    return build_segments(info, m);
+    return build_derived(info, m);
 }
 
 // ---- analysis files and copies ------------------------------------------------------
@@ -908,7 +942,7 @@ int sptrsv_load_analysis(const char* path, sp_mat_t* mat, dfr_analysis_info_t* i
             hipMemcpy(*a.dev, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
             st = fail(SPTRSV_E_ALLOC, "analysis arrays");
     }
-    if (st == SPTRSV_OK) st = build_segments(info, mat);
+    if (st == SPTRSV_OK) st = build_derived(info, mat);
     if (st != SPTRSV_OK) free_info_arrays(info);
     return st;
 }
@@ -941,7 +975,7 @@ int sptrsv_copy_analysis(sp_mat_t* src_mat, dfr_analysis_info_t* src, sp_mat_t* 
             hipMemcpy(*to[i].dev, *from[i].dev, bytes, hipMemcpyDeviceToDevice) != hipSuccess)
             st = fail(SPTRSV_E_ALLOC, "analysis arrays");
     }
-    if (st == SPTRSV_OK) st = build_segments(dst, dst_mat);
+    if (st == SPTRSV_OK) st = build_derived(dst, dst_mat);
     if (st != SPTRSV_OK) free_info_arrays(dst);
     return st;
 }
@@ -961,7 +995,7 @@ int multirow_analysis_base_GPU(dfr_analysis_info_t** info, sp_mat_t* gpu_L, MODE
 
 int sptrsv_analysis_segments(const dfr_analysis_info_t* info, int* n_split_rows, int* n_segments) {
     if (!info || !n_segments) return fail(SPTRSV_E_INVALID_ARG, "null info or count");
-    const SegTable* t = segments_of(info);
+    const SegTable* t = info->ibase_row64 ? segments_of(info) : nullptr;  // of the layout in info
     *n_segments = t ? t->n_segs : 0;
     if (n_split_rows) *n_split_rows = t ? t->n_split : 0;
     return SPTRSV_OK;

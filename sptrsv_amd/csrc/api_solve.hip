@@ -169,17 +169,39 @@ bool block_walk_fits(const sp_mat_t* m) {
     return pv->near_rows || m->nr < kBandRows * std::max(pv->band_levels, 1) || m->nr >= kWideRows * pv->band_levels;
 }
 
+// Where and how wide the packed walk (variant 6) runs, by the waves of a level.
+// Up to 100 the 32 CUs of one XCD have enough to do: 30 to 46 waves (random, n =
+// 3*10^4 to 10^6) 143 -> 2.8 ms against 274 us -> 5.7 ms on the whole device, 58
+// (power-law, n = 10^5) 204 against 241 us, 75 (3D grid 60^3) 161 against 250 us,
+// but 145 (power-law, n = 3*10^5) 418 against 306 us.  With less than 20 waves
+// the fewer pollers hand over sooner (2D grid 1000^2, 17 waves: 1.18 ms with 4
+// waves per CU, 1.6 with 16); on the whole device likewise, up to 400 (3D grid
+// 128^3, 340 waves: 643 us with 4 per CU, 766 with 16; power-law n = 2*10^6, 730
+// waves: 1.09 ms and 0.76).
+struct PackedShape {
+    bool local;  // one XCD
+    int wg, cu_waves;
+};
+static PackedShape packed_shape(int n_waves, int nlevs) {
+    const double w = (double)n_waves / std::max(nlevs, 1);
+    if (w < 20) return {true, 256, 4};
+    if (w < 100) return {true, 1024, 16};
+    if (w < 400) return {false, 256, 4};
+    return {false, 1024, 16};
+}
+
 // The same with the analysis at hand: ORDER and MULTIROW solves with one
-// right-hand side take the level walk where it fits, or, for banded matrices
-// with less than four rows per level, the block walk: it takes about 40 ns a
-// row, the level walk 170 to 200 ns a level (bandwidth 9, n = 5000: 0.21 ms
-// against 1.00).
+// right-hand side take the level walk where it fits, else the packed walk; for
+// banded matrices with less than four rows per level the block walk: it takes
+// about 40 ns a row, the level walk 170 to 200 ns a level (bandwidth 9, n =
+// 5000: 0.21 ms against 1.00).
 constexpr long long kChainRows = 4;
 static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
     sptrsv_config_t c = shape_for(m, kernel, k);
     if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1) {
         if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;
         else if (level_walk_fits(m, info)) c.variant = 4;
+        else if (packed_waves(info).base) c.variant = 6;
     }
     return c;
 }
@@ -191,6 +213,12 @@ int default_config(const sp_mat_t* m, const dfr_analysis_info_t* info, int preci
     if (info && info->mode == ORDER && has_order(info)) kernel = SPTRSV_KERNEL_ORDER;
     if (info && info->mode == MULTIROW && has_waves(info)) kernel = SPTRSV_KERNEL_MULTIROW;
     *out = analysed_shape_for(m, info, kernel, k);
+    // an ALL analysis asks for no kernel, and may be there for one solve only:
+    // the packed walk, which needs no plan, or natural order for a chain
+    if (k == 1 && info && info->mode == ALL && has_waves(info) && analysed_shape_for(m, info, SPTRSV_KERNEL_MULTIROW, k).variant != 5) {
+        *out = shape_for(m, SPTRSV_KERNEL_MULTIROW, k);
+        out->variant = 6;
+    }
     return SPTRSV_OK;
 }
 
@@ -277,14 +305,14 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
         return fail(SPTRSV_E_INVALID_ARG, "unknown kernel");
     if (out->kernel == SPTRSV_KERNEL_JACOBI && precision != SPTRSV_PREC_MIXED)
         return fail(SPTRSV_E_INVALID_ARG, "JACOBI is the bulk solver of the MIXED path only");
-    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 5))
-        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..5");
+    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 6))
+        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..6");
     if (out->variant == 5 && out->kernel != SPTRSV_KERNEL_JACOBI && (K > 1 || out->reorder == 1))
         return fail(SPTRSV_E_INVALID_ARG, "the block walk (variant 5) takes one right-hand side and the matrix as given");
-    if (out->variant == 4 && out->kernel != SPTRSV_KERNEL_JACOBI &&
+    if ((out->variant == 4 || out->variant == 6) && out->kernel != SPTRSV_KERNEL_JACOBI &&
         (K > 1 || out->kernel == SPTRSV_KERNEL_SIMPLE || out->reorder == 1))
-        return fail(SPTRSV_E_INVALID_ARG, "the level walk (variant 4) takes ORDER or MULTIROW, one right-hand side and "
-                                          "the matrix as given");
+        return fail(SPTRSV_E_INVALID_ARG, "the level and packed walks (variants 4 and 6) take ORDER or MULTIROW, one "
+                                          "right-hand side and the matrix as given");
     if (out->variant == 3 && out->kernel != SPTRSV_KERNEL_JACOBI &&
         (K > 1 || out->kernel == SPTRSV_KERNEL_MULTIROW))
         return fail(SPTRSV_E_INVALID_ARG, "the in-degree walk (variant 3) takes SIMPLE or ORDER and one right-hand side");
@@ -396,7 +424,7 @@ KtPair kernel_timer_pair(hipStream_t, int launches, int kind) {
 // not split): multirow walks with one right-hand side over an analysis with
 // a segment table.
 static size_t split_part_words(const dfr_analysis_info_t* info, const sptrsv_config_t& c, int k) {
-    if (c.kernel != SPTRSV_KERNEL_MULTIROW || pow2_ceil(k) != 1 || !split_rows_on(c)) return 0;
+    if ((c.kernel != SPTRSV_KERNEL_MULTIROW && c.variant != 6) || pow2_ceil(k) != 1 || !split_rows_on(c)) return 0;
     const SegTable* sg = segments_of(info);
     return sg ? 2 * (size_t)sg->n_segs : 0;
 }
@@ -600,6 +628,8 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         c = shape_for(m, c.kernel, k);
     }
     // a trace is written by the walks row by row
+    const PackedWaves pw = c.variant == 6 ? packed_waves(info) : PackedWaves{};
+    if (c.variant == 6 && (pv->trace || !pw.base)) c = shape_for(m, c.kernel, k);
     if (c.variant == 5 && (pv->trace || !(pv->banded || pv->max_row <= kBlockRow + 1))) {
         c = shape_for(m, c.kernel, k);
         if (c.variant == 5) c.variant = 1;
@@ -649,8 +679,28 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         const int per_cu = c.cu_waves > 0 ? c.cu_waves : 4;
         A.persist_grid = (long long)device_cus() * std::max(1, per_cu / std::max(1, c.wg / kWave));
     }
-    // long rows split into segments: multirow walks, one right-hand side
-    const size_t part_words = split_part_words(info, c, k);
+    if (c.variant == 6) {
+        const PackedShape ps = packed_shape(pw.n, info->nlevs);
+        kind = ps.local ? KK_XCD_MULTIROW : KK_PERSIST_MULTIROW;
+        A.wbase = pw.base;
+        A.wsize = pw.size;
+        A.n_waves = pw.n;
+        A.dyn_lds = pv->lds_pad;
+        A.persist_grid = (long long)device_cus() * (ps.cu_waves / (ps.wg / kWave));
+        A.claim_rounds = 1;
+        c.wg = ps.wg;
+        c.lanes = 32;  // the layout's widest rows
+    }
+    // long rows split into segments: multirow walks, one right-hand side.  No
+    // partials can be allocated while the stream is captured: rows stay whole.
+    size_t part_words = split_part_words(info, c, k);
+    if (part_words && !part_ext && pv->part_words < part_words) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            part_words = 0;
+        }
+    }
     if (part_words) {
         const SegTable* sg = segments_of(info);
         if (!part_ext) SPT_TRY(reserve_part(m, info));
@@ -986,8 +1036,15 @@ int sptrsv_solve_mixed_noalloc(sp_mat_t* mat, dfr_analysis_info_t* info, const s
     // the published words, then (split long rows) the segment partials from
     // the next 256-byte boundary
     const size_t pub_words = (size_t)n * k;
-    const size_t part_words = split_part_words(info, c, k);
+    size_t part_words = split_part_words(info, c, k);
     const size_t part_at = (pub_words + 31) / 32 * 32;
+    // only a solve that names MULTIROW, or an analysis made for it, asks for
+    // split rows: others keep theirs whole where the partials find no room
+    if (part_at + part_words > (size_t)SPTRSV_NOALLOC_MAX_WORDS && c.variant == 6 &&
+        (c.kernel == SPTRSV_KERNEL_ORDER || (!named && info->mode == ALL))) {
+        c.split_rows = -1;
+        part_words = 0;
+    }
     if (part_words && part_at + part_words > (size_t)SPTRSV_NOALLOC_MAX_WORDS)
         return fail(SPTRSV_E_CAPACITY, "n * k plus the split rows' " + std::to_string(part_words) +
                                            " partial words exceed the allocation-free scratch of " +
@@ -1160,6 +1217,9 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
 
     // level by level in one workgroup, where a level is small
     if (K == 1 && has_order(info) && level_walk_fits(mat, info)) shapes.push_back({SPTRSV_KERNEL_ORDER, ref, 256, 1, 4, 0});
+    // the packed walk, which an ORDER analysis has no other shape for
+    if (K == 1 && has_order(info))
+        shapes.push_back({has_waves(info) ? SPTRSV_KERNEL_MULTIROW : SPTRSV_KERNEL_ORDER, ref, 256, 1, 6, 0});
     // blocks of 64 rows in natural order
     if (K == 1 && block_walk_fits(mat)) shapes.push_back({SPTRSV_KERNEL_SIMPLE, ref, 256, 1, 5, 0});
 

@@ -82,8 +82,10 @@ struct LevelPlan {
     void *structure = nullptr, *shared = nullptr, *kind[3] = {};
 };
 
+constexpr int kCounterWords = 8;
+
 struct MatPriv {
-    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4], [5] row shape, others spare (device)
+    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4], [5] row shape, [6] XCD of a packed walk, others spare (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
     size_t pub_words = 0;
     uint64_t* part = nullptr;    // published partial sums of long-row segments, 2 per segment (device)
@@ -183,6 +185,13 @@ struct SegTable {
 // The analysis's segment table, or null when it has none.
 const SegTable* segments_of(const dfr_analysis_info_t* info);
 int build_segments(dfr_analysis_info_t* info, sp_mat_t* m);
+// The wave64 layout of an analysis, whatever its mode (base null: none).
+struct PackedWaves {
+    const int* base = nullptr;
+    const int* size = nullptr;
+    int n = 0;
+};
+PackedWaves packed_waves(const dfr_analysis_info_t* info);
 // Identifies an analysis for the captured-solve cache: unique per analysis
 // built, loaded or copied (never reused); 0 for none.
 unsigned long long analysis_id(const dfr_analysis_info_t* info);

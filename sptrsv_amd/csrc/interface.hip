@@ -87,12 +87,12 @@ int ensure_priv(sp_mat_t* m) {
         rate > 0)
         pv->wall_rate_khz = rate;
     pv->watchdog_ticks = (long long)(watchdog_ms_default() * pv->wall_rate_khz);
-    hipError_t e = hipMalloc(&pv->counters, 8 * sizeof(int));
+    hipError_t e = hipMalloc(&pv->counters, kCounterWords * sizeof(int));
     if (e != hipSuccess) {
         delete pv;
         return hip_fail(e, "hipMalloc counters", __FILE__, __LINE__);
     }
-    SPT_HIP(hipMemset(pv->counters, 0, 8 * sizeof(int)));
+    SPT_HIP(hipMemset(pv->counters, 0, kCounterWords * sizeof(int)));
     m->priv = pv;
     std::lock_guard<std::mutex> g(g_live_mu);
     g_live.insert(pv);

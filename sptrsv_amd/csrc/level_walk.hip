@@ -525,11 +525,11 @@ __global__ __launch_bounds__(WG) void k_level_walk(LwArgs A) {
 // ---- host ------------------------------------------------------------------------------
 
 // A level's share of the matrix up to which one CU streaming it all beats the
-// walks that use the whole device: at 21 KB (random n = 15000 to 30000) 110 us
-// against 203 and 174 against 275, at 24 KB (2D grid 707^2) 0.79 ms against
-// 1.8; at 35 KB (random n = 10^6, whose plan no longer stays in the Infinity
-// Cache) 5.7 ms against 5.5.
-constexpr double kLwLevelBytes = 26.0 * 1024.0;
+// packed walk.  Rows of at most kLwU off-diagonals, a lane each: 0.60 ms against
+// 0.68 at 20 KB (2D grid 600^2), 0.79 against 0.80 at 23.5 (707^2), 1.31 against
+// 1.18 at 33 (1000^2).  Longer rows, spread over lanes with room left over: 55
+// us against 86 at 12 KB (random n = 10000), 114 against 102 at 15 (n = 15000).
+constexpr double kLwLevelBytes = 13.0 * 1024.0, kLwShortLevelBytes = 26.0 * 1024.0;
 constexpr long long kLwMaxEntries = 1ll << 27;  // buffer descriptors address 4 GB
 // Share of far entries above which the walk is not taken (their loads wait).
 constexpr double kLwFarShare = 0.01;
@@ -542,7 +542,8 @@ constexpr double kLwSliceBytes = 64.0 * (kLwU * 20 + 20 + 16), kLwPlanShare = 96
 bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     if (!info || !info->iorder || !info->inv_iorder || !info->bucket_off || !info->level || info->nlevs < 1) return false;
     if (info->n != m->nr || m->nr < 1 || m->nnz > kLwMaxEntries || !analysis_id(info)) return false;
-    return (12.0 * m->nnz + 32.0 * m->nr) / info->nlevs <= kLwLevelBytes;
+    const bool lane_rows = static_cast<const MatPriv*>(m->priv)->max_row <= kLwU + 1;
+    return (12.0 * m->nnz + 32.0 * m->nr) / info->nlevs <= (lane_rows ? kLwShortLevelBytes : kLwLevelBytes);
 }
 
 static void free_level_plan(LevelPlan& L) {

@@ -692,7 +692,7 @@ __device__ __forceinline__ int multirow_item(const SolveArgs& A, int t) { return
 __device__ __forceinline__ int multirow_items(const SolveArgs& A) { return A.items ? A.n_items : A.n_waves; }
 
 // A segment item of a split long row (defined with the lean walk below).
-template <class P, int U>
+template <class P, int U, bool LOCAL = false>
 __device__ __forceinline__ void fast_segment(const SolveArgs& A, int lane, int g);
 
 // (level, class) packed waves (multirow): wave w solves the rows at iorder
@@ -837,7 +837,14 @@ __device__ __forceinline__ void fold_entries(const SolveArgs& A, int L, int e, i
     }
 }
 
-template <class P, int U, bool SPLIT = false>
+// LOCAL: every wave that polls is on this wave's XCD.
+template <class T, bool LOCAL>
+__device__ __forceinline__ void publish(T* p, T v) {
+    if constexpr (LOCAL) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else publish_global(p, v);
+}
+
+template <class P, int U, bool SPLIT = false, bool LOCAL = false>
 __device__ __forceinline__ void fast_rows(const SolveArgs& A, int L, int lane, int row) {
     using word = typename P::word;
     using Acc = typename P::Acc;
@@ -907,14 +914,14 @@ __device__ __forceinline__ void fast_rows(const SolveArgs& A, int L, int lane, i
         typename P::Out o{};
         const word w = P::finish(A, dg, t, o);
         if (A.trace) A.trace[3 * xi + 2] = wall_clock64();
-        publish_global(&gpub[xi], w);
+        publish<word, LOCAL>(&gpub[xi], w);
         P::emit(A, caller_index(A, row, 0), o, w);
     }
 }
 
 // Segment item g of a split long row: the whole wave folds entries
 // [seg_lo[g], seg_hi[g]) from zero and publishes the partial sum.
-template <class P, int U>
+template <class P, int U, bool LOCAL>
 __device__ __forceinline__ void fast_segment(const SolveArgs& A, int lane, int g) {
     using Acc = typename P::Acc;
     const long long t0 = wall_clock64();
@@ -927,7 +934,7 @@ __device__ __forceinline__ void fast_segment(const SolveArgs& A, int lane, int g
         uint64_t w[P::kPartWords];
         P::part_pack(t, w);
 #pragma unroll
-        for (int i = 0; i < P::kPartWords; ++i) publish_global(&A.part[2 * (size_t)g + i], w[i]);
+        for (int i = 0; i < P::kPartWords; ++i) publish<uint64_t, LOCAL>(&A.part[2 * (size_t)g + i], w[i]);
     }
 }
 
@@ -1068,9 +1075,26 @@ __device__ __forceinline__ int claim_block(int* ctr, int items_per_block, int* s
     return *s_slot;
 }
 
-template <class P, int WG, int U, int MODE>
+//
+// LOCAL: the same walk by the workgroups of one XCD; those that land on another
+// leave at once (the first to arrive chooses).  A hand-off from one XCD to
+// another takes 365 ns at best, the store going to memory and the poll past
+// the L2; inside one XCD a plain store is in the L2 that every CU polls, and it
+// takes 211 ns.  Where the rows of a level keep 32 CUs busy and no more, that
+// is what counts (MULTIROW solve, whole device -> one XCD: random n = 10^6, 253
+// rows per level, 5.7 -> 2.8 ms; n = 30000 274 -> 143 us).
+template <class P, int WG, int U, int MODE, bool LOCAL = false>
 __global__ __launch_bounds__(WG) void k_persist(SolveArgs A) {
     __shared__ int s_base;
+    if constexpr (LOCAL) {
+        if (threadIdx.x == 0) {
+            const int me = 1 + (__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15);  // HW_REG_XCC_ID
+            const int old = atomicCAS(A.ticket + 6, 0, me);
+            s_base = old == 0 || old == me;
+        }
+        __syncthreads();
+        if (!s_base) return;
+    }
     constexpr int NW = WG / kWave;
     const int wv = threadIdx.x >> 6;
     const int lane = threadIdx.x & (kWave - 1);
@@ -1082,7 +1106,7 @@ __global__ __launch_bounds__(WG) void k_persist(SolveArgs A) {
             if constexpr (MODE == 2) {
                 const int w = multirow_item(A, t);
                 if (w < 0) {
-                    fast_segment<P, U>(A, lane, -w - 1);
+                    fast_segment<P, U, LOCAL>(A, lane, -w - 1);
                     continue;
                 }
                 const int vs = A.wsize[w];
@@ -1090,10 +1114,10 @@ __global__ __launch_bounds__(WG) void k_persist(SolveArgs A) {
                 const int wb = A.wbase[w];
                 const int seg = lane / L;
                 const int row = seg < A.wbase[w + 1] - wb ? A.iorder[wb + seg] : -1;
-                fast_rows<P, U, true>(A, L, lane, row);
+                fast_rows<P, U, true, LOCAL>(A, L, lane, row);
             } else {
                 const int row = (MODE == 1) ? A.iorder[t] : t;
-                fast_rows<P, U>(A, A.L, lane, lane < A.L ? row : -1);
+                fast_rows<P, U, false, LOCAL>(A, A.L, lane, lane < A.L ? row : -1);
             }
         }
     }
@@ -1153,7 +1177,10 @@ __global__ void k_prepare(T* pub, size_t count, T unsolved, int* ticket, uint64_
                           const int* ia, int* indeg, int n_indeg) {
     const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    if (i0 == 0) *ticket = 0;
+    if (i0 == 0) {
+        *ticket = 0;
+        ticket[6] = 0;  // XCD of a LOCAL walk
+    }
     for (size_t i = i0; i < count; i += stride) pub[i] = unsolved;
     for (size_t i = i0; i < part_count; i += stride) part[i] = kUnsolved64;
     for (size_t i = i0; i < (size_t)n_indeg; i += stride) indeg[i] = ia[i + 1] - ia[i] - 1;
@@ -1172,6 +1199,7 @@ enum KernelKind {
     KK_PERSIST_MULTIROW = 9,  // persistent walk over multirow waves (lean for K == 1)
     KK_INDEG_SIMPLE = 10,     // in-degree walk, natural order (K == 1)
     KK_INDEG_ORDER = 11,      // in-degree walk, level order (K == 1)
+    KK_XCD_MULTIROW = 12,     // KK_PERSIST_MULTIROW by the workgroups of one XCD (K == 1)
 };
 
 // Launch of a persistent kernel with A.persist_grid workgroups, clamped to
@@ -1228,6 +1256,8 @@ hipError_t launch_k(int kind, const SolveArgs& A, hipStream_t s) {
                 return launch_persist<P, WG, U, 1>(A, s);
             case KK_PERSIST_MULTIROW:
                 return launch_persist<P, WG, U, 2>(A, s);
+            case KK_XCD_MULTIROW:
+                return launch_persistent(&k_persist<P, WG, U, 2, true>, WG, A, s);
             case KK_INDEG_SIMPLE:
                 hipLaunchKernelGGL((k_indeg<P, WG, U, false>), dim3(grid), dim3(WG), A.dyn_lds, s, A);
                 return hipGetLastError();
