@@ -178,6 +178,7 @@ bool block_walk_fits(const sp_mat_t* m) {
 // waves per CU, 1.6 with 16); on the whole device likewise, up to 400 (3D grid
 // 128^3, 340 waves: 643 us with 4 per CU, 766 with 16; power-law n = 2*10^6, 730
 // waves: 1.09 ms and 0.76).
+constexpr int kXcds = 8;
 struct PackedShape {
     bool local;  // one XCD
     int wg, cu_waves;
@@ -203,6 +204,22 @@ static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_
         else if (level_walk_fits(m, info)) c.variant = 4;
         else if (packed_waves(info).base) c.variant = 6;
     }
+    if (kernel == SPTRSV_KERNEL_ORDER && k > 1 && info && info->nlevs > 0) {
+        // the persistent walk, with as many entry lanes as rows have entries
+        // while that leaves at most 1100 waves a level (3D grid 40^3, 2
+        // right-hand sides, 1 -> 4 lanes: 212 -> 100 us; 128^3, 16: 1372 waves,
+        // 0.98 -> 1.28 ms with two lanes); short rows rather stay on one XCD
+        // (128 waves; 60^3, 4: 254 us with one lane, 331 with two)
+        const int K = pow2_ceil(k), avg = m->nnz / m->nr;
+        const double waves = (double)m->nr / info->nlevs * K / kWave;
+        const double most = avg < 8 && waves <= 128.0 ? 128.0 : 1100.0;
+        c.variant = 2;
+        c.wg = 1024;
+        c.cu_waves = 16;
+        c.lanes = 1;
+        while (2 * c.lanes * K <= kWave && 2 * c.lanes <= avg && 2 * c.lanes * waves <= most)
+            c.lanes *= 2;
+    }
     return c;
 }
 
@@ -212,6 +229,9 @@ int default_config(const sp_mat_t* m, const dfr_analysis_info_t* info, int preci
     int kernel = SPTRSV_KERNEL_SIMPLE;
     if (info && info->mode == ORDER && has_order(info)) kernel = SPTRSV_KERNEL_ORDER;
     if (info && info->mode == MULTIROW && has_waves(info)) kernel = SPTRSV_KERNEL_MULTIROW;
+    // several right-hand sides walk in level order whichever analysis it is: the
+    // 64-lane layout is made for one (16, 3D grid 128^3: 10.9 ms against 0.98)
+    if (k > 1 && has_order(info)) kernel = SPTRSV_KERNEL_ORDER;
     *out = analysed_shape_for(m, info, kernel, k);
     // an ALL analysis asks for no kernel, and may be there for one solve only:
     // the packed walk, which needs no plan, or natural order for a chain
@@ -245,6 +265,7 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
             out->lanes = d.lanes;
             if (cfg->variant == 0) out->variant = d.variant;
             if (cfg->wg <= 0) out->wg = d.wg;
+            if (shape_open(*cfg) && k > 1) out->cu_waves = d.cu_waves;
         }
     } else if (pv->tuned[precision] && pv->tuned_k[precision] == k &&
                (pv->tuned_cfg[precision].kernel == SPTRSV_KERNEL_SIMPLE ||
@@ -691,6 +712,21 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         c.wg = ps.wg;
         c.lanes = 32;  // the layout's widest rows
     }
+    const int u = c.window > 0 ? c.window : window_for(pv, (kind == KK_MULTIROW || kind == KK_FAST_MULTIROW) ? 32 : c.lanes);
+    // Several right-hand sides in level order: on one XCD while its 32 CUs hold
+    // at least four times the waves of a level (waves of a level / waves held,
+    // whole device -> one XCD: 54 / 512 1317 -> 875 us, 19 / 128 156 -> 106, 76 /
+    // 256 332 -> 293; but 54 / 128 996 -> 1222 and 108 / 256 910 -> 988) and its
+    // L2 the words a level reads (0.25 MB 1172 -> 895 us, 0.55 MB 3.24 -> 3.38 ms).
+    if (K > 1 && kind == KK_PERSIST_ORDER && info->nlevs > 0) {
+        const double level = (double)A.n * (K * c.lanes) / kWave / info->nlevs;
+        const double words = (double)m->nnz * K * sizeof(typename P::word) / info->nlevs;
+        const long long held = A.persist_grid / kXcds * (c.wg / kWave);
+        A.local = 4 * level <= (double)held && words <= 400e3;
+        A.short_rows = pv->max_row - 1 <= u * c.lanes;
+        // of longer rows, levels count where two items fit in one
+        if (A.short_rows || 2 * kWave * (long long)info->nlevs <= (long long)A.n * K * c.lanes) A.level = info->level;
+    }
     // long rows split into segments: multirow walks, one right-hand side.  No
     // partials can be allocated while the stream is captured: rows stay whole.
     size_t part_words = split_part_words(info, c, k);
@@ -717,7 +753,6 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
                        static_cast<word*>(pub), words, P::kUnsolved, pv->counters, A.part, part_words, sm->ia,
                        A.indeg, A.indeg ? m->nr : 0);
     SPT_HIP(hipGetLastError());
-    int u = c.window > 0 ? c.window : window_for(pv, (kind == KK_MULTIROW || kind == KK_FAST_MULTIROW) ? 32 : c.lanes);
     const KtPair ev = timed ? kernel_timer_pair(s) : KtPair{};
     if (ev) SPT_HIP(hipEventRecord(ev[0], s));
     const hipError_t e = c.variant == 5 ? launch_block_rows<P>(A, block_walk_in_order(m), pv->max_row - 1, s) : launch_solve<P, 64>(kind, K, c.wg, u, A, s);

@@ -49,6 +49,7 @@ struct SolveArgs {
     void* pub;              // published words, n*k (x itself for F64/F32)
     double* x_out;          // MIXED: FP64 solution n*k
     const int* iorder;      // ORDER / MULTIROW
+    const int* level;       // of each row (ORDER; null: not asked for)
     const int* wbase;       // MULTIROW: first iorder position of each wave
     const int* wsize;       // MULTIROW: lanes per row of each wave (0 = diagonal only)
     int n_waves;            // MULTIROW
@@ -62,6 +63,9 @@ struct SolveArgs {
     unsigned dyn_lds;       // extra LDS bytes per workgroup (caps resident waves; unused by the kernels)
     long long persist_grid; // persistent kernels: workgroups to launch
     int claim_rounds;       // persistent kernels: items per wave in each claimed block
+    // persistent walk in level order, several right-hand sides: by one XCD only;
+    // every row in one window of its lanes
+    int local, short_rows;
     // long-row segments of the multirow walks, one right-hand side (null
     // items: rows are never split)
     const int* items;       // walk order: wave w >= 0, segment g as -(g + 1)
@@ -99,6 +103,11 @@ __device__ __forceinline__ T poll_global(const T* p) {
 template <class T>
 __device__ __forceinline__ void publish_global(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// For readers on this XCD: a plain store, which stays in its L2.
+template <class T>
+__device__ __forceinline__ void publish_near(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 template <class T>
 __device__ __forceinline__ T poll_lds(const T* p) {
@@ -605,7 +614,8 @@ __device__ __forceinline__ void sf_rows(const SolveArgs& A, int L, int lane, int
             const typename P::Out so = pending ? pend_o : P::bcast_out(pend_o, src);
             if (pending && row >= lds_lo && row < lds_hi) publish_lds(&s_pub[row - lds_lo], pend_w);
             if (A.trace && pending) A.trace[3 * xi + 2] = wall_clock64();
-            publish_global(&gpub[sxi], sw);
+            if (K > 1 && A.local) publish_near(&gpub[sxi], sw);
+            else publish_global(&gpub[sxi], sw);
             P::emit(A, sbi, so, sw);  // x in the caller's order: nobody waits on it
             pending = false;
             asm volatile("" ::: "memory");
@@ -740,12 +750,15 @@ __global__ __launch_bounds__(WG) void k_multirow(SolveArgs A) {
 // Folds entries [lo, hi) into acc: lane e of a group of L lanes takes
 // entries lo + e, lo + e + L, ... in that order, in chunks of U whose
 // dependencies are all present before the chunk is folded.
-template <class P, int U>
+// With K right-hand sides lane r of the K of an entry takes column r of the
+// dependency's row.
+template <class P, int U, int K = 1>
 __device__ __forceinline__ void fold_entries(const SolveArgs& A, int L, int e, int lane, bool live, int lo, int hi,
-                                             typename P::Acc& acc, long long t0, bool& expired, int& spins) {
+                                             typename P::Acc& acc, long long t0, bool& expired, int& spins, int r = 0) {
     using word = typename P::word;
     using Val = typename P::Val;
     const word* gpub = static_cast<const word*>(A.pub);
+    auto at = [&](int c) { return K == 1 ? (size_t)c : (size_t)c * A.k + r; };
     // Entries of the next chunk are loaded before the current chunk is
     // polled (chunks of up to 4 entries per lane), so a long row pays the
     // entry-load latency once, not per chunk.
@@ -798,7 +811,7 @@ __device__ __forceinline__ void fold_entries(const SolveArgs& A, int L, int e, i
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 w[u] = P::kUnsolved;
-                if (pend[u]) w[u] = poll_global(&gpub[col[u]]);
+                if (pend[u]) w[u] = poll_global(&gpub[at(col[u])]);
             }
             bool any = false;
 #pragma unroll
@@ -840,7 +853,7 @@ __device__ __forceinline__ void fold_entries(const SolveArgs& A, int L, int e, i
 // LOCAL: every wave that polls is on this wave's XCD.
 template <class T, bool LOCAL>
 __device__ __forceinline__ void publish(T* p, T v) {
-    if constexpr (LOCAL) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if constexpr (LOCAL) publish_near(p, v);
     else publish_global(p, v);
 }
 
@@ -935,6 +948,42 @@ __device__ __forceinline__ void fast_segment(const SolveArgs& A, int lane, int g
         P::part_pack(t, w);
 #pragma unroll
         for (int i = 0; i < P::kPartWords; ++i) publish<uint64_t, LOCAL>(&A.part[2 * (size_t)g + i], w[i]);
+    }
+}
+
+// Rows of one level, several right-hand sides: a group of L entry lanes x K
+// right-hand-side lanes per row (lane e * K + r), as sf_rows lays it out.  No
+// row waits for another of the wave, so the lean polling turn serves (16
+// right-hand sides, 3D grid 128^3: 1.11 -> 0.98 ms).
+template <class P, int K, int U>
+__device__ __forceinline__ void level_rows(const SolveArgs& A, int L, int lane, int row) {
+    using word = typename P::word;
+    using Acc = typename P::Acc;
+    word* gpub = static_cast<word*>(A.pub);
+    const int G = L * K, e = (lane & (G - 1)) / K, r = lane & (K - 1);
+    const bool live = row >= 0 && r < A.k;
+    int rs = 0, dpos = 0;
+    if (live) {
+        rs = A.ia[row];
+        dpos = A.ia[row + 1] - 1;
+    }
+    const bool lead = live && e == 0;
+    const size_t xi = (size_t)(live ? row : 0) * A.k + r;
+    const size_t bi = live ? caller_index(A, row, r) : 0;
+    Acc acc = lead ? P::seed(A, bi) : P::zero();
+    typename P::Diag dg{};
+    if (lead) dg = P::diag(A, dpos);
+    const long long t0 = wall_clock64();
+    bool expired = false;
+    int spins = 0;
+    fold_entries<P, U, K>(A, L, e, lane, live, rs, dpos, acc, t0, expired, spins, r);
+    const Acc t = group_reduce<P, K>(acc, G);
+    if (lead) {
+        typename P::Out o{};
+        const word w = P::finish(A, dg, t, o);
+        if (A.local) publish_near(&gpub[xi], w);
+        else publish_global(&gpub[xi], w);
+        P::emit(A, bi, o, w);
     }
 }
 
@@ -1075,9 +1124,20 @@ __device__ __forceinline__ int claim_block(int* ctr, int items_per_block, int* s
     return *s_slot;
 }
 
-//
+// Whether this workgroup is on the XCD of a walk by one XCD only: the first to
+// arrive chooses it.
+__device__ __forceinline__ bool on_chosen_xcd(const SolveArgs& A, int* s_slot) {
+    if (threadIdx.x == 0) {
+        const int me = 1 + (__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15);  // HW_REG_XCC_ID
+        const int old = atomicCAS(A.ticket + 6, 0, me);
+        *s_slot = old == 0 || old == me;
+    }
+    __syncthreads();
+    return *s_slot != 0;
+}
+
 // LOCAL: the same walk by the workgroups of one XCD; those that land on another
-// leave at once (the first to arrive chooses).  A hand-off from one XCD to
+// leave at once.  A hand-off from one XCD to
 // another takes 365 ns at best, the store going to memory and the poll past
 // the L2; inside one XCD a plain store is in the L2 that every CU polls, and it
 // takes 211 ns.  Where the rows of a level keep 32 CUs busy and no more, that
@@ -1086,15 +1146,7 @@ __device__ __forceinline__ int claim_block(int* ctr, int items_per_block, int* s
 template <class P, int WG, int U, int MODE, bool LOCAL = false>
 __global__ __launch_bounds__(WG) void k_persist(SolveArgs A) {
     __shared__ int s_base;
-    if constexpr (LOCAL) {
-        if (threadIdx.x == 0) {
-            const int me = 1 + (__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15);  // HW_REG_XCC_ID
-            const int old = atomicCAS(A.ticket + 6, 0, me);
-            s_base = old == 0 || old == me;
-        }
-        __syncthreads();
-        if (!s_base) return;
-    }
+    if (LOCAL && !on_chosen_xcd(A, &s_base)) return;
     constexpr int NW = WG / kWave;
     const int wv = threadIdx.x >> 6;
     const int lane = threadIdx.x & (kWave - 1);
@@ -1133,6 +1185,7 @@ __global__ __launch_bounds__(WG) void k_persist(SolveArgs A) {
 template <class P, int K, int WG, int U, int MODE>
 __global__ __launch_bounds__(WG) void k_persist_rows(SolveArgs A) {
     __shared__ int s_base;
+    if (A.local && !on_chosen_xcd(A, &s_base)) return;
     constexpr int NW = WG / kWave;
     const int wv = threadIdx.x >> 6;
     const int lane = threadIdx.x & (kWave - 1);
@@ -1163,6 +1216,28 @@ __global__ __launch_bounds__(WG) void k_persist_rows(SolveArgs A) {
             for (int j = wv; j < B && b0 + j < items; j += NW) {
                 const int pos = (b0 + j) * rpw + (lane >> lgG);
                 const int row = pos < A.n ? (MODE == 1 ? A.iorder[pos] : pos) : -1;
+                if constexpr (MODE == 1 && K > 1) {
+                    // Short rows go one level at a time: an item that reaches
+                    // into the next level (as at every level's end) solved by
+                    // the general engine held up that level (3D grid 30^3, 3
+                    // right-hand sides, on one XCD: 158 -> 121 us).  Rows longer
+                    // than a window wait for it several times over, and several
+                    // levels of them one after the other cost more than that
+                    // (random n = 4000, 2 right-hand sides: 228 -> 285 us).
+                    if (!A.trace && A.level) {
+                        const int lev = row >= 0 ? A.level[row] : 0;
+                        uint64_t todo = __ballot(row >= 0);
+                        const int l0 = __builtin_amdgcn_readfirstlane(lev);
+                        if (A.short_rows || !__ballot(row >= 0 && lev != l0)) {
+                            while (todo) {
+                                const bool in = row >= 0 && lev == __builtin_amdgcn_readlane(lev, __builtin_ctzll(todo));
+                                level_rows<P, K, U>(A, A.L, lane, in ? row : -1);
+                                todo &= ~__ballot(in);
+                            }
+                            continue;
+                        }
+                    }
+                }
                 sf_rows<P, K, U>(A, A.L, lane, row, nullptr, 0, 0);
             }
         }
