@@ -291,16 +291,21 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * of the analysis's 64-lane layout, by the workgroups of one XCD where a level
  * has few rows, with a workgroup size and wave count of its own (a traced
  * solve takes the lean path; rows are split as for MULTIROW, but stay whole
- * where the stream is captured before the partial sums' workspace exists);
- * cu_waves caps the waves
+ * where the stream is captured before the partial sums' workspace exists); 7 is
+ * the group walk (one right-hand side, natural order whatever the kernel): lanes
+ * per row as given, every row of a wave publishing on its own, by the workgroups
+ * of one XCD with 16 waves per CU (a traced solve takes the lean path); cu_waves
+ * caps the waves
  * resident per CU (0 = hardware limit): every resident wave polls, and past a
  * few thousand polling waves the dependency hand-off latency grows several
  * fold, so deep dependency chains run fastest with a small cap.  With lanes
  * = 0 the lanes (and, when variant is 0, the variant) come from the tuned
  * shape of the kernel, else from the default shape (SIMPLE: the block walk for
- * banded matrices and grid-like ones, else the lean path; ORDER and MULTIROW:
- * the level walk where a level's share of the matrix is small, else the packed
- * walk); MULTIROW takes its lanes
+ * banded matrices and grid-like ones, the group walk where rows depend on rows
+ * up to some thousands back, else variants 0 or 2; ORDER and MULTIROW: the level
+ * walk where a level's share of the matrix is small, else the group or the
+ * packed walk; several right-hand sides with an analysis: variant 2 of ORDER);
+ * MULTIROW takes its lanes
  * per row from the analysis and ignores a nonzero lanes. */
 typedef struct {
     int kernel;

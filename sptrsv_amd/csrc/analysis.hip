@@ -31,6 +31,7 @@
 namespace sptrsv {
 
 unsigned lds_pad_for(int cu_waves, int wg);
+int device_cus();
 
 // Tile of the level pass from the integer average nnz/n, as
 // aux_call_kernel_analysis_L_coop_groups picks it (analysis_csr.cu:215-240):
@@ -628,9 +629,10 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     // entries) take one lane per row on the general engine: 64 consecutive
     // rows per wave keep many more rows in flight, which a natural-order walk
     // of a grid-like matrix needs to find ready rows.  Other matrices keep
-    // the reference's tile rule.  Before all these, the block walk where it is
-    // the natural-order solve's default.
+    // the reference's tile rule.  Before all these, the block walk or the group
+    // walk where it is the natural-order solve's default.
     const bool blocks = block_walk_fits(m);
+    const int group_lanes = group_walk_lanes(m);
     int kind = KK_SIMPLE;
     unsigned dyn_lds = 0;
     const int avg = n > 0 ? m->nnz / n : 0;
@@ -642,6 +644,11 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         dyn_lds = lds_pad_for(4, wg);
     } else if (avg < 6 && pv->max_row <= 64) {
         lanes = 1;
+    }
+    if (group_lanes) {
+        kind = KK_XCD_SIMPLE;
+        lanes = group_lanes;
+        wg = 1024;
     }
     {
         SolveArgs A{};
@@ -657,7 +664,9 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         A.ticket = pv->counters;
         A.err = pv->counters + 1;
         A.wd_ticks = pv->watchdog_ticks;
-        A.dyn_lds = blocks ? 0 : dyn_lds;
+        A.dyn_lds = blocks || group_lanes ? 0 : dyn_lds;
+        A.persist_grid = device_cus();
+        A.claim_rounds = 1;
         hipLaunchKernelGGL((k_prepare<uint32_t>), dim3(grid_for(n)), dim3(256), 0, s,
                            reinterpret_cast<uint32_t*>(info->level), (size_t)n, 0u, pv->counters, nullptr,
                            (size_t)0, nullptr, nullptr, 0);

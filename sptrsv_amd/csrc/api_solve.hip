@@ -121,6 +121,7 @@ static int window_for(const MatPriv* pv, int lanes) { return (pv->max_row > 2 * 
 // takes the lean path (one row per wave for SIMPLE/ORDER, with lanes covering
 // a typical row: the next power of two >= nnz/n, 4..64); several take the
 // general engine with the reference's lanes rule.
+static void simple_shape(const sp_mat_t* m, sptrsv_config_t* c);
 static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
     sptrsv_config_t c{};
     c.kernel = kernel;
@@ -131,7 +132,7 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
         c.variant = 1;
         int avg = m->nr > 0 ? m->nnz / m->nr : 1;
         c.lanes = std::min(kWave, std::max(4, pow2_ceil(avg)));
-        if (kernel == SPTRSV_KERNEL_SIMPLE && block_walk_fits(m)) c.variant = 5;
+        if (kernel == SPTRSV_KERNEL_SIMPLE) simple_shape(m, &c);
     } else {
         c.variant = 0;
         int lanes = reference_lanes(m);
@@ -165,19 +166,61 @@ bool block_walk_in_order(const sp_mat_t* m) {
 
 bool block_walk_fits(const sp_mat_t* m) {
     const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
-    if (!pv->banded) return pv->near_rows && pv->max_row <= kBlockRow + 1;
+    // (3D grid 10^3: 34.6 us against 30.0, 14^3: 45.5 against 50.3)
+    if (!pv->banded) return pv->near_rows && pv->max_row <= kBlockRow + 1 && m->nr >= 2500;
     return pv->near_rows || m->nr < kBandRows * std::max(pv->band_levels, 1) || m->nr >= kWideRows * pv->band_levels;
 }
 
+// Natural order, one right-hand side.
+//  * Blocks of 64 rows where block_walk_fits says so.
+//  * Where rows depend on rows up to some thousands back, the group walk: a
+//    chain sets the pace, and one XCD's waves hold the rows that can be solved
+//    (nearest dependency 620 rows back, n = 10^6: 5.84 -> 2.04 ms against a row
+//    per wave on the whole device; 1340 back, n = 3*10^5: 875 -> 315 us).  Eight
+//    lanes a row serve rows of 4 to 40 entries within 8 % of the best; long
+//    rows take 32 (power-law n = 6000, 116 -> 80 us, 16 lanes 102; n = 9000, 1600
+//    back, no better than what follows).
+//  * Further back it is the rows in flight that count: several rows per wave
+//    (5700 back, n = 3*10^5: 863 -> 331 us; power-law n = 10^6 2.92 -> 0.73 ms),
+//    with long rows, which the others of their wave wait for, only from further
+//    on (n = 10^5, 18000 back: 367 -> 287 us; 3*10^4, 5400 back: 176 either way).
+//  * What is left: a row per wave, 4 polling waves per CU, which hand over
+//    sooner than as many as fit (power-law n = 3*10^4 176 -> 152 us) unless few
+//    rows need no claims either (3D grid 10^3 30.3 against 29.6 us).
+constexpr int kGroupLanes = 8;
+static void simple_shape(const sp_mat_t* m, sptrsv_config_t* c) {
+    const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
+    const bool long_rows = pv->max_row > 256;
+    if (block_walk_fits(m)) {
+        c->variant = 5;
+    } else if (!pv->near_rows && pv->nearest < (long_rows ? 1500.0 : 2000.0)) {
+        c->variant = 7;
+        c->lanes = long_rows ? 32 : kGroupLanes;
+    } else if (pv->nearest >= (long_rows ? 12000.0 : 2000.0)) {
+        c->variant = 0;
+        c->wg = 1024;
+    } else if (m->nr >= 2500) {
+        c->variant = 2;
+        c->cu_waves = 4;
+        if (long_rows) c->lanes = kWave;
+    }
+}
+
+int group_walk_lanes(const sp_mat_t* m) {
+    sptrsv_config_t c{};
+    simple_shape(m, &c);
+    return c.variant == 7 ? c.lanes : 0;
+}
+
 // Where and how wide the packed walk (variant 6) runs, by the waves of a level.
-// Up to 100 the 32 CUs of one XCD have enough to do: 30 to 46 waves (random, n =
-// 3*10^4 to 10^6) 143 -> 2.8 ms against 274 us -> 5.7 ms on the whole device, 58
-// (power-law, n = 10^5) 204 against 241 us, 75 (3D grid 60^3) 161 against 250 us,
-// but 145 (power-law, n = 3*10^5) 418 against 306 us.  With less than 20 waves
-// the fewer pollers hand over sooner (2D grid 1000^2, 17 waves: 1.18 ms with 4
-// waves per CU, 1.6 with 16); on the whole device likewise, up to 400 (3D grid
-// 128^3, 340 waves: 643 us with 4 per CU, 766 with 16; power-law n = 2*10^6, 730
-// waves: 1.09 ms and 0.76).
+// Up to 100 the 32 CUs of one XCD have enough to do: 29 to 46 waves (random, n =
+// 3*10^4 to 10^6) 129 us -> 2.47 ms against 245 us -> 4.93 ms on the whole device,
+// 58 (power-law, n = 10^5) 199 against 254 us, 75 (3D grid 60^3) 165 against 248
+// us, but 145 (power-law, n = 3*10^5) 412 against 318 us.  With less than 20 waves
+// the fewer pollers hand over sooner (2D grid 1000^2, 17 waves: 1.08 ms with 4
+// waves per CU, 1.33 with 16); on the whole device likewise, up to 400 (3D grid
+// 128^3, 340 waves: 629 us with 4 per CU, 798 with 16; power-law n = 2*10^6, 730
+// waves: 1.10 ms and 0.77).
 constexpr int kXcds = 8;
 struct PackedShape {
     bool local;  // one XCD
@@ -192,10 +235,14 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 }
 
 // The same with the analysis at hand: ORDER and MULTIROW solves with one
-// right-hand side take the level walk where it fits, else the packed walk; for
-// banded matrices with less than four rows per level the block walk: it takes
-// about 40 ns a row, the level walk 170 to 200 ns a level (bandwidth 9, n =
-// 5000: 0.21 ms against 1.00).
+// right-hand side take the level walk where it fits, else the packed walk.  Two
+// kinds of matrices keep natural order all the same: banded ones with less than
+// four rows per level the block walk, which takes about 40 ns a row, the level
+// walk 170 to 200 ns a level (bandwidth 9, n = 5000: 0.21 ms against 1.00); and
+// where the packed walk would stay on one XCD, rows of up to 64 entries the
+// group walk, whose lanes read consecutive rows (random n = 10^6 2.04 against
+// 2.47 ms, n = 3*10^4 109 against 129 us; 20 entries of the last 3000, n =
+// 3*10^5, 2.45 against 2.81 ms).
 constexpr long long kChainRows = 4;
 static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
     sptrsv_config_t c = shape_for(m, kernel, k);
@@ -203,6 +250,12 @@ static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_
         if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;
         else if (level_walk_fits(m, info)) c.variant = 4;
         else if (packed_waves(info).base) c.variant = 6;
+        const int lanes = group_walk_lanes(m);
+        if (c.variant == 6 && lanes && priv_of(const_cast<sp_mat_t*>(m))->max_row <= 65 &&
+            packed_shape(packed_waves(info).n, info->nlevs).local) {
+            c.variant = 7;
+            c.lanes = lanes;
+        }
     }
     if (kernel == SPTRSV_KERNEL_ORDER && k > 1 && info && info->nlevs > 0) {
         // the persistent walk, with as many entry lanes as rows have entries
@@ -235,9 +288,10 @@ int default_config(const sp_mat_t* m, const dfr_analysis_info_t* info, int preci
     *out = analysed_shape_for(m, info, kernel, k);
     // an ALL analysis asks for no kernel, and may be there for one solve only:
     // the packed walk, which needs no plan, or natural order for a chain
-    if (k == 1 && info && info->mode == ALL && has_waves(info) && analysed_shape_for(m, info, SPTRSV_KERNEL_MULTIROW, k).variant != 5) {
-        *out = shape_for(m, SPTRSV_KERNEL_MULTIROW, k);
-        out->variant = 6;
+    if (k == 1 && info && info->mode == ALL && has_waves(info)) {
+        *out = analysed_shape_for(m, info, SPTRSV_KERNEL_MULTIROW, k);
+        if (out->variant == 4) out->variant = 6;
+        if (out->variant != 6) out->kernel = SPTRSV_KERNEL_SIMPLE;
     }
     return SPTRSV_OK;
 }
@@ -258,14 +312,15 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
             // lanes not given: those of the tuned shape for the kernel, else
             // of the default shape; so is the variant unless one is named
             const sptrsv_config_t& t = pv->tuned_cfg[precision];
-            sptrsv_config_t d = (pv->tuned[precision] && pv->tuned_k[precision] == k && t.kernel == cfg->kernel)
-                                    ? t
-                                    : shape_open(*cfg) ? analysed_shape_for(m, info, cfg->kernel, k)
-                                                       : shape_for(m, cfg->kernel, k);
+            const bool tuned = pv->tuned[precision] && pv->tuned_k[precision] == k && t.kernel == cfg->kernel;
+            const bool open = shape_open(*cfg) && !tuned;
+            sptrsv_config_t d = tuned ? t
+                                : open ? analysed_shape_for(m, info, cfg->kernel, k)
+                                       : shape_for(m, cfg->kernel, k);
             out->lanes = d.lanes;
             if (cfg->variant == 0) out->variant = d.variant;
             if (cfg->wg <= 0) out->wg = d.wg;
-            if (shape_open(*cfg) && k > 1) out->cu_waves = d.cu_waves;
+            if (open) out->cu_waves = d.cu_waves;
         }
     } else if (pv->tuned[precision] && pv->tuned_k[precision] == k &&
                (pv->tuned_cfg[precision].kernel == SPTRSV_KERNEL_SIMPLE ||
@@ -326,10 +381,11 @@ static int resolve_config(sp_mat_t* m, dfr_analysis_info_t* info, int precision,
         return fail(SPTRSV_E_INVALID_ARG, "unknown kernel");
     if (out->kernel == SPTRSV_KERNEL_JACOBI && precision != SPTRSV_PREC_MIXED)
         return fail(SPTRSV_E_INVALID_ARG, "JACOBI is the bulk solver of the MIXED path only");
-    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 6))
-        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..6");
-    if (out->variant == 5 && out->kernel != SPTRSV_KERNEL_JACOBI && (K > 1 || out->reorder == 1))
-        return fail(SPTRSV_E_INVALID_ARG, "the block walk (variant 5) takes one right-hand side and the matrix as given");
+    if (out->kernel != SPTRSV_KERNEL_JACOBI && (out->variant < 0 || out->variant > 7))
+        return fail(SPTRSV_E_INVALID_ARG, "variant must be 0..7");
+    if ((out->variant == 5 || out->variant == 7) && out->kernel != SPTRSV_KERNEL_JACOBI && (K > 1 || out->reorder == 1))
+        return fail(SPTRSV_E_INVALID_ARG, "the block and group walks (variants 5 and 7) take one right-hand side and "
+                                          "the matrix as given");
     if ((out->variant == 4 || out->variant == 6) && out->kernel != SPTRSV_KERNEL_JACOBI &&
         (K > 1 || out->kernel == SPTRSV_KERNEL_SIMPLE || out->reorder == 1))
         return fail(SPTRSV_E_INVALID_ARG, "the level and packed walks (variants 4 and 6) take ORDER or MULTIROW, one "
@@ -446,6 +502,7 @@ KtPair kernel_timer_pair(hipStream_t, int launches, int kind) {
 // a segment table.
 static size_t split_part_words(const dfr_analysis_info_t* info, const sptrsv_config_t& c, int k) {
     if ((c.kernel != SPTRSV_KERNEL_MULTIROW && c.variant != 6) || pow2_ceil(k) != 1 || !split_rows_on(c)) return 0;
+    if (c.variant == 5 || c.variant == 7) return 0;  // natural order, rows whole
     const SegTable* sg = segments_of(info);
     return sg ? 2 * (size_t)sg->n_segs : 0;
 }
@@ -650,10 +707,11 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
     }
     // a trace is written by the walks row by row
     const PackedWaves pw = c.variant == 6 ? packed_waves(info) : PackedWaves{};
-    if (c.variant == 6 && (pv->trace || !pw.base)) c = shape_for(m, c.kernel, k);
-    if (c.variant == 5 && (pv->trace || !(pv->banded || pv->max_row <= kBlockRow + 1))) {
+    // a trace is written by the walks row by row
+    if ((c.variant >= 5 && pv->trace) || (c.variant == 6 && !pw.base) ||
+        (c.variant == 5 && !pv->banded && pv->max_row > kBlockRow + 1)) {
         c = shape_for(m, c.kernel, k);
-        if (c.variant == 5) c.variant = 1;
+        if (c.variant >= 5) c.variant = 1;
     }
     const sp_mat_t* sm = lv ? lv->mat : m;
     const int K = pow2_ceil(k);
@@ -700,6 +758,14 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         const int per_cu = c.cu_waves > 0 ? c.cu_waves : 4;
         A.persist_grid = (long long)device_cus() * std::max(1, per_cu / std::max(1, c.wg / kWave));
     }
+    if (c.variant == 7) {
+        // natural order whatever the kernel: one workgroup of 16 waves per CU
+        kind = KK_XCD_SIMPLE;
+        A.dyn_lds = pv->lds_pad;
+        A.persist_grid = device_cus();
+        A.claim_rounds = 1;
+        c.wg = 1024;
+    }
     if (c.variant == 6) {
         const PackedShape ps = packed_shape(pw.n, info->nlevs);
         kind = ps.local ? KK_XCD_MULTIROW : KK_PERSIST_MULTIROW;
@@ -709,6 +775,7 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         A.dyn_lds = pv->lds_pad;
         A.persist_grid = (long long)device_cus() * (ps.cu_waves / (ps.wg / kWave));
         A.claim_rounds = 1;
+        A.groups = 1;
         c.wg = ps.wg;
         c.lanes = 32;  // the layout's widest rows
     }
@@ -1257,6 +1324,8 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
         shapes.push_back({has_waves(info) ? SPTRSV_KERNEL_MULTIROW : SPTRSV_KERNEL_ORDER, ref, 256, 1, 6, 0});
     // blocks of 64 rows in natural order
     if (K == 1 && block_walk_fits(mat)) shapes.push_back({SPTRSV_KERNEL_SIMPLE, ref, 256, 1, 5, 0});
+    if (K == 1 && group_walk_lanes(mat))
+        shapes.push_back({SPTRSV_KERNEL_SIMPLE, group_walk_lanes(mat), 256, 1, 7, 0});
 
     hipEvent_t e0, e1;
     SPT_HIP(hipEventCreate(&e0));

@@ -82,10 +82,10 @@ struct LevelPlan {
     void *structure = nullptr, *shared = nullptr, *kind[3] = {};
 };
 
-constexpr int kCounterWords = 8;
+constexpr int kCounterWords = 16;
 
 struct MatPriv {
-    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4], [5] row shape, [6] XCD of a packed walk, others spare (device)
+    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4] to [7] row shape, [8] XCD of a packed walk, others spare (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
     size_t pub_words = 0;
     uint64_t* part = nullptr;    // published partial sums of long-row segments, 2 per segment (device)
@@ -114,6 +114,7 @@ struct MatPriv {
     int max_row = 0;             // longest row (entries incl. diagonal)
     bool banded = false;         // no column more than 63 rows back
     int band_levels = 0;         // banded: number of levels (0: not known)
+    double nearest = 0.0;        // mean distance of a row's last off-diagonal
     bool near_rows = false;      // at least half of the rows depend on one of the kNear rows before them
     long long* trace = nullptr;  // per-row timeline (profiling), 3*n*k
     size_t trace_len = 0;
@@ -221,12 +222,14 @@ struct RowShape {
     bool wide = false;      // a column 64 or more rows back
     int levels = 0;         // while !wide; 0: not counted
     long long near = 0;     // rows whose last off-diagonal is at most kNear rows back
-    // of the `seen` rows that near was counted over
+    long long dist = 0;     // sum of the rows' distances to their last off-diagonal
+    // of the `seen` rows that near and dist were counted over
     void install(MatPriv* pv, long long rows, long long seen) const {
         pv->max_row = longest;
         pv->banded = !wide && rows > 0;
         pv->band_levels = wide ? 0 : levels;
         pv->near_rows = seen > 0 && 2 * near >= seen;
+        pv->nearest = seen > 0 ? (double)dist / (double)seen : 0.0;
     }
 };
 // The same of a matrix made on the device (its longest row given; waits).
@@ -235,6 +238,8 @@ int install_row_shape(sp_mat_t* m, int longest);
 // it takes its rows in order (banded kernel).
 bool block_walk_fits(const sp_mat_t* m);
 bool block_walk_in_order(const sp_mat_t* m);
+// Lanes per row of the group walk where that is the natural-order default, else 0.
+int group_walk_lanes(const sp_mat_t* m);
 void free_info_arrays(dfr_analysis_info_t* info);
 // The analysis of `copy`, the level-ordered copy made for analysis `src`,
 // derived from `src` (levels permuted, iorder the identity, the rest shared).

@@ -145,25 +145,36 @@ void free_mat(sp_mat_t* m) {
 }
 
 // out[0]: a column 64 or more rows back; out[1]: rows whose last off-diagonal
-// is nearer.  A thread leaves a row at its first far column, so long rows of
+// is at most kNear rows back; dist: the sum of those distances.  A thread leaves a row at its first far column, so long rows of
 // wide matrices cost one load.
 __global__ __launch_bounds__(256) void k_row_shape(const int* __restrict__ ia, const int* __restrict__ ja, int n,
-                                                   int* __restrict__ out) {
+                                                   int* __restrict__ out, unsigned long long* __restrict__ dist) {
     __shared__ int s_near, s_wide;
-    if (threadIdx.x == 0) s_near = s_wide = 0;
+    __shared__ unsigned long long s_dist;
+    if (threadIdx.x == 0) {
+        s_near = s_wide = 0;
+        s_dist = 0;
+    }
     __syncthreads();
     int near = 0, wide = 0;
+    unsigned long long far = 0;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         const int lo = ia[i], hi = ia[i + 1] - 1;
-        if (lo < hi) near += (int)i - ja[hi - 1] <= kNear;
+        if (lo < hi) {
+            const int d = (int)i - ja[hi - 1];
+            near += d <= kNear;
+            far += d;
+        }
         for (int p = lo; p < hi && !wide; ++p) wide = (int)i - ja[p] >= kWave;
     }
     if (near) atomicAdd(&s_near, near);
+    if (far) atomicAdd(&s_dist, far);
     if (wide) s_wide = 1;
     __syncthreads();
     if (threadIdx.x == 0) {
         if (s_wide) out[0] = 1;
         if (s_near) atomicAdd(&out[1], s_near);
+        if (s_dist) atomicAdd(dist, s_dist);
     }
 }
 
@@ -172,13 +183,14 @@ int install_row_shape(sp_mat_t* m, int longest) {
     shape.longest = longest;
     const int n = m->nr;
     if (n > 0) {
-        int h[2] = {0, 0}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
+        int h[4] = {}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
         hipLaunchKernelGGL(k_row_shape, dim3(std::min<unsigned>(ceil_div(n, 256), 512)), dim3(256), 0, nullptr, m->ia,
-                           m->ja, n, d);
+                           m->ja, n, d, reinterpret_cast<unsigned long long*>(d + 2));
         SPT_HIP(hipGetLastError());
         SPT_HIP(hipMemcpy(h, d, sizeof(h), hipMemcpyDeviceToHost));
         shape.wide = h[0] != 0;
         shape.near = h[1];
+        memcpy(&shape.dist, h + 2, sizeof(shape.dist));
     }
     shape.install(priv_of(m), n, n);
     return SPTRSV_OK;
@@ -212,7 +224,10 @@ static int validate_host_csr(const int* ia, const int* ja, int n, RowShape* shap
         }
         lev[i % kWave] = level;
         shape->levels = std::max(shape->levels, level);
-        shape->near += e - s > 1 && i - ja[e - 2] <= kNear;
+        if (e - s > 1) {
+            shape->near += i - ja[e - 2] <= kNear;
+            shape->dist += i - ja[e - 2];
+        }
         shape->longest = std::max<int>(shape->longest, (int)(e - s));
     }
     return SPTRSV_OK;

@@ -36,15 +36,17 @@ unsigned row_grid(long long count) {
 // row (i, or n-1-i for an upper triangle); dpos[i] = the diagonal entry used
 // (-1 for a unit diagonal); out[0] bit 1 = column outside [0, n), bit 2 = a
 // missing diagonal; out[1] = a kept column 64 or more rows away; out[2] of the
-// out[3] rows of every eighth workgroup have their last kept one within kNear.
+// out[3] rows of every eighth workgroup have their last kept one within kNear,
+// and out[4..5] is the sum of their distances to it.
 __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, const int* __restrict__ ja, int n,
                                                    int upper, int unit, int* __restrict__ len, int* __restrict__ dpos,
                                                    int* __restrict__ out) {
     int wide = 0, near = 0, rows = 0;
+    unsigned long long dist = 0;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
          t += (long long)gridDim.x * blockDim.x) {
         const int i = (int)t;
-        int kept = 0, d = -1, flags = 0, last = kWave;
+        int kept = 0, d = -1, flags = 0, last = 0;
         for (int p = ia[i]; p < ia[i + 1]; ++p) {
             const int j = ja[p];
             if (j < 0 || j >= n) flags |= 1;
@@ -59,20 +61,27 @@ __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, c
         if (flags) atomicOr(out, flags);
         len[upper ? n - 1 - i : i] = kept + 1;
         dpos[i] = unit ? -1 : d;
-        near += last <= kNear;
+        near += kept > 0 && last <= kNear;
+        dist += last;
         ++rows;
     }
     if (wide) out[1] = 1;
     if ((blockIdx.x & 7) == 0) {
         __shared__ int s_near, s_rows;
-        if (threadIdx.x == 0) s_near = s_rows = 0;
+        __shared__ unsigned long long s_dist;
+        if (threadIdx.x == 0) {
+            s_near = s_rows = 0;
+            s_dist = 0;
+        }
         __syncthreads();
         if (near) atomicAdd(&s_near, near);
         atomicAdd(&s_rows, rows);
+        atomicAdd(&s_dist, dist);
         __syncthreads();
         if (threadIdx.x == 0) {
             atomicAdd(&out[2], s_near);
             atomicAdd(&out[3], s_rows);
+            atomicAdd(reinterpret_cast<unsigned long long*>(out + 4), s_dist);
         }
     }
 }
@@ -122,17 +131,17 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     int *len = nullptr, *dpos = nullptr, *bad = nullptr;
     chk(hipMalloc(&len, 4 * ((size_t)n + 1)), "hipMalloc lengths");
     chk(hipMalloc(&dpos, 4 * (size_t)std::max(n, 1)), "hipMalloc diagonal positions");
-    chk(hipMalloc(&bad, 16), "hipMalloc flag");
+    chk(hipMalloc(&bad, 24), "hipMalloc flag");
     chk(hipMalloc(&m->ia, 4 * ((size_t)n + 1)), "hipMalloc ia");
     if (st == SPTRSV_OK) chk(hipMemset(len, 0, 4 * ((size_t)n + 1)), "clear lengths");
-    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 16), "clear flag");
+    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 24), "clear flag");
     if (st == SPTRSV_OK && n > 0) {
         hipLaunchKernelGGL(k_tri_count, dim3(row_grid(n)), dim3(256), 0, nullptr, ia, ja, n, upper ? 1 : 0,
                            unit ? 1 : 0, len, dpos, bad);
         chk(hipGetLastError(), "triangle count");
     }
-    int h_out[4] = {};
-    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 16, hipMemcpyDeviceToHost), "read flag");
+    int h_out[6] = {};
+    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 24, hipMemcpyDeviceToHost), "read flag");
     const int h_bad = h_out[0];
     if (st == SPTRSV_OK && (h_bad & 1)) st = fail(SPTRSV_E_INVALID_CSR, "column index outside [0, n)");
     if (st == SPTRSV_OK && (h_bad & 2)) st = fail(SPTRSV_E_INVALID_CSR, "a row has no diagonal entry (non-unit diagonal)");
@@ -156,6 +165,7 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
         for (int r = 0; r < n; ++r) shape.longest = std::max(shape.longest, ia_h[r + 1] - ia_h[r]);
         shape.wide = h_out[1] != 0;
         shape.near = h_out[2];
+        memcpy(&shape.dist, h_out + 4, sizeof(shape.dist));
         shape.install(priv_of(m), n, h_out[3]);
         chk(hipDeviceSynchronize(), "triangle sync");
     }

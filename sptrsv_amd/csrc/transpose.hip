@@ -129,6 +129,7 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
         dp->banded = from->banded;
         dp->band_levels = from->band_levels;
         dp->near_rows = from->near_rows;
+        dp->nearest = from->nearest;
     }
     // the sorted payload is the value map of the new handle
     MatPriv* sp = priv_of(src);
