@@ -190,27 +190,38 @@ __global__ void k_scan_apply(const int* in, int* out, long long n, const int* of
     }
 }
 
+size_t scan_scratch(long long n) {
+    size_t total = 0;
+    for (long long b = (n + kScanTile - 1) / kScanTile; b > 1; b = (b + kScanTile - 1) / kScanTile) total += (size_t)b;
+    return total;
+}
+
 // out[i] = sum_{j<i} in[j]; in and out may alias.
-int exclusive_scan(const int* in, int* out, long long n, hipStream_t s) {
+int exclusive_scan(const int* in, int* out, long long n, hipStream_t s, int* scratch) {
     if (n <= 0) return SPTRSV_OK;
-    long long blocks = (n + kScanTile - 1) / kScanTile;
+    const long long blocks = (n + kScanTile - 1) / kScanTile;
     if (blocks == 1) {
         hipLaunchKernelGGL(k_scan_apply, dim3(1), dim3(kScanThreads), 0, s, in, out, n, nullptr);
         SPT_HIP(hipGetLastError());
         return SPTRSV_OK;
     }
-    int* sums = nullptr;
-    SPT_HIP(hipMalloc(&sums, blocks * sizeof(int)));
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)blocks), dim3(kScanThreads), 0, s, in, n, sums);
-    int st = hipGetLastError() == hipSuccess ? exclusive_scan(sums, sums, blocks, s)
+    int* own = nullptr;
+    if (!scratch) {
+        SPT_HIP(hipMalloc(&own, scan_scratch(n) * sizeof(int)));
+        scratch = own;
+    }
+    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)blocks), dim3(kScanThreads), 0, s, in, n, scratch);
+    int st = hipGetLastError() == hipSuccess ? exclusive_scan(scratch, scratch, blocks, s, scratch + blocks)
                                              : fail(SPTRSV_E_HIP, "scan reduce launch");
     if (st == SPTRSV_OK) {
         hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)blocks), dim3(kScanThreads), 0, s, in, out, n,
-                           sums);
+                           scratch);
         if (hipGetLastError() != hipSuccess) st = fail(SPTRSV_E_HIP, "scan apply launch");
     }
-    if (hipStreamSynchronize(s) != hipSuccess && st == SPTRSV_OK) st = fail(SPTRSV_E_HIP, "scan sync");
-    (void)hipFree(sums);
+    if (own) {
+        if (hipStreamSynchronize(s) != hipSuccess && st == SPTRSV_OK) st = fail(SPTRSV_E_HIP, "scan sync");
+        (void)hipFree(own);
+    }
     return st;
 }
 
@@ -275,24 +286,48 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const int* __restrict
     }
 }
 
+size_t sort_scratch(int n) {
+    const long long hist = 256LL * ((n + kRsTile - 1) / kRsTile);
+    return (size_t)hist + scan_scratch(hist);
+}
+
+__global__ void k_longest(const int* __restrict__ ia, int n, int* __restrict__ out) {
+    __shared__ int s_max;
+    if (threadIdx.x == 0) s_max = 0;
+    __syncthreads();
+    int m = 0;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+        m = max(m, ia[i + 1] - ia[i]);
+    atomicMax(&s_max, m);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(out, s_max);
+}
+
+int longest_row(const int* ia, int n, int* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_longest, dim3(std::max<unsigned>(1, std::min<unsigned>(ceil_div(n, 1024), 512))), dim3(256), 0, s,
+                       ia, n, out);
+    return hipGetLastError() == hipSuccess ? SPTRSV_OK : fail(SPTRSV_E_HIP, "longest row");
+}
+
 // Sorts (keys, vals) by key, stably; max_key bounds the keys.  The result is
 // left in (keys, vals); tk/tv are scratch of the same length.
 int radix_sort_pairs(int* keys, int* vals, int* tk, int* tv, int n, int max_key,
-                            hipStream_t s) {
+                     hipStream_t s, int* scratch) {
     if (n <= 1) return SPTRSV_OK;
     int bits = 0;
     while (bits < 31 && (max_key >> bits) != 0) ++bits;
     int passes = std::max(1, (bits + 7) / 8);
     int ntiles = (n + kRsTile - 1) / kRsTile;
-    int* hist = nullptr;
-    SPT_HIP(hipMalloc(&hist, sizeof(int) * 256 * (size_t)ntiles));
+    int* own = nullptr;
+    if (!scratch) SPT_HIP(hipMalloc(&own, sizeof(int) * sort_scratch(n)));
+    int *hist = scratch ? scratch : own, *sums = hist + 256LL * ntiles;
     int st = SPTRSV_OK;
     int *ki = keys, *vi = vals, *ko = tk, *vo = tv;
     for (int p = 0; p < passes && st == SPTRSV_OK; ++p) {
         int shift = 8 * p;
         hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kRsThreads), 0, s, ki, n, shift, hist, ntiles);
         if (hipGetLastError() != hipSuccess) { st = fail(SPTRSV_E_HIP, "radix hist"); break; }
-        st = exclusive_scan(hist, hist, 256LL * ntiles, s);
+        st = exclusive_scan(hist, hist, 256LL * ntiles, s, sums);
         if (st != SPTRSV_OK) break;
         hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kRsThreads), 0, s, ki, vi, ko, vo, n, shift,
                            hist, ntiles);
@@ -305,8 +340,10 @@ int radix_sort_pairs(int* keys, int* vals, int* tk, int* tv, int n, int max_key,
             hipMemcpyAsync(vals, vi, sizeof(int) * (size_t)n, hipMemcpyDeviceToDevice, s) != hipSuccess)
             st = fail(SPTRSV_E_HIP, "radix copy back");
     }
-    if (hipStreamSynchronize(s) != hipSuccess && st == SPTRSV_OK) st = fail(SPTRSV_E_HIP, "radix sort sync");
-    (void)hipFree(hist);
+    if (own) {
+        if (hipStreamSynchronize(s) != hipSuccess && st == SPTRSV_OK) st = fail(SPTRSV_E_HIP, "radix sort sync");
+        (void)hipFree(own);
+    }
     return st;
 }
 
@@ -371,6 +408,9 @@ struct InfoPriv {
     // wave64 layout of an ORDER analysis, for the packed walk (derived data;
     // MULTIROW and ALL analyses have it in info)
     int *wbase = nullptr, *wsize = nullptr, n_waves = 0;
+    // the arrays of info sized by the matrix, where they were made together
+    void* block = nullptr;
+    size_t block_bytes = 0;
     unsigned long long id = 0;  // unique per analysis built, loaded or copied
 };
 static std::mutex g_info_mu;
@@ -426,8 +466,12 @@ void free_info_arrays(dfr_analysis_info_t* info) {
     int* arrays[] = {ip->wbase, ip->wsize, info->lev_size, info->warp_lev, info->inv_iorder, info->iorder,
                      info->ibase_row, info->ivect_size_warp, info->row_ctr, info->level,
                      info->bucket_off, info->ibase_row64, info->ivect_size_wave};
-    for (int* p : arrays)
-        if (p) (void)hipFree(p);
+    const char* lo = static_cast<const char*>(ip->block);
+    for (int* p : arrays) {
+        const char* q = reinterpret_cast<const char*>(p);
+        if (p && !(lo && q >= lo && q < lo + ip->block_bytes)) (void)hipFree(p);
+    }
+    if (ip->block) (void)hipFree(ip->block);
     delete ip;
     MODE mode = info->mode;
     *info = dfr_analysis_info_t{};
@@ -435,14 +479,13 @@ void free_info_arrays(dfr_analysis_info_t* info) {
 }
 
 // Warp arrays for one lane width.
+// wpb: nb + 1 ints, then scan_scratch(nb + 1); on return the waves before each bucket.
 static int build_warps(const int* bucket_cnt, const int* bucket_off, int nb, int lanes, int n,
-                       int** base, int** vsize, int* count, int** warp_off_out, hipStream_t s) {
-    int* wpb = nullptr;
-    SPT_HIP(hipMalloc(&wpb, sizeof(int) * (size_t)(nb + 1)));
+                       int** base, int** vsize, int* count, int* wpb, hipStream_t s) {
     hipLaunchKernelGGL(k_warps_per_bucket, dim3(grid_for(nb + 1)), dim3(256), 0, s, bucket_cnt, nb,
                        lanes, wpb);
     SPT_HIP(hipGetLastError());
-    SPT_TRY(exclusive_scan(wpb, wpb, nb + 1, s));
+    SPT_TRY(exclusive_scan(wpb, wpb, nb + 1, s, wpb + nb + 1));
     int total = 0;
     SPT_HIP(hipMemcpyAsync(&total, wpb + nb, sizeof(int), hipMemcpyDeviceToHost, s));
     SPT_HIP(hipStreamSynchronize(s));
@@ -452,10 +495,6 @@ static int build_warps(const int* bucket_cnt, const int* bucket_off, int nb, int
                        bucket_off, nb, lanes, *base, *vsize, n);
     SPT_HIP(hipGetLastError());
     *count = total;
-    if (warp_off_out)
-        *warp_off_out = wpb;
-    else
-        SPT_HIP(hipFree(wpb));
     return SPTRSV_OK;
 }
 
@@ -591,14 +630,18 @@ static int build_derived(dfr_analysis_info_t* info, sp_mat_t* m) {
     if (info->mode == ORDER && info->n > 0 && owns_info(info)) {
         InfoPriv* ip = static_cast<InfoPriv*>(info->priv);
         const int nb = 7 * info->nlevs;
-        int* cnt = nullptr;
-        SPT_HIP(hipMalloc(&cnt, sizeof(int) * (size_t)(nb + 1)));
+        int *cnt = nullptr, *wpb = nullptr;
+        void* tmp = nullptr;
+        Arena ar;
+        ar.add(&cnt, nb + 1);
+        ar.add(&wpb, nb + 1 + scan_scratch(nb + 1));
+        SPT_HIP(ar.get(&tmp));
         hipLaunchKernelGGL(k_bucket_counts, dim3(grid_for(nb)), dim3(256), 0, nullptr, info->bucket_off, nb, cnt);
         int st = hipGetLastError() == hipSuccess ? SPTRSV_OK : fail(SPTRSV_E_HIP, "bucket counts");
         if (st == SPTRSV_OK)
-            st = build_warps(cnt, info->bucket_off, nb, 64, info->n, &ip->wbase, &ip->wsize, &ip->n_waves, nullptr, nullptr);
+            st = build_warps(cnt, info->bucket_off, nb, 64, info->n, &ip->wbase, &ip->wsize, &ip->n_waves, wpb, nullptr);
         if (st == SPTRSV_OK && hipStreamSynchronize(nullptr) != hipSuccess) st = fail(SPTRSV_E_HIP, "wave layout");
-        (void)hipFree(cnt);
+        (void)hipFree(tmp);
         if (st != SPTRSV_OK) return st;
     }
     return build_segments(info, m);
@@ -613,12 +656,26 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     info->priv = new_info_priv();
     info->mode = mode;
     info->n = n;
-    SPT_HIP(hipMalloc(&info->row_ctr, sizeof(int)));
+    InfoPriv* ip = static_cast<InfoPriv*>(info->priv);
+    {
+        Arena ar;
+        ar.add(&info->row_ctr, 1);
+        if (n > 0) {
+            ar.add(&info->level, n);
+            ar.add(&info->iorder, n);
+            ar.add(&info->inv_iorder, n);
+        }
+        const hipError_t e = ar.get(&ip->block);
+        if (e != hipSuccess) {
+            info->row_ctr = info->level = info->iorder = info->inv_iorder = nullptr;
+            return hip_fail(e, "hipMalloc analysis", __FILE__, __LINE__);
+        }
+        ip->block_bytes = ar.total;
+    }
     SPT_HIP(hipMemset(info->row_ctr, 0, sizeof(int)));
     if (n == 0) return SPTRSV_OK;
 
     // 1. levels: sync-free max-plus pass (0 = unsolved).
-    SPT_HIP(hipMalloc(&info->level, sizeof(int) * (size_t)n));
     int lanes = 2, wg = 256;
     solve_config_for_analysis(m, &lanes, &wg);
     // Levels are integers, so every correct pass gives the same array; the
@@ -677,8 +734,7 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         if (e != hipSuccess) return hip_fail(e, "level pass", __FILE__, __LINE__);
     }
     // 2. nlevs
-    int* d_max = nullptr;
-    SPT_HIP(hipMalloc(&d_max, sizeof(int) * 2));
+    int* d_max = pv->counters + 10;
     SPT_HIP(hipMemsetAsync(d_max, 0, sizeof(int) * 2, s));
     hipLaunchKernelGGL(k_max, dim3(std::min<unsigned>(grid_for(n), 1024)), dim3(256), 0, s,
                        info->level, n, d_max);
@@ -687,7 +743,6 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     SPT_HIP(hipMemcpyAsync(h_max, d_max, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
     SPT_HIP(hipMemcpyAsync(&h_max[1], pv->counters + 1, sizeof(int), hipMemcpyDeviceToHost, s));
     SPT_HIP(hipStreamSynchronize(s));
-    (void)hipFree(d_max);
     if (h_max[1]) {
         int zero = 0;
         (void)hipMemcpy(pv->counters + 1, &zero, sizeof(int), hipMemcpyHostToDevice);
@@ -702,12 +757,23 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     const int nb = 7 * nlevs;
 
     // 3. keys and histograms
-    int *key = nullptr, *tk = nullptr, *tv = nullptr, *bucket_cnt = nullptr;
-    SPT_HIP(hipMalloc(&key, sizeof(int) * (size_t)n));
-    SPT_HIP(hipMalloc(&tk, sizeof(int) * (size_t)n));
-    SPT_HIP(hipMalloc(&tv, sizeof(int) * (size_t)n));
-    SPT_HIP(hipMalloc(&info->iorder, sizeof(int) * (size_t)n));
-    SPT_HIP(hipMalloc(&bucket_cnt, sizeof(int) * (size_t)(nb + 1)));
+    int *key = nullptr, *tk = nullptr, *tv = nullptr, *bucket_cnt = nullptr, *scratch = nullptr, *wpb = nullptr;
+    struct Temp {
+        void* p = nullptr;
+        ~Temp() {
+            if (p) (void)hipFree(p);
+        }
+    } tmp;
+    {
+        Arena ar;
+        ar.add(&key, n);
+        ar.add(&tk, n);
+        ar.add(&tv, n);
+        ar.add(&bucket_cnt, nb + 1);
+        ar.add(&scratch, std::max(sort_scratch(n), scan_scratch(nb + 1)));
+        ar.add(&wpb, nb + 1 + scan_scratch(nb + 1));
+        SPT_HIP(ar.get(&tmp.p));
+    }
     SPT_HIP(hipMalloc(&info->bucket_off, sizeof(int) * (size_t)(nb + 1)));
     SPT_HIP(hipMalloc(&info->lev_size, sizeof(int) * (size_t)nlevs));
     hipLaunchKernelGGL(k_fill_int, dim3(grid_for(nb + 1)), dim3(256), 0, s, bucket_cnt, (size_t)(nb + 1), 0);
@@ -727,7 +793,6 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         SPT_HIP(hipMemcpyAsync(&bad, pv->counters + 2, sizeof(int), hipMemcpyDeviceToHost, s));
         SPT_HIP(hipStreamSynchronize(s));
         if (bad) {
-            (void)hipFree(key); (void)hipFree(tk); (void)hipFree(tv); (void)hipFree(bucket_cnt);
             int zero = 0;
             (void)hipMemcpy(pv->counters + 2, &zero, sizeof(int), hipMemcpyHostToDevice);
             return fail(SPTRSV_E_HIP, "level pass left a row without a valid level");
@@ -735,39 +800,23 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     }
 
     // 4. iorder = stable sort of rows by key
-    int st = radix_sort_pairs(key, info->iorder, tk, tv, n, nb - 1, s);
-    (void)hipFree(tk);
-    (void)hipFree(tv);
-    (void)hipFree(key);
-    if (st != SPTRSV_OK) { (void)hipFree(bucket_cnt); return st; }
+    SPT_TRY(radix_sort_pairs(key, info->iorder, tk, tv, n, nb - 1, s, scratch));
 
     // 5. bucket offsets
-    SPT_TRY(exclusive_scan(bucket_cnt, info->bucket_off, nb + 1, s));
-    SPT_HIP(hipMalloc(&info->inv_iorder, sizeof(int) * (size_t)n));
+    SPT_TRY(exclusive_scan(bucket_cnt, info->bucket_off, nb + 1, s, scratch));
     hipLaunchKernelGGL(k_inverse, dim3(grid_for(n)), dim3(256), 0, s, info->iorder, n, info->inv_iorder);
     SPT_HIP(hipGetLastError());
 
     // 6. warp arrays (MULTIROW / ALL), 32-lane reference layout and 64-lane layout
     if (mode == MULTIROW || mode == ALL) {
-        int* warp_off = nullptr;
-        st = build_warps(bucket_cnt, info->bucket_off, nb, 32, n, &info->ibase_row,
-                         &info->ivect_size_warp, &info->n_warps, &warp_off, s);
-        if (st == SPTRSV_OK) {
-            st = build_warps(bucket_cnt, info->bucket_off, nb, 64, n, &info->ibase_row64,
-                             &info->ivect_size_wave, &info->n_waves, nullptr, s);
-        }
-        if (st == SPTRSV_OK) {
-            if (hipMalloc(&info->warp_lev, sizeof(int) * (size_t)(nlevs + 1)) != hipSuccess) {
-                st = fail(SPTRSV_E_ALLOC, "warp_lev");
-            } else {
-                hipLaunchKernelGGL(k_warp_lev, dim3(grid_for(nlevs + 1)), dim3(256), 0, s, warp_off,
-                                   nlevs, info->warp_lev);
-            }
-        }
-        if (warp_off) (void)hipFree(warp_off);
+        SPT_TRY(build_warps(bucket_cnt, info->bucket_off, nb, 64, n, &info->ibase_row64,
+                            &info->ivect_size_wave, &info->n_waves, wpb, s));
+        SPT_TRY(build_warps(bucket_cnt, info->bucket_off, nb, 32, n, &info->ibase_row,
+                            &info->ivect_size_warp, &info->n_warps, wpb, s));
+        SPT_HIP(hipMalloc(&info->warp_lev, sizeof(int) * (size_t)(nlevs + 1)));
+        hipLaunchKernelGGL(k_warp_lev, dim3(grid_for(nlevs + 1)), dim3(256), 0, s, wpb, nlevs, info->warp_lev);
+        SPT_HIP(hipGetLastError());
     }
-    (void)hipFree(bucket_cnt);
-    if (st != SPTRSV_OK) return st;
     SPT_HIP(hipStreamSynchronize(s));
     return build_derived(info, m);
 }

@@ -4,9 +4,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <array>
 #include <map>
 #include <string>
+#include <vector>
 
 #include "sptrsv_amd.h"
 
@@ -36,6 +38,34 @@ constexpr int kWave = 64;
 // "row not solved yet".  Levels use 0 (levels are >= 1).
 constexpr uint64_t kUnsolved64 = ~0ull;
 constexpr uint32_t kUnsolved32 = ~0u;
+
+// ---- device memory -----------------------------------------------------------
+// Carves arrays out of one allocation (an allocation costs tens of
+// microseconds, its release more, and both wait): add() every array, then get().
+struct Arena {
+    struct Part {
+        void** p;
+        size_t bytes;
+    };
+    std::vector<Part> parts;
+    size_t total = 0;
+    template <class T>
+    void add(T** p, size_t count) {
+        const size_t bytes = (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+        parts.push_back({reinterpret_cast<void**>(p), bytes});
+        total += bytes;
+    }
+    hipError_t get(void** block) {
+        const hipError_t e = hipMalloc(block, total);
+        if (e != hipSuccess) return e;
+        char* at = static_cast<char*>(*block);
+        for (const Part& q : parts) {
+            *q.p = at;
+            at += q.bytes;
+        }
+        return e;
+    }
+};
 
 // ---- library-private state hung off sp_mat_t::priv ------------------------
 struct Workspace;  // defined in solve.hip
@@ -85,6 +115,7 @@ struct LevelPlan {
 constexpr int kCounterWords = 16;
 
 struct MatPriv {
+    void* block = nullptr;       // holds ia, ja, a, a32 and src_perm of a handle made on the device
     int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4] to [7] row shape, [8] XCD of a packed walk, others spare (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
     size_t pub_words = 0;
@@ -246,7 +277,10 @@ void free_info_arrays(dfr_analysis_info_t* info);
 int level_copy_analysis(const dfr_analysis_info_t* src, sp_mat_t* copy, dfr_analysis_info_t* dst);
 
 // out[i] = sum_{j<i} in[j] on the device (in and out may alias)
-int exclusive_scan(const int* in, int* out, long long n, hipStream_t s);
+// With scratch (scan_scratch(n) ints) it only launches; else it allocates and
+// waits.
+int exclusive_scan(const int* in, int* out, long long n, hipStream_t s, int* scratch = nullptr);
+size_t scan_scratch(long long n);
 // Kernel timer (api_solve.hip): the next (start, stop) event pair while
 // timing is enabled and the stream is not being captured, else an empty
 // pair (false); the caller records it around `launches` consecutive
@@ -260,7 +294,11 @@ constexpr int kTimeSyncFree = 1;   // sync-free solve passes (kernel timer kinds
 constexpr int kTimeSweeps = 2;     // a refinement step's Jacobi sweeps
 KtPair kernel_timer_pair(hipStream_t s, int launches = 1, int kind = kTimeSyncFree);
 // stable LSD radix sort of (keys, vals) by key in [0, max_key]; tk/tv scratch
-int radix_sort_pairs(int* keys, int* vals, int* tk, int* tv, int n, int max_key, hipStream_t s);
+// (with sort_scratch(n) ints of scratch it only launches).
+int radix_sort_pairs(int* keys, int* vals, int* tk, int* tv, int n, int max_key, hipStream_t s, int* scratch = nullptr);
+size_t sort_scratch(int n);
+// Longest row of a device row-pointer array into *out (device, zero before).
+int longest_row(const int* ia, int n, int* out, hipStream_t s);
 
 // ---- launch helpers ----------------------------------------------------------
 inline unsigned ceil_div(long long a, long long b) { return (unsigned)((a + b - 1) / b); }

@@ -101,11 +101,16 @@ int ensure_priv(sp_mat_t* m) {
 
 void free_mat(sp_mat_t* m) {
     if (!m) return;
-    if (m->ia) (void)hipFree(m->ia);
-    if (m->ja) (void)hipFree(m->ja);
-    if (m->a) (void)hipFree(m->a);
-    if (m->a32) (void)hipFree(m->a32);
     MatPriv* pv = priv_of(m);
+    if (pv && pv->block) {
+        (void)hipFree(pv->block);
+        pv->src_perm = nullptr;
+    } else {
+        if (m->ia) (void)hipFree(m->ia);
+        if (m->ja) (void)hipFree(m->ja);
+        if (m->a) (void)hipFree(m->a);
+        if (m->a32) (void)hipFree(m->a32);
+    }
     if (pv) {
         {
             // first, so that no freed analysis looks at this matrix any more

@@ -552,33 +552,6 @@ static void free_level_plan(LevelPlan& L) {
     L = LevelPlan{};
 }
 
-// Carves arrays out of one allocation (an allocation costs several
-// microseconds, more than a small solve): add() every array, then get().
-struct LwArena {
-    struct Part {
-        void** p;
-        size_t bytes;
-    };
-    std::vector<Part> parts;
-    size_t total = 0;
-    template <class T>
-    void add(T** p, size_t count) {
-        const size_t bytes = (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
-        parts.push_back({reinterpret_cast<void**>(p), bytes});
-        total += bytes;
-    }
-    hipError_t get(void** block) {
-        const hipError_t e = hipMalloc(block, total);
-        if (e != hipSuccess) return e;
-        char* at = static_cast<char*>(*block);
-        for (const Part& q : parts) {
-            *q.p = at;
-            at += q.bytes;
-        }
-        return e;
-    }
-};
-
 // A matrix's plans are looked up and released under this lock: a thread that
 // frees an analysis releases its plans in every live matrix.
 static std::mutex g_lw_mu;
@@ -694,7 +667,7 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
         const int over_cap = 64 + L.n_slices / 4;
         int2* slice = nullptr;
         unsigned* step = nullptr;
-        LwArena ar;
+        Arena ar;
         ar.add(&slice, L.n_slices);
         ar.add(&step, L.n_steps_all);
         ar.add(&L.col, slots * kLwU);
@@ -735,9 +708,9 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
 static hipError_t lw_alloc_kind(LevelPlan& L, int kind, int n) {
     const size_t slots = (size_t)L.n_slices * kWave, rb = kind == 1 ? 8 : 12;
     const int k = kind == 1 ? 1 : 0;  // mixed shares FP64's slot records
-    LwArena ar;
+    Arena ar;
     if (kind != 1 && !L.shared) {
-        LwArena sh;
+        Arena sh;
         sh.add(reinterpret_cast<char**>(&L.rec[0]), slots * kLwU * rb);
         sh.add(reinterpret_cast<char**>(&L.frec[0]), L.far ? slots * rb : 0);
         sh.add(reinterpret_cast<char**>(&L.orec[0]), (size_t)L.n_over * kWave * rb);

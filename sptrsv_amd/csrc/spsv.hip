@@ -128,32 +128,44 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     auto chk = [&](hipError_t e, const char* what) {
         if (e != hipSuccess && st == SPTRSV_OK) st = hip_fail(e, what, __FILE__, __LINE__);
     };
-    int *len = nullptr, *dpos = nullptr, *bad = nullptr;
-    chk(hipMalloc(&len, 4 * ((size_t)n + 1)), "hipMalloc lengths");
-    chk(hipMalloc(&dpos, 4 * (size_t)std::max(n, 1)), "hipMalloc diagonal positions");
-    chk(hipMalloc(&bad, 24), "hipMalloc flag");
-    chk(hipMalloc(&m->ia, 4 * ((size_t)n + 1)), "hipMalloc ia");
+    int *len = nullptr, *dpos = nullptr, *bad = nullptr, *ia_s = nullptr, *scratch = nullptr;
+    Arena work;
+    work.add(&len, (size_t)n + 1);
+    work.add(&dpos, n);
+    work.add(&bad, 8);
+    work.add(&ia_s, (size_t)n + 1);
+    work.add(&scratch, scan_scratch((long long)n + 1));
+    void* tmp = nullptr;
+    chk(work.get(&tmp), "hipMalloc triangle work");
     if (st == SPTRSV_OK) chk(hipMemset(len, 0, 4 * ((size_t)n + 1)), "clear lengths");
-    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 24), "clear flag");
+    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 32), "clear flag");
     if (st == SPTRSV_OK && n > 0) {
         hipLaunchKernelGGL(k_tri_count, dim3(row_grid(n)), dim3(256), 0, nullptr, ia, ja, n, upper ? 1 : 0,
                            unit ? 1 : 0, len, dpos, bad);
         chk(hipGetLastError(), "triangle count");
     }
-    int h_out[6] = {};
-    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 24, hipMemcpyDeviceToHost), "read flag");
+    // row pointers, and the longest row, before what came out is looked at: one
+    // wait for all
+    if (st == SPTRSV_OK) st = exclusive_scan(len, ia_s, (long long)n + 1, nullptr, scratch);
+    if (st == SPTRSV_OK && n > 0) st = longest_row(ia_s, n, bad + 6, nullptr);
+    int h_out[8] = {};
+    int total = 0;
+    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 32, hipMemcpyDeviceToHost), "read flag");
     const int h_bad = h_out[0];
     if (st == SPTRSV_OK && (h_bad & 1)) st = fail(SPTRSV_E_INVALID_CSR, "column index outside [0, n)");
     if (st == SPTRSV_OK && (h_bad & 2)) st = fail(SPTRSV_E_INVALID_CSR, "a row has no diagonal entry (non-unit diagonal)");
-    if (st == SPTRSV_OK) st = exclusive_scan(len, m->ia, (long long)n + 1, nullptr);
-    std::vector<int> ia_h((size_t)n + 1, 0);
-    if (st == SPTRSV_OK) chk(hipMemcpy(ia_h.data(), m->ia, 4 * ia_h.size(), hipMemcpyDeviceToHost), "read ia");
-    const int total = ia_h[n];
+    if (st == SPTRSV_OK) chk(hipMemcpy(&total, ia_s + n, 4, hipMemcpyDeviceToHost), "read ia");
     m->nnz = total;
-    if (st == SPTRSV_OK) chk(hipMalloc(&m->ja, 4 * (size_t)std::max(total, 1)), "hipMalloc ja");
-    if (st == SPTRSV_OK) chk(hipMalloc(&m->a, 8 * (size_t)std::max(total, 1)), "hipMalloc a");
-    if (st == SPTRSV_OK) chk(hipMalloc(&m->a32, 4 * (size_t)std::max(total, 1)), "hipMalloc a32");
-    if (st == SPTRSV_OK) chk(hipMalloc(&priv_of(m)->src_perm, 4 * (size_t)std::max(total, 1)), "hipMalloc value map");
+    const size_t ne = (size_t)std::max(total, 1);
+    Arena keep;
+    keep.add(&m->ia, (size_t)n + 1);
+    keep.add(&m->ja, ne);
+    keep.add(&m->a, ne);
+    keep.add(&m->a32, ne);
+    keep.add(&priv_of(m)->src_perm, ne);
+    if (st == SPTRSV_OK) chk(keep.get(&priv_of(m)->block), "hipMalloc triangle");
+    if (st == SPTRSV_OK)
+        chk(hipMemcpyAsync(m->ia, ia_s, 4 * ((size_t)n + 1), hipMemcpyDeviceToDevice, nullptr), "copy ia");
     priv_of(m)->src_count = nnz;
     if (st == SPTRSV_OK && n > 0) {
         hipLaunchKernelGGL(k_tri_fill, dim3(row_grid(n)), dim3(256), 0, nullptr, ia, ja, a, n, upper ? 1 : 0, dpos,
@@ -162,16 +174,15 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     }
     if (st == SPTRSV_OK) {
         RowShape shape;
-        for (int r = 0; r < n; ++r) shape.longest = std::max(shape.longest, ia_h[r + 1] - ia_h[r]);
+        shape.longest = h_out[6];
         shape.wide = h_out[1] != 0;
         shape.near = h_out[2];
         memcpy(&shape.dist, h_out + 4, sizeof(shape.dist));
         shape.install(priv_of(m), n, h_out[3]);
-        chk(hipDeviceSynchronize(), "triangle sync");
     }
     if (st == SPTRSV_OK) st = convert_values_to_f32(m);
-    for (int* p : {len, dpos, bad})
-        if (p) (void)hipFree(p);
+    if (st == SPTRSV_OK) chk(hipDeviceSynchronize(), "triangle sync");
+    if (tmp) (void)hipFree(tmp);
     if (st != SPTRSV_OK) free_mat(m);
     return st;
 }

@@ -90,22 +90,27 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
         if (e != hipSuccess && st == SPTRSV_OK) st = hip_fail(e, what, __FILE__, __LINE__);
     };
     const size_t ne = (size_t)std::max(nnz, 1);
-    chk(hipMalloc(&dst->ia, sizeof(int) * (size_t)(n + 1)), "hipMalloc ia");
-    chk(hipMalloc(&dst->ja, sizeof(int) * ne), "hipMalloc ja");
-    chk(hipMalloc(&dst->a32, sizeof(float) * ne), "hipMalloc a32");
-    if (f64) chk(hipMalloc(&dst->a, sizeof(double) * ne), "hipMalloc a");
-    int *keys = nullptr, *vals = nullptr, *tk = nullptr, *tv = nullptr;
-    chk(hipMalloc(&keys, sizeof(int) * ne), "hipMalloc keys");
-    chk(hipMalloc(&vals, sizeof(int) * ne), "hipMalloc vals");
-    chk(hipMalloc(&tk, sizeof(int) * ne), "hipMalloc sort keys");
-    chk(hipMalloc(&tv, sizeof(int) * ne), "hipMalloc sort vals");
+    int *keys = nullptr, *vals = nullptr, *tk = nullptr, *tv = nullptr, *scratch = nullptr;
+    Arena keep, work;
+    keep.add(&dst->ia, (size_t)n + 1);
+    keep.add(&dst->ja, ne);
+    keep.add(&dst->a32, ne);
+    if (f64) keep.add(&dst->a, ne);
+    keep.add(&vals, ne);  // in the end the value map of the new handle
+    chk(keep.get(&priv_of(dst)->block), "hipMalloc transpose");
+    work.add(&keys, ne);
+    work.add(&tk, ne);
+    work.add(&tv, ne);
+    work.add(&scratch, std::max(sort_scratch(nnz), scan_scratch((long long)n + 1)));
+    void* tmp = nullptr;
+    if (st == SPTRSV_OK) chk(work.get(&tmp), "hipMalloc transpose sort");
     if (st == SPTRSV_OK) chk(hipMemset(dst->ia, 0, sizeof(int) * (size_t)(n + 1)), "clear counts");
     if (st == SPTRSV_OK && n > 0) {
         hipLaunchKernelGGL(k_tr_keys, dim3(tr_grid(nnz)), dim3(256), 0, nullptr, src->ja, n, nnz, keys, vals,
                            dst->ia);
         chk(hipGetLastError(), "transpose keys");
-        if (st == SPTRSV_OK) st = radix_sort_pairs(keys, vals, tk, tv, nnz, n - 1, nullptr);
-        if (st == SPTRSV_OK) st = exclusive_scan(dst->ia, dst->ia, (long long)n + 1, nullptr);
+        if (st == SPTRSV_OK) st = radix_sort_pairs(keys, vals, tk, tv, nnz, n - 1, nullptr, scratch);
+        if (st == SPTRSV_OK) st = exclusive_scan(dst->ia, dst->ia, (long long)n + 1, nullptr, scratch);
         if (st == SPTRSV_OK) {
             if (f64)
                 hipLaunchKernelGGL(k_tr_fill<true>, dim3(tr_grid(nnz)), dim3(256), 0, nullptr, src->ia, n, nnz,
@@ -117,12 +122,12 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
         }
     }
     if (st == SPTRSV_OK && n > 0) {
-        std::vector<int> ia((size_t)n + 1);
-        chk(hipMemcpy(ia.data(), dst->ia, sizeof(int) * ia.size(), hipMemcpyDeviceToHost), "read row pointers");
-        int mr = 0;
-        for (int r = 0; r < n && st == SPTRSV_OK; ++r) mr = std::max(mr, ia[r + 1] - ia[r]);
-        if (st == SPTRSV_OK && ia[n] != nnz) st = fail(SPTRSV_E_INVALID_CSR, "transpose row pointers do not sum to nnz");
         MatPriv* dp = priv_of(dst);
+        int mr = 0, end = 0, *longest = dp->counters + 4;  // zero since the handle was made
+        st = longest_row(dst->ia, n, longest, nullptr);
+        if (st == SPTRSV_OK) chk(hipMemcpy(&mr, longest, sizeof(int), hipMemcpyDeviceToHost), "read longest row");
+        if (st == SPTRSV_OK) chk(hipMemcpy(&end, dst->ia + n, sizeof(int), hipMemcpyDeviceToHost), "read row pointers");
+        if (st == SPTRSV_OK && end != nnz) st = fail(SPTRSV_E_INVALID_CSR, "transpose row pointers do not sum to nnz");
         const MatPriv* from = priv_of(src);
         dp->max_row = mr;
         // distances and levels are those of the source; near rows as there
@@ -140,11 +145,9 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
     if (st == SPTRSV_OK) {
         priv_of(dst)->src_perm = vals;
         priv_of(dst)->src_count = sp->src_count;
-        vals = nullptr;
+        chk(hipDeviceSynchronize(), "transpose sync");
     }
-    for (int* p : {keys, vals, tk, tv})
-        if (p) (void)hipFree(p);
-    if (st == SPTRSV_OK) chk(hipDeviceSynchronize(), "transpose sync");
+    if (tmp) (void)hipFree(tmp);
     if (st != SPTRSV_OK) free_mat(dst);
     return st;
 }
