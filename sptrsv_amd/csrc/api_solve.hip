@@ -1317,15 +1317,17 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
         }
     }
 
+    // walks with a shape of their own, tried against the best of the above
+    std::vector<sptrsv_config_t> walks;
     // level by level in one workgroup, where a level is small
-    if (K == 1 && has_order(info) && level_walk_fits(mat, info)) shapes.push_back({SPTRSV_KERNEL_ORDER, ref, 256, 1, 4, 0});
+    if (K == 1 && has_order(info) && level_walk_fits(mat, info)) walks.push_back({SPTRSV_KERNEL_ORDER, ref, 256, 1, 4, 0});
     // the packed walk, which an ORDER analysis has no other shape for
     if (K == 1 && has_order(info))
-        shapes.push_back({has_waves(info) ? SPTRSV_KERNEL_MULTIROW : SPTRSV_KERNEL_ORDER, ref, 256, 1, 6, 0});
+        walks.push_back({has_waves(info) ? SPTRSV_KERNEL_MULTIROW : SPTRSV_KERNEL_ORDER, ref, 256, 1, 6, 0});
     // blocks of 64 rows in natural order
-    if (K == 1 && block_walk_fits(mat)) shapes.push_back({SPTRSV_KERNEL_SIMPLE, ref, 256, 1, 5, 0});
+    if (K == 1 && block_walk_fits(mat)) walks.push_back({SPTRSV_KERNEL_SIMPLE, ref, 256, 1, 5, 0});
     if (K == 1 && group_walk_lanes(mat))
-        shapes.push_back({SPTRSV_KERNEL_SIMPLE, group_walk_lanes(mat), 256, 1, 7, 0});
+        walks.push_back({SPTRSV_KERNEL_SIMPLE, group_walk_lanes(mat), 256, 1, 7, 0});
 
     hipEvent_t e0, e1;
     SPT_HIP(hipEventCreate(&e0));
@@ -1347,7 +1349,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     // Stage 1: every shape without and with a tight residency cap.
     std::vector<std::pair<float, sptrsv_config_t>> ranked;
     for (auto c : shapes) {
-        for (int cw : (c.variant == 2 ? std::vector<int>{2, 8} : c.variant >= 4 ? std::vector<int>{0} : std::vector<int>{0, 4})) {
+        for (int cw : (c.variant == 2 ? std::vector<int>{2, 8} : std::vector<int>{0, 4})) {
             c.cu_waves = cw;
             float t = time_cfg(c);
             if (status != SPTRSV_OK) break;
@@ -1373,7 +1375,6 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
             }
             if (dup) continue;
             ++taken;
-            if (c.variant >= 4) continue;  // nothing to cap
             for (int cw : (c.variant == 2 ? std::vector<int>{1, 3, 4, 6, 12, 16}
                                           : std::vector<int>{32, 16, 8, 2})) {
                 c.cu_waves = cw;
@@ -1388,7 +1389,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     }
     // Stage 3 (long rows): the best shape of each kernel with 16 entries per
     // lane in flight instead of 4, which shortens the load chain of a long row.
-    if (status == SPTRSV_OK && K == 1 && pv->max_row > 64 && bc.variant < 4) {
+    if (status == SPTRSV_OK && K == 1 && pv->max_row > 64) {
         for (int kern : {SPTRSV_KERNEL_SIMPLE, SPTRSV_KERNEL_ORDER, SPTRSV_KERNEL_MULTIROW}) {
             auto it = std::find_if(ranked.begin(), ranked.end(),
                                    [&](const auto& r) { return r.second.kernel == kern; });
@@ -1430,7 +1431,7 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
     }
     // Stage 6 (level-ordered copy): the best ORDER / MULTIROW shape walked on
     // the copy; the copy is released again when it loses.
-    if (status == SPTRSV_OK && precision != SPTRSV_PREC_F32 && bc.variant < 3 &&
+    if (status == SPTRSV_OK && precision != SPTRSV_PREC_F32 && bc.variant != 3 &&
         (bc.kernel == SPTRSV_KERNEL_ORDER || bc.kernel == SPTRSV_KERNEL_MULTIROW)) {
         sptrsv_config_t c = bc;
         c.reorder = 1;
@@ -1440,6 +1441,21 @@ int sptrsv_autotune(sp_mat_t* mat, dfr_analysis_info_t* info, int precision, int
             bc = c;
         }
         if (bc.reorder != 1) drop_level_copy(pv);
+    }
+    // Stage 7: the walks with a shape of their own, with whole rows too where
+    // they split them.
+    for (const sptrsv_config_t& walk : walks) {
+        for (int split : {0, -1}) {
+            sptrsv_config_t c = walk;
+            c.split_rows = split;
+            if (status != SPTRSV_OK || (split && split_part_words(info, walk, k) == 0)) break;
+            const float t = time_cfg(c);
+            if (status == SPTRSV_OK && t < best_t) {
+                if (bc.reorder == 1) drop_level_copy(pv);
+                best_t = t;
+                bc = c;
+            }
+        }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
