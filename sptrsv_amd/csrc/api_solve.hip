@@ -156,7 +156,7 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
 // count (diagonal, n = 10^6: 0.19 ms against 2.8).
 // Rows are taken in order (banded kernel) unless a level has 16 rows or more
 // and they are short (2D grid of 50^2: 81 us against 118).
-constexpr long long kBandRows = 16, kWideRows = 1024;
+constexpr long long kWideRows = 1024;
 bool block_walk_in_order(const sp_mat_t* m) {
     const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
     if (!pv->banded) return false;

@@ -11,6 +11,12 @@
 // bound by throughput rather than by any one member's chain).  The prepare kernel and the solve are
 // captured once in a hipGraph and replayed.
 //
+// Banded members with few rows per level are left out of the tasks: a chain a
+// row at a time through memory costs 0.8 us a row, whatever runs beside it.
+// The block walk solves them, block 0 of every member first, on a second
+// stream (16 members of up to n = 60000, FP64: 75.7 -> 2.3 ms; of up to 2000
+// 2.45 -> 0.14 ms).
+//
 // Mixed precision adds a second per-matrix choice: a strictly diagonally
 // dominant member may instead be solved by certified Jacobi refinement
 // (iterative.hip) over tiles cut inside that member, which turns a deep
@@ -33,7 +39,7 @@
 namespace sptrsv {
 
 int upload_concat(const int* n, const int* const* ia, const int* const* ja, const double* const* a,
-                  int nmat, sp_mat_t* m, std::vector<long long>& row_off);
+                  int nmat, sp_mat_t* m, std::vector<long long>& row_off, std::vector<RowShape>* shapes);
 int jacobi_solve(sp_mat_t* m, const sptrsv_config_t& c, int k, const double* b, double* x, hipStream_t s);
 int jacobi_tune(sp_mat_t* m, int k, int reps, sptrsv_config_t* best, float* best_ms);
 int reserve_jacobi(sp_mat_t* m, int k);
@@ -102,10 +108,12 @@ __global__ void k_shift(int* p, long long count, int off) {
         p[i] += off;
 }
 
+constexpr int kBandTicket = 12;  // word of the blocks' ticket
+
 template <class P>
 __global__ void k_batch_prepare(P* pub, size_t count, P unsolved, int* ticket) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) *ticket = 0;
+    if (i == 0) ticket[0] = ticket[kBandTicket] = 0;
     for (; i < count; i += (size_t)gridDim.x * blockDim.x) pub[i] = unsolved;
 }
 
@@ -128,6 +136,11 @@ struct sptrsv_batch {
     int ntasks = 0;
     Task* d_tasks_sf = nullptr;          // MIXED: the sync-free matrices only
     int ntasks_sf = 0;
+    // banded members with few rows per level: blocks of 64 rows, a member's in
+    // order, solved by the block walk instead (FP64: all; MIXED: sync-free ones)
+    std::vector<char> band;
+    int2* d_blocks[2] = {nullptr, nullptr};
+    int nblocks[2] = {0, 0};
     hipStream_t aux = nullptr;           // Jacobi half of a MIXED solve
     bool serial = false;                 // MIXED: Jacobi half, then the sync-free half, on one stream
     std::vector<long long> ent_off;      // nmat+1: first entry of each matrix
@@ -270,17 +283,44 @@ int upload_tasks(const std::vector<std::vector<Task>>& per, Task** d, int* count
     return SPTRSV_OK;
 }
 
+// Blocks of the given members, block 0 of every member first.
+int upload_blocks(const sptrsv_batch_t* bt, const std::vector<int>& members, int2** d, int* count) {
+    std::vector<int2> all;
+    long long longest = 0;
+    for (int m : members) longest = std::max(longest, bt->row_off[m + 1] - bt->row_off[m]);
+    for (long long j = 0; j < longest; j += kWave)
+        for (int m : members)
+            if (bt->row_off[m] + j < bt->row_off[m + 1])
+                all.push_back({(int)(bt->row_off[m] + j), (int)bt->row_off[m + 1]});
+    if (*d) (void)hipFree(*d);
+    *d = nullptr;
+    *count = 0;
+    if (all.empty()) return SPTRSV_OK;
+    SPT_HIP(hipMalloc(d, sizeof(int2) * all.size()));
+    SPT_HIP(hipMemcpy(*d, all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice));
+    *count = (int)all.size();
+    return SPTRSV_OK;
+}
+
 int build_tasks(sptrsv_batch_t* bt) {
     const int nmat = (int)bt->lanes.size();
     std::vector<std::vector<Task>> per(nmat), per_sf(nmat);
+    std::vector<int> band, band_sf;
     for (int m = 0; m < nmat; ++m) {
+        const bool sf = bt->choice[m] != SPTRSV_KERNEL_JACOBI;
+        if (bt->band[m]) {
+            band.push_back(m);
+            if (sf) band_sf.push_back(m);
+            continue;
+        }
         matrix_tasks(bt, m, bt->lanes[m], per[m]);
-        if (bt->choice[m] != SPTRSV_KERNEL_JACOBI) per_sf[m] = per[m];
+        if (sf) per_sf[m] = per[m];
     }
     drop_batch_graphs(bt);
     SPT_TRY(upload_tasks(per, &bt->d_tasks, &bt->ntasks));
     SPT_TRY(upload_tasks(per_sf, &bt->d_tasks_sf, &bt->ntasks_sf));
-    return SPTRSV_OK;
+    SPT_TRY(upload_blocks(bt, band, &bt->d_blocks[0], &bt->nblocks[0]));
+    return upload_blocks(bt, band_sf, &bt->d_blocks[1], &bt->nblocks[1]);
 }
 
 // Hands the tiles of the matrices whose choice is JACOBI to the Jacobi path.
@@ -304,9 +344,10 @@ int install_jacobi(sptrsv_batch_t* bt) {
     return SPTRSV_OK;
 }
 
+// fork: the blocks run beside the tasks on the auxiliary stream.
 template <class P>
-int launch_batch(sptrsv_batch_t* bt, const Task* tasks, int ntasks, const void* b, void* pub,
-                 double* x_out, hipStream_t s) {
+int launch_batch(sptrsv_batch_t* bt, const Task* tasks, int ntasks, const int2* blocks, int nblocks, bool fork,
+                 const void* b, void* pub, double* x_out, hipStream_t s) {
     MatPriv* pv = priv_of(&bt->mat);
     SolveArgs A{};
     A.n = bt->mat.nr;
@@ -327,6 +368,22 @@ int launch_batch(sptrsv_batch_t* bt, const Task* tasks, int ntasks, const void* 
     hipLaunchKernelGGL((k_batch_prepare<word>), dim3(pg), dim3(256), 0, s, static_cast<word*>(pub),
                        words, P::kUnsolved, pv->counters);
     SPT_HIP(hipGetLastError());
+    fork = fork && nblocks > 0 && ntasks > 0;
+    if (nblocks > 0) {
+        hipStream_t bs = fork ? bt->aux : s;
+        if (fork) {
+            SPT_HIP(hipEventRecord(bt->fork_ev, s));
+            SPT_HIP(hipStreamWaitEvent(bs, bt->fork_ev, 0));
+        }
+        SolveArgs B = A;
+        B.ticket = pv->counters + kBandTicket;
+        const KtPair ev = kernel_timer_pair(bs);
+        if (ev) SPT_HIP(hipEventRecord(ev[0], bs));
+        const hipError_t e = launch_band_blocks<P>(B, blocks, nblocks, bs);
+        if (e != hipSuccess) return hip_fail(e, "batch block walk", __FILE__, __LINE__);
+        if (ev) SPT_HIP(hipEventRecord(ev[1], bs));
+        if (fork) SPT_HIP(hipEventRecord(bt->join_ev, bs));
+    }
     if (ntasks > 0) {
         const KtPair ev = kernel_timer_pair(s);
         if (ev) SPT_HIP(hipEventRecord(ev[0], s));
@@ -334,16 +391,19 @@ int launch_batch(sptrsv_batch_t* bt, const Task* tasks, int ntasks, const void* 
         SPT_HIP(hipGetLastError());
         if (ev) SPT_HIP(hipEventRecord(ev[1], s));
     }
+    if (fork) SPT_HIP(hipStreamWaitEvent(s, bt->join_ev, 0));
     return SPTRSV_OK;
 }
 
 int batch_solve_tasks(sptrsv_batch_t* bt, int precision, const Task* tasks, int ntasks,
-                      const double* b, double* x, hipStream_t s) {
+                      const double* b, double* x, hipStream_t s, const int2* blocks = nullptr, int nblocks = 0,
+                      bool fork = false) {
     MatPriv* pv = priv_of(&bt->mat);
-    if (precision == SPTRSV_PREC_F64) return launch_batch<PolF64>(bt, tasks, ntasks, b, x, nullptr, s);
+    if (precision == SPTRSV_PREC_F64) 
+        return launch_batch<PolF64>(bt, tasks, ntasks, blocks, nblocks, fork, b, x, nullptr, s);
     if (precision == SPTRSV_PREC_MIXED) {
         if (pv->pub_words < (size_t)bt->mat.nr) return fail(SPTRSV_E_INVALID_ARG, "workspace missing");
-        return launch_batch<PolMixed>(bt, tasks, ntasks, b, pv->pub, x, s);
+        return launch_batch<PolMixed>(bt, tasks, ntasks, blocks, nblocks, fork, b, pv->pub, x, s);
     }
     return fail(SPTRSV_E_INVALID_ARG, "batched solves take FP64 or MIXED precision");
 }
@@ -361,14 +421,17 @@ int sync_free_half(sptrsv_batch_t* bt, int precision, const double* b, double* x
         SPT_HIP(hipGetLastError());
         return SPTRSV_OK;
     }
-    if (bt->ntasks_sf > 0) return batch_solve_tasks(bt, precision, bt->d_tasks_sf, bt->ntasks_sf, b, x, s);
+    if (bt->ntasks_sf > 0 || bt->nblocks[1] > 0)
+        return batch_solve_tasks(bt, precision, bt->d_tasks_sf, bt->ntasks_sf, b, x, s, bt->d_blocks[1], bt->nblocks[1],
+                                 bt->n_jacobi == 0);
     return SPTRSV_OK;
 }
 
 // The whole batched solve: FP64 runs every matrix sync-free; MIXED runs the
 // Jacobi matrices on the auxiliary stream while the sync-free ones run on s.
 int batch_solve_all(sptrsv_batch_t* bt, int precision, const double* b, double* x, hipStream_t s) {
-    if (precision != SPTRSV_PREC_MIXED) return batch_solve_tasks(bt, precision, bt->d_tasks, bt->ntasks, b, x, s);
+    if (precision != SPTRSV_PREC_MIXED)
+        return batch_solve_tasks(bt, precision, bt->d_tasks, bt->ntasks, b, x, s, bt->d_blocks[0], bt->nblocks[0], true);
     if (bt->n_jacobi == 0) return sync_free_half(bt, precision, b, x, s);
     if (bt->serial) {  // the two halves one after the other, each with the whole device
         SPT_TRY(jacobi_solve(&bt->mat, bt->jac_cfg, 1, b, x, s));
@@ -488,13 +551,17 @@ int sptrsv_batch_create(int nmat, const int* n, const int* const* ia, const int*
         std::lock_guard<std::mutex> g(g_batch_mu);
         g_batches.insert(bt);
     }
-    int st = upload_concat(n, ia, ja, a, nmat, &bt->mat, bt->row_off);
+    std::vector<RowShape> shapes;
+    int st = upload_concat(n, ia, ja, a, nmat, &bt->mat, bt->row_off, &shapes);
     if (st != SPTRSV_OK) {
         std::lock_guard<std::mutex> g(g_batch_mu);
         g_batches.erase(bt);
         delete bt;
         return st;
     }
+    bt->band.assign(nmat, 0);
+    for (int m = 0; m < nmat; ++m)
+        bt->band[m] = n[m] > 0 && !shapes[m].wide && n[m] < kBandRows * shapes[m].levels;
     bt->lanes.resize(nmat);
     bt->avg.resize(nmat);
     bt->delta.resize(nmat);
@@ -787,7 +854,7 @@ int tune_mixed(sptrsv_batch_t* bt, TuneScratch& ts) {
     // work in order, so they progress next to the Jacobi stream too.
     bt->serial = false;
     bt->use_sub = false;
-    if (bt->ntasks_sf > 0) {
+    if (bt->ntasks_sf > 0 || bt->nblocks[1] > 0) {
         SPT_TRY(build_sub(bt));
         bool sub_ok = bt->sub.nr > 0;
         if (sub_ok) {
@@ -936,6 +1003,8 @@ void sptrsv_batch_destroy(sptrsv_batch_t* bt) {
     }
     drop_batch_graphs(bt);
     if (bt->d_tasks) (void)hipFree(bt->d_tasks);
+    for (int2* p : bt->d_blocks)
+        if (p) (void)hipFree(p);
     if (bt->d_sub) (void)hipFree(bt->d_sub);
     if (bt->d_tasks_sf) (void)hipFree(bt->d_tasks_sf);
     if (bt->cap_stream) (void)hipStreamDestroy(bt->cap_stream);

@@ -201,8 +201,10 @@ __global__ __launch_bounds__(64) void k_block_short(SolveArgs A) {
 // eight at a time.  A wave whose predecessor has published nothing yet sleeps
 // between polls: 500 waves spinning made every hand-off slower (n = 50000 3.09
 // -> 2.04 ms).
+// blocks (of several matrices in one): first row and the matrix's end row of
+// each block, else the blocks of one matrix in order.
 template <class P>
-__global__ __launch_bounds__(64) void k_block_band(SolveArgs A) {
+__global__ __launch_bounds__(64) void k_block_band(SolveArgs A, const int2* __restrict__ blocks) {
     using word = typename P::word;
     using Acc = typename P::Acc;
     using O = BlkOps<P>;
@@ -210,10 +212,15 @@ __global__ __launch_bounds__(64) void k_block_band(SolveArgs A) {
     // [column][lane]: the block before, then this one
     __shared__ typename O::V coef[LEVEL ? 1 : 2 * kWave * kWave];
     const int lane = threadIdx.x;
-    const int base = claim_rows(A);
-    if (base >= A.n) return;
+    int base = claim_rows(A), end = A.n;
+    if (blocks) {
+        const int2 bk = blocks[base / kWave];
+        base = bk.x;
+        end = bk.y;
+    }
+    if (base >= end) return;
     const int row = base + lane, before = base - kWave;
-    const bool live = row < A.n;
+    const bool live = row < end;
     word* gpub = static_cast<word*>(A.pub);
     int p = 0, dpos = 0;
     if (live) {
@@ -312,7 +319,7 @@ template <class P>
 hipError_t launch_block_rows(const SolveArgs& A, bool banded, int longest, hipStream_t s) {
     const dim3 grid(ceil_div(A.n, kWave)), wg(kWave);
     if (banded)
-        hipLaunchKernelGGL((k_block_band<P>), grid, wg, 0, s, A);
+        hipLaunchKernelGGL((k_block_band<P>), grid, wg, 0, s, A, static_cast<const int2*>(nullptr));
     else if (longest <= kBlockRow / 2)
         hipLaunchKernelGGL((k_block_short<P, kBlockRow / 2>), grid, wg, A.dyn_lds, s, A);
     else if (longest <= kBlockRow)
@@ -321,6 +328,13 @@ hipError_t launch_block_rows(const SolveArgs& A, bool banded, int longest, hipSt
         return hipErrorInvalidValue;
     return hipGetLastError();
 }
+template <class P>
+hipError_t launch_band_blocks(const SolveArgs& A, const int2* blocks, int count, hipStream_t s) {
+    hipLaunchKernelGGL((k_block_band<P>), dim3((unsigned)count), dim3(kWave), 0, s, A, blocks);
+    return hipGetLastError();
+}
+template hipError_t launch_band_blocks<PolF64>(const SolveArgs&, const int2*, int, hipStream_t);
+template hipError_t launch_band_blocks<PolMixed>(const SolveArgs&, const int2*, int, hipStream_t);
 template hipError_t launch_block_rows<PolF64>(const SolveArgs&, bool, int, hipStream_t);
 template hipError_t launch_block_rows<PolF32>(const SolveArgs&, bool, int, hipStream_t);
 template hipError_t launch_block_rows<PolMixed>(const SolveArgs&, bool, int, hipStream_t);

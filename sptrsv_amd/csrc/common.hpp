@@ -271,6 +271,8 @@ bool block_walk_fits(const sp_mat_t* m);
 bool block_walk_in_order(const sp_mat_t* m);
 // Lanes per row of the group walk where that is the natural-order default, else 0.
 int group_walk_lanes(const sp_mat_t* m);
+// Rows per level below which a banded matrix is taken in order.
+constexpr long long kBandRows = 16;
 void free_info_arrays(dfr_analysis_info_t* info);
 // The analysis of `copy`, the level-ordered copy made for analysis `src`,
 // derived from `src` (levels permuted, iorder the identity, the rest shared).

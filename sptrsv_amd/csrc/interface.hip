@@ -313,15 +313,22 @@ static unsigned add_grid(size_t count) {
 // Uploads nmat host CSR lower triangles as one block-diagonal matrix with
 // global row and column indices; row_off receives the first row of each.
 int upload_concat(const int* n, const int* const* ia, const int* const* ja, const double* const* a,
-                  int nmat, sp_mat_t* m, std::vector<long long>& row_off) {
+                  int nmat, sp_mat_t* m, std::vector<long long>& row_off, std::vector<RowShape>* shapes) {
     memset(m, 0, sizeof(*m));
     row_off.assign(nmat + 1, 0);
     std::vector<long long> nnz_off(nmat + 1, 0);
     RowShape shape;
     for (int q = 0; q < nmat; ++q) {
         if (n[q] < 0) return fail(SPTRSV_E_INVALID_ARG, "negative size");
-        int st = validate_host_csr(ia[q], ja[q], n[q], &shape);
+        RowShape own;
+        int st = validate_host_csr(ia[q], ja[q], n[q], &own);
         if (st != SPTRSV_OK) return fail(st, "matrix " + std::to_string(q) + ": " + g_last_error);
+        shapes->push_back(own);
+        shape.longest = std::max(shape.longest, own.longest);
+        shape.wide |= own.wide;
+        shape.levels = std::max(shape.levels, own.levels);
+        shape.near += own.near;
+        shape.dist += own.dist;
         row_off[q + 1] = row_off[q] + n[q];
         nnz_off[q + 1] = nnz_off[q] + (n[q] > 0 ? (long long)ia[q][n[q]] - ia[q][0] : 0);
     }

@@ -1517,5 +1517,9 @@ extern template hipError_t launch_solve<PolLevel, 1>(int, int, int, int, const S
 constexpr int kBlockRow = 8;
 template <class P>
 hipError_t launch_block_rows(const SolveArgs& A, bool banded, int longest, hipStream_t s);
+// The banded kernel over blocks of several matrices, each matrix's in order
+// (count blocks: first row, end row of the matrix).
+template <class P>
+hipError_t launch_band_blocks(const SolveArgs& A, const int2* blocks, int count, hipStream_t s);
 
 }  // namespace sptrsv

@@ -173,3 +173,31 @@ def test_refusals():
     I.free_device_analysis(mat, None)
     db.free()
     dx.free()
+
+
+@pytest.mark.parametrize("prec", [I.PREC_F64, I.PREC_MIXED])
+def test_batch_members_in_blocks(prec):
+    """Banded members of a batch go through the block walk beside the others,
+    eager and replayed."""
+    from sptrsv_amd.interface import System
+
+    shapes = [(1, [1]), (63, [1, 2]), (64, range(1, 64)), (65, [1]), (200, [1, 17]), (700, [1, 64]), (500, [2, 90, 300]),
+              (1500, range(1, 18)), (300, [])]
+    systems, refs = [], []
+    for q, (n, offsets) in enumerate(shapes):
+        ia, ja, a, b = matrix(n, offsets, seed=q)
+        systems.append(System(n, ia, ja, a, b))
+        refs.append(O.fwd_f64(ia, ja, a, b))
+    ref = np.concatenate(refs)
+    bt = I.Batch(systems)
+    bt.tune(prec, tune=False)
+    db = I.DeviceArray.from_numpy(np.concatenate([s.b for s in systems]))
+    dx = I.DeviceArray(len(ref), np.float64)
+    for graph in (False, True, True, True):
+        bt.solve(prec, db, dx, graph=graph)
+        I.synchronize()
+        assert bt.check() == 0, L.last_error()
+        assert relerr(dx.numpy(), ref) <= BARS[prec]
+    bt.close()
+    db.free()
+    dx.free()
