@@ -292,15 +292,22 @@ size_t sort_scratch(int n) {
 }
 
 __global__ void k_longest(const int* __restrict__ ia, int n, int* __restrict__ out) {
-    __shared__ int s_max;
-    if (threadIdx.x == 0) s_max = 0;
+    __shared__ int s_max, s_long;
+    if (threadIdx.x == 0) s_max = s_long = 0;
     __syncthreads();
-    int m = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        m = max(m, ia[i + 1] - ia[i]);
+    int m = 0, longer = 0;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+        const int len = ia[i + 1] - ia[i];
+        m = max(m, len);
+        longer += len > kLongRow + 1;
+    }
     atomicMax(&s_max, m);
+    if (longer) atomicAdd(&s_long, longer);
     __syncthreads();
-    if (threadIdx.x == 0) atomicMax(out, s_max);
+    if (threadIdx.x == 0) {
+        atomicMax(out, s_max);
+        if (s_long) atomicAdd(&out[1], s_long);
+    }
 }
 
 int longest_row(const int* ia, int n, int* out, hipStream_t s) {

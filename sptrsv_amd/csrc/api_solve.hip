@@ -179,7 +179,7 @@ bool block_walk_fits(const sp_mat_t* m) {
 //    per wave on the whole device; 1340 back, n = 3*10^5: 875 -> 315 us).  Eight
 //    lanes a row serve rows of 4 to 40 entries within 8 % of the best; long
 //    rows take 32 (power-law n = 6000, 116 -> 80 us, 16 lanes 102; n = 9000, 1600
-//    back, no better than what follows).
+//    back, no better than what follows), unless they are rare (1 in 200).
 //  * Further back it is the rows in flight that count: several rows per wave
 //    (5700 back, n = 3*10^5: 863 -> 331 us; power-law n = 10^6 2.92 -> 0.73 ms),
 //    with long rows, which the others of their wave wait for, only from further
@@ -190,7 +190,7 @@ bool block_walk_fits(const sp_mat_t* m) {
 constexpr int kGroupLanes = 8;
 static void simple_shape(const sp_mat_t* m, sptrsv_config_t* c) {
     const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
-    const bool long_rows = pv->max_row > 256;
+    const bool long_rows = pv->max_row > 256 && (pv->many_long || pv->max_row > 4096);
     if (block_walk_fits(m)) {
         c->variant = 5;
     } else if (!pv->near_rows && pv->nearest < (long_rows ? 1500.0 : 2000.0)) {
@@ -239,8 +239,8 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 // kinds of matrices keep natural order all the same: banded ones with less than
 // four rows per level the block walk, which takes about 40 ns a row, the level
 // walk 170 to 200 ns a level (bandwidth 9, n = 5000: 0.21 ms against 1.00); and
-// where the packed walk would stay on one XCD, rows of up to 64 entries the
-// group walk, whose lanes read consecutive rows (random n = 10^6 2.04 against
+// where the packed walk would stay on one XCD, rows of up to 64 entries, but for a
+// few, the group walk, whose lanes read consecutive rows (random n = 10^6 2.04 against
 // 2.47 ms, n = 3*10^4 109 against 129 us; 20 entries of the last 3000, n =
 // 3*10^5, 2.45 against 2.81 ms).
 constexpr long long kChainRows = 4;
@@ -251,7 +251,8 @@ static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_
         else if (level_walk_fits(m, info)) c.variant = 4;
         else if (packed_waves(info).base) c.variant = 6;
         const int lanes = group_walk_lanes(m);
-        if (c.variant == 6 && lanes && priv_of(const_cast<sp_mat_t*>(m))->max_row <= 65 &&
+        const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
+        if (c.variant == 6 && lanes && (pv->max_row <= kLongRow + 1 || (!pv->many_long && pv->max_row <= 4096)) &&
             packed_shape(packed_waves(info).n, info->nlevs).local) {
             c.variant = 7;
             c.lanes = lanes;

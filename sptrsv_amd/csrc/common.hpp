@@ -116,7 +116,7 @@ constexpr int kCounterWords = 16;
 
 struct MatPriv {
     void* block = nullptr;       // holds ia, ja, a, a32 and src_perm of a handle made on the device
-    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4] to [7] row shape, [8] XCD of a packed walk, others spare (device)
+    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4] to [7], [9] row shape, [8] XCD of a walk, [10], [11] analysis, [12] batch (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
     size_t pub_words = 0;
     uint64_t* part = nullptr;    // published partial sums of long-row segments, 2 per segment (device)
@@ -145,6 +145,7 @@ struct MatPriv {
     int max_row = 0;             // longest row (entries incl. diagonal)
     bool banded = false;         // no column more than 63 rows back
     int band_levels = 0;         // banded: number of levels (0: not known)
+    bool many_long = false;      // more than one row in 200 has over kLongRow off-diagonals
     double nearest = 0.0;        // mean distance of a row's last off-diagonal
     bool near_rows = false;      // at least half of the rows depend on one of the kNear rows before them
     long long* trace = nullptr;  // per-row timeline (profiling), 3*n*k
@@ -247,19 +248,21 @@ int level_plan_values_changed(sp_mat_t* m);
 // Releases what the live matrices keep for the analysis with this id.
 void analysis_freed(unsigned long long id);
 // What the rows of a matrix look like, for the choice of a walk.
-constexpr int kNear = 8;
+constexpr int kNear = 8, kLongRow = 64;
 struct RowShape {
     int longest = 0;        // entries, with the diagonal
     bool wide = false;      // a column 64 or more rows back
     int levels = 0;         // while !wide; 0: not counted
     long long near = 0;     // rows whose last off-diagonal is at most kNear rows back
+    long long long_rows = 0;  // rows of more than kLongRow off-diagonals
     long long dist = 0;     // sum of the rows' distances to their last off-diagonal
-    // of the `seen` rows that near and dist were counted over
+    // of the `seen` rows that near, long_rows and dist were counted over
     void install(MatPriv* pv, long long rows, long long seen) const {
         pv->max_row = longest;
         pv->banded = !wide && rows > 0;
         pv->band_levels = wide ? 0 : levels;
         pv->near_rows = seen > 0 && 2 * near >= seen;
+        pv->many_long = 200 * long_rows > seen;
         pv->nearest = seen > 0 ? (double)dist / (double)seen : 0.0;
     }
 };
@@ -299,7 +302,8 @@ KtPair kernel_timer_pair(hipStream_t s, int launches = 1, int kind = kTimeSyncFr
 // (with sort_scratch(n) ints of scratch it only launches).
 int radix_sort_pairs(int* keys, int* vals, int* tk, int* tv, int n, int max_key, hipStream_t s, int* scratch = nullptr);
 size_t sort_scratch(int n);
-// Longest row of a device row-pointer array into *out (device, zero before).
+// Longest row of a device row-pointer array into out[0], rows of more than
+// kLongRow off-diagonals into out[1] (device, zero before).
 int longest_row(const int* ia, int n, int* out, hipStream_t s);
 
 // ---- launch helpers ----------------------------------------------------------

@@ -150,18 +150,19 @@ void free_mat(sp_mat_t* m) {
 }
 
 // out[0]: a column 64 or more rows back; out[1]: rows whose last off-diagonal
-// is at most kNear rows back; dist: the sum of those distances.  A thread leaves a row at its first far column, so long rows of
+// is at most kNear rows back; out[5]: rows of more than kLongRow off-diagonals;
+// dist: the sum of the distances.  A thread leaves a row at its first far column, so long rows of
 // wide matrices cost one load.
 __global__ __launch_bounds__(256) void k_row_shape(const int* __restrict__ ia, const int* __restrict__ ja, int n,
                                                    int* __restrict__ out, unsigned long long* __restrict__ dist) {
-    __shared__ int s_near, s_wide;
+    __shared__ int s_near, s_wide, s_long;
     __shared__ unsigned long long s_dist;
     if (threadIdx.x == 0) {
-        s_near = s_wide = 0;
+        s_near = s_wide = s_long = 0;
         s_dist = 0;
     }
     __syncthreads();
-    int near = 0, wide = 0;
+    int near = 0, wide = 0, longer = 0;
     unsigned long long far = 0;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         const int lo = ia[i], hi = ia[i + 1] - 1;
@@ -169,17 +170,20 @@ __global__ __launch_bounds__(256) void k_row_shape(const int* __restrict__ ia, c
             const int d = (int)i - ja[hi - 1];
             near += d <= kNear;
             far += d;
+            longer += hi - lo > kLongRow;
         }
         for (int p = lo; p < hi && !wide; ++p) wide = (int)i - ja[p] >= kWave;
     }
     if (near) atomicAdd(&s_near, near);
     if (far) atomicAdd(&s_dist, far);
+    if (longer) atomicAdd(&s_long, longer);
     if (wide) s_wide = 1;
     __syncthreads();
     if (threadIdx.x == 0) {
         if (s_wide) out[0] = 1;
         if (s_near) atomicAdd(&out[1], s_near);
         if (s_dist) atomicAdd(dist, s_dist);
+        if (s_long) atomicAdd(&out[5], s_long);
     }
 }
 
@@ -188,13 +192,14 @@ int install_row_shape(sp_mat_t* m, int longest) {
     shape.longest = longest;
     const int n = m->nr;
     if (n > 0) {
-        int h[4] = {}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
+        int h[6] = {}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
         hipLaunchKernelGGL(k_row_shape, dim3(std::min<unsigned>(ceil_div(n, 256), 512)), dim3(256), 0, nullptr, m->ia,
                            m->ja, n, d, reinterpret_cast<unsigned long long*>(d + 2));
         SPT_HIP(hipGetLastError());
         SPT_HIP(hipMemcpy(h, d, sizeof(h), hipMemcpyDeviceToHost));
         shape.wide = h[0] != 0;
         shape.near = h[1];
+        shape.long_rows = h[5];
         memcpy(&shape.dist, h + 2, sizeof(shape.dist));
     }
     shape.install(priv_of(m), n, n);
@@ -234,6 +239,7 @@ static int validate_host_csr(const int* ia, const int* ja, int n, RowShape* shap
             shape->dist += i - ja[e - 2];
         }
         shape->longest = std::max<int>(shape->longest, (int)(e - s));
+        shape->long_rows += e - s > kLongRow + 1;
     }
     return SPTRSV_OK;
 }
@@ -328,6 +334,7 @@ int upload_concat(const int* n, const int* const* ia, const int* const* ja, cons
         shape.wide |= own.wide;
         shape.levels = std::max(shape.levels, own.levels);
         shape.near += own.near;
+        shape.long_rows += own.long_rows;
         shape.dist += own.dist;
         row_off[q + 1] = row_off[q] + n[q];
         nnz_off[q + 1] = nnz_off[q] + (n[q] > 0 ? (long long)ia[q][n[q]] - ia[q][0] : 0);

@@ -175,6 +175,8 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     if (st == SPTRSV_OK) {
         RowShape shape;
         shape.longest = h_out[6];
+        // of all rows, so scaled to the ones seen
+        shape.long_rows = n > 0 ? (long long)h_out[7] * h_out[3] / n : 0;
         shape.wide = h_out[1] != 0;
         shape.near = h_out[2];
         memcpy(&shape.dist, h_out + 4, sizeof(shape.dist));

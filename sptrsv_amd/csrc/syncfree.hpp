@@ -1207,12 +1207,13 @@ __device__ __forceinline__ bool on_chosen_xcd(const SolveArgs& A, int* s_slot) {
 }
 
 // LOCAL: the same walk by the workgroups of one XCD; those that land on another
-// leave at once.  A hand-off from one XCD to
-// another takes 365 ns at best, the store going to memory and the poll past
-// the L2; inside one XCD a plain store is in the L2 that every CU polls, and it
-// takes 211 ns.  Where the rows of a level keep 32 CUs busy and no more, that
-// is what counts (MULTIROW solve, whole device -> one XCD: random n = 10^6, 253
-// rows per level, 5.7 -> 2.8 ms; n = 30000 274 -> 143 us).
+// leave at once.  A hand-off from one XCD to another takes 365 ns at best, the
+// store going to memory and the poll past the L2; inside one XCD a plain store
+// is in the L2 that every CU polls, and it takes 211 ns.  Where the rows of a
+// level keep 32 CUs busy and no more, that is what counts (MULTIROW solve, whole
+// device -> one XCD: random n = 10^6, 253 rows per level, 4.93 -> 2.47 ms; n =
+// 30000 245 -> 129 us).  In natural order (MODE 0) an item is the 64 / L rows of
+// a wave.
 template <class P, int WG, int U, int MODE, bool LOCAL = false>
 __global__ __launch_bounds__(WG) void k_persist(SolveArgs A) {
     __shared__ int s_base;

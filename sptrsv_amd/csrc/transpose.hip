@@ -123,13 +123,14 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
     }
     if (st == SPTRSV_OK && n > 0) {
         MatPriv* dp = priv_of(dst);
-        int mr = 0, end = 0, *longest = dp->counters + 4;  // zero since the handle was made
+        int rows[2] = {}, end = 0, *longest = dp->counters + 4;  // zero since the handle was made
         st = longest_row(dst->ia, n, longest, nullptr);
-        if (st == SPTRSV_OK) chk(hipMemcpy(&mr, longest, sizeof(int), hipMemcpyDeviceToHost), "read longest row");
+        if (st == SPTRSV_OK) chk(hipMemcpy(rows, longest, sizeof(rows), hipMemcpyDeviceToHost), "read longest row");
         if (st == SPTRSV_OK) chk(hipMemcpy(&end, dst->ia + n, sizeof(int), hipMemcpyDeviceToHost), "read row pointers");
         if (st == SPTRSV_OK && end != nnz) st = fail(SPTRSV_E_INVALID_CSR, "transpose row pointers do not sum to nnz");
         const MatPriv* from = priv_of(src);
-        dp->max_row = mr;
+        dp->max_row = rows[0];
+        dp->many_long = 200LL * rows[1] > n;
         // distances and levels are those of the source; near rows as there
         dp->banded = from->banded;
         dp->band_levels = from->band_levels;
