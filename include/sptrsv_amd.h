@@ -281,9 +281,9 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * side): one workgroup solves level by level with the results exchanged in
  * LDS, from a plan that is made on first use for the matrix and analysis (20
  * bytes for each of 64 * 5 slots per group of up to 64 rows of a level,
- * released with either; the lean path runs instead while a stream is captured
- * before the plan exists, while a trace is taken, and where no plan can be
- * made); 5 is the block walk (one right-hand side, natural order whatever the
+ * released with either; the packed walk runs instead while a stream is captured
+ * before the plan exists and where no plan can be made, the lean path while a
+ * trace is taken); 5 is the block walk (one right-hand side, natural order whatever the
  * kernel): 64 consecutive rows per wave, results of the block's own rows
  * exchanged in registers, for columns at most 63 rows back or rows of at most
  * 8 off-diagonals (other matrices, and a traced solve, take the lean path); 6

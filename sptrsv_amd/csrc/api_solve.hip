@@ -121,7 +121,6 @@ static int window_for(const MatPriv* pv, int lanes) { return (pv->max_row > 2 * 
 // takes the lean path (one row per wave for SIMPLE/ORDER, with lanes covering
 // a typical row: the next power of two >= nnz/n, 4..64); several take the
 // general engine with the reference's lanes rule.
-static void simple_shape(const sp_mat_t* m, sptrsv_config_t* c);
 static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
     sptrsv_config_t c{};
     c.kernel = kernel;
@@ -132,7 +131,6 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
         c.variant = 1;
         int avg = m->nr > 0 ? m->nnz / m->nr : 1;
         c.lanes = std::min(kWave, std::max(4, pow2_ceil(avg)));
-        if (kernel == SPTRSV_KERNEL_SIMPLE) simple_shape(m, &c);
     } else {
         c.variant = 0;
         int lanes = reference_lanes(m);
@@ -246,6 +244,7 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 constexpr long long kChainRows = 4;
 static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
     sptrsv_config_t c = shape_for(m, kernel, k);
+    if (kernel == SPTRSV_KERNEL_SIMPLE && k == 1) simple_shape(m, &c);
     if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1) {
         if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;
         else if (level_walk_fits(m, info)) c.variant = 4;
@@ -705,14 +704,13 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
         }
         if (done) return SPTRSV_OK;
         c = shape_for(m, c.kernel, k);
+        c.variant = 6;  // no plan: the packed walk needs none
     }
-    // a trace is written by the walks row by row
     const PackedWaves pw = c.variant == 6 ? packed_waves(info) : PackedWaves{};
     // a trace is written by the walks row by row
     if ((c.variant >= 5 && pv->trace) || (c.variant == 6 && !pw.base) ||
         (c.variant == 5 && !pv->banded && pv->max_row > kBlockRow + 1)) {
         c = shape_for(m, c.kernel, k);
-        if (c.variant >= 5) c.variant = 1;
     }
     const sp_mat_t* sm = lv ? lv->mat : m;
     const int K = pow2_ceil(k);
