@@ -244,6 +244,7 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 constexpr long long kChainRows = 4;
 static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
     sptrsv_config_t c = shape_for(m, kernel, k);
+    if (!m->priv) return c;  // a struct that no call has filled: nothing is known of its rows
     if (kernel == SPTRSV_KERNEL_SIMPLE && k == 1) simple_shape(m, &c);
     if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1) {
         if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;

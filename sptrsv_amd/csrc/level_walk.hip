@@ -541,7 +541,7 @@ constexpr double kLwSliceBytes = 64.0 * (kLwU * 20 + 20 + 16), kLwPlanShare = 96
 // side is the level walk.
 bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     if (!info || !info->iorder || !info->inv_iorder || !info->bucket_off || !info->level || info->nlevs < 1) return false;
-    if (info->n != m->nr || m->nr < 1 || m->nnz > kLwMaxEntries || !analysis_id(info)) return false;
+    if (!m->priv || info->n != m->nr || m->nr < 1 || m->nnz > kLwMaxEntries || !analysis_id(info)) return false;
     const bool lane_rows = static_cast<const MatPriv*>(m->priv)->max_row <= kLwU + 1;
     return (12.0 * m->nnz + 32.0 * m->nr) / info->nlevs <= (lane_rows ? kLwShortLevelBytes : kLwLevelBytes);
 }
