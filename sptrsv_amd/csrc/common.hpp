@@ -239,12 +239,11 @@ void drop_graphs(MatPriv* pv);
 void free_mat(sp_mat_t* m);  // device arrays and private state; zeroes *m
 // Releases a matrix's level-ordered copy (if any).
 void drop_level_copy(MatPriv* pv);
-// Level walk: whether it is the default shape of an analysed solve, its plan's
-// release and the plan's values after the matrix's changed.
+// Level walk: whether it is the default shape of an analysed solve, and its
+// plan's release.
 bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info);
 void drop_level_plans(MatPriv* pv);
 void drop_level_plan(MatPriv* pv, unsigned long long id);
-int level_plan_values_changed(sp_mat_t* m);
 // Releases what the live matrices keep for the analysis with this id.
 void analysis_freed(unsigned long long id);
 // What the rows of a matrix look like, for the choice of a walk.

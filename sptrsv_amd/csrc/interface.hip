@@ -531,7 +531,6 @@ int sptrsv_update_values(sp_mat_t* mat, const double* vals, long long count, int
     // the margin into their launches, so they are dropped; a tuned Jacobi
     // choice may no longer apply (dominance can be lost)
     if (mat->a) SPT_TRY(jacobi_values_changed(mat));
-    SPT_TRY(level_plan_values_changed(mat));
     drop_level_copy(pv);  // holds the old values; rebuilt on its next use
     drop_graphs(pv);
     for (int p = 0; p < 3; ++p)

@@ -15,7 +15,8 @@
 // a step of a wave is about 40 instructions (addresses computed in the kernel
 // made it 450, and the walk five times slower).
 //
-// Plan (built on the device for one matrix and analysis, on first use): slices
+// Plan (built on the device for one matrix and analysis, on first use; its
+// records are written before every walk, see k_lw_fill): slices
 // of 64 / L rows of one level and one row-length group, L lanes per row so
 // that a lane has at most kLwU entries.  A step is NW slices of a level, one
 // per wave, closed by a barrier.  Slices have a fixed size: kLwU records per
@@ -35,7 +36,7 @@
 // overflow list of their slice.
 //
 // Measured (default shape of csr_L_solve_order / _multirow before -> now): 2D
-// grid factor of 64^2 (127 levels) 120 -> 22 us, of 250^2 516 -> 125 us, random
+// grid factor of 64^2 (127 levels) 120 -> 27 us, of 250^2 516 -> 125 us, random
 // n = 2000 95 -> 23 us and 15000 203 -> 110 us, bandwidth 9 with one row per
 // level n = 5000 3.74 -> 1.00 ms: 0.15 to 0.2 us a level while a step is one or
 // two slices, 0.55 us with eight (the CU then takes in about 65 GB/s).
@@ -233,63 +234,87 @@ __global__ void k_lw_slots(const int* __restrict__ ia, const int* __restrict__ j
     if (lane == 0 && far_all) atomicAdd(&flags[2], far_all);
 }
 
-// Records of slots: the value, then the LDS byte address of a near dependency's
+// Before every walk, the records in the form it uses them, from the values the
+// matrix holds then: sp_mat_t::a and a32 may be written in place between solves.
+// The launch costs 5 us (2D grid factor 64^2, 22.1 -> 27.5 us) and 60 MB of
+// traffic over the whole device at 707^2, where it replaces a rewrite of the
+// records at every value update (two updates and two solves 1803 -> 1693 us).
+template <class T>
+struct LwFill {
+    const int2* slice;
+    int n_slices;
+    const unsigned *col, *fcol, *ocol;
+    const int *from, *ffrom, *ofrom;
+    long long n_over_slots;
+    const int *over, *order, *diag_from;
+    const T* a;
+    unsigned *rec, *frec, *orec, *rowrec;  // frec null: no far entries
+    float* piv32;
+    const T* b;  // b into position order (bp null: the walk reads it in place)
+    T* bp;
+    int n;
+};
+
+// Record of a slot: the value, then the LDS byte address of a near dependency's
 // word, or the byte offset of a far one's in memory (kLwNone: none).
 template <class T>
-__global__ void k_lw_records(const unsigned* __restrict__ col, const int* __restrict__ from, long long count, bool far,
-                             const T* __restrict__ a, unsigned* __restrict__ rec) {
+__device__ __forceinline__ void lw_record(unsigned c, int q, bool far, const T* __restrict__ a, unsigned* __restrict__ rec,
+                                          size_t i) {
     constexpr int W = 1 + sizeof(T) / 4;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-         i += (long long)gridDim.x * blockDim.x) {
-        const unsigned c = col[i];
-        const int q = from[i];
-        const T v = c && q >= 0 ? a[q] : T(0);
-        unsigned w[W - 1];
-        __builtin_memcpy(w, &v, sizeof(T));
-        const unsigned p = (c & ~kLwFar) - 1u;
-        for (int j = 0; j + 1 < W; ++j) rec[i * W + j] = w[j];
-        rec[i * W + W - 1] = far ? (c ? p * (unsigned)sizeof(T) : kLwNone)
-                                 : (c ? kLwRing0 + (p & (kLwRing - 1)) : (unsigned)kLwZero) * (unsigned)sizeof(T);
-    }
+    const T v = c && q >= 0 ? a[q] : T(0);
+    unsigned w[W - 1];
+    __builtin_memcpy(w, &v, sizeof(T));
+    const unsigned p = (c & ~kLwFar) - 1u;
+#pragma unroll
+    for (int j = 0; j + 1 < W; ++j) rec[i * W + j] = w[j];
+    rec[i * W + W - 1] = far ? (c ? p * (unsigned)sizeof(T) : kLwNone)
+                             : (c ? kLwRing0 + (p & (kLwRing - 1)) : (unsigned)kLwZero) * (unsigned)sizeof(T);
 }
 
-// Row records of every lane: word index and flags, the complement of the
-// row's byte offset in b and x (of its position's when order is null), then the reciprocal of the diagonal (FP64, FP32) or the diagonal with
-// piv32 its reciprocal in FP32 (mixed).
+// Slot records and row records, a wave per slice; overflow records; b.  Row
+// record of every lane: word index and flags, the complement of the row's byte
+// offset in b and x (of its position's where b passes through position order),
+// then the reciprocal of the diagonal (FP64, FP32) or the diagonal, with piv32
+// its reciprocal in FP32 (mixed).
+// b goes into position order, and x out of it, for matrices of more than
+// kLwInPlace rows: the rows of a level are scattered over b and x, and a gather
+// of 8 bytes costs the one CU that walks a whole line.
 template <class T, bool MIXED>
-__global__ void k_lw_rows(const int2* __restrict__ slice, int n_slices, const int* __restrict__ over,
-                          const int* __restrict__ order, const int* __restrict__ diag_from, const T* __restrict__ a,
-                          unsigned* __restrict__ rowrec, float* __restrict__ piv32) {
+__global__ void k_lw_fill(LwFill<T> F) {
     constexpr int W = 2 + sizeof(T) / 4;
     const int lane = threadIdx.x & (kWave - 1);
-    const int waves = (gridDim.x * blockDim.x) / kWave;
-    for (int s = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; s < n_slices; s += waves) {
-        const int2 d = slice[s];
+    const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long long)gridDim.x * blockDim.x;
+    for (long long s = t0 / kWave; s < F.n_slices; s += stride / kWave) {
+        const int2 d = F.slice[s];
         const int rows = d.y & 255, lg = (d.y >> 8) & 255, rl = lane >> lg;
-        const unsigned flags = ((unsigned)lg << kLwIndexBits) | (over[s] >= 0 ? kLwOverflow : 0u);
+#pragma unroll
+        for (int u = 0; u < kLwU; ++u) {
+            const size_t i = ((size_t)s * kLwU + u) * kWave + lane;
+            lw_record(F.col[i], F.from[i], false, F.a, F.rec, i);
+        }
+        const size_t i = (size_t)s * kWave + lane;
+        if (F.frec) lw_record(F.fcol[i], F.ffrom[i], true, F.a, F.frec, i);
+        const unsigned flags = ((unsigned)lg << kLwIndexBits) | (F.over[s] >= 0 ? kLwOverflow : 0u);
         unsigned r[4] = {(unsigned)lane | flags, ~kLwNone, 0u, 0u};
         float p32 = 0.0f;
         if (rl < rows && (lane & ((1 << lg) - 1)) == 0) {
             const int p = d.x + rl;
-            const T dg = a[diag_from[p]];
+            const T dg = F.a[F.diag_from[p]];
             T v = MIXED ? dg : T(1) / dg;
             if (MIXED) p32 = 1.0f / (float)dg;
             r[0] = (unsigned)(kLwRing0 + (p & (kLwRing - 1))) | flags;
-            r[1] = ~((unsigned)(order ? order[p] : p) * (unsigned)sizeof(T));
+            r[1] = ~((unsigned)(F.bp ? p : F.order[p]) * (unsigned)sizeof(T));
             __builtin_memcpy(r + 2, &v, sizeof(T));
         }
-        for (int j = 0; j < W; ++j) rowrec[((size_t)s * kWave + lane) * W + j] = r[j];
-        if (MIXED) piv32[(size_t)s * kWave + lane] = p32;
+#pragma unroll
+        for (int j = 0; j < W; ++j) F.rowrec[i * W + j] = r[j];
+        if (MIXED) F.piv32[i] = p32;
     }
+    for (long long i = t0; i < F.n_over_slots; i += stride) lw_record(F.ocol[i], F.ofrom[i], false, F.a, F.orec, i);
+    if (F.bp)
+        for (long long p = t0; p < F.n; p += stride) F.bp[p] = F.b[F.order[p]];
 }
 
-// b into position order, and x out of it: matrices of more than kLwInPlace
-// rows (the rows of a level are scattered over b and x, and a gather of 8 bytes
-// costs the one CU that walks a whole line).
-template <class T>
-__global__ void k_lw_gather(const T* __restrict__ src, const int* __restrict__ order, int n, T* __restrict__ dst) {
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) dst[p] = src[order[p]];
-}
 template <class T>
 __global__ void k_lw_scatter(const T* __restrict__ src, const int* __restrict__ order, int n, T* __restrict__ dst) {
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x)
@@ -596,42 +621,6 @@ static LwShape lw_shape(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     return sh;
 }
 
-template <class T>
-static int lw_values_of(const sp_mat_t* m, LevelPlan& L, const T* a, unsigned* rec, unsigned* frec, unsigned* orec,
-                        hipStream_t s) {
-    const long long slots = (long long)L.n_slices * kWave;
-    hipLaunchKernelGGL(k_lw_records<T>, dim3(lw_grid(slots * kLwU)), dim3(256), 0, s, L.col, L.from, slots * kLwU, false, a,
-                       rec);
-    if (L.far)
-        hipLaunchKernelGGL(k_lw_records<T>, dim3(lw_grid(slots)), dim3(256), 0, s, L.fcol, L.ffrom, slots, true, a, frec);
-    if (L.n_over)
-        hipLaunchKernelGGL(k_lw_records<T>, dim3(lw_grid((long long)L.n_over * kWave)), dim3(256), 0, s, L.ocol, L.ofrom,
-                           (long long)L.n_over * kWave, false, a, orec);
-    SPT_HIP(hipGetLastError());
-    return SPTRSV_OK;
-}
-
-// Records of one kind (0 FP64, 1 FP32, 2 mixed, which shares FP64's slots).
-static int lw_values(const sp_mat_t* m, LevelPlan& L, int kind, hipStream_t s) {
-    const unsigned g = lw_grid((long long)L.n_slices * kWave);
-    const int2* slice = static_cast<const int2*>(L.slice);
-    if (kind == 1) {
-        SPT_TRY(lw_values_of<float>(m, L, m->a32, L.rec[1], L.frec[1], L.orec[1], s));
-        hipLaunchKernelGGL((k_lw_rows<float, false>), dim3(g), dim3(256), 0, s, slice, L.n_slices, L.over, L.permuted ? nullptr : L.order,
-                           L.diag_from, m->a32, static_cast<unsigned*>(L.rows[1]), (float*)nullptr);
-    } else {
-        SPT_TRY(lw_values_of<double>(m, L, m->a, L.rec[0], L.frec[0], L.orec[0], s));
-        if (L.rows[0])
-            hipLaunchKernelGGL((k_lw_rows<double, false>), dim3(g), dim3(256), 0, s, slice, L.n_slices, L.over, L.permuted ? nullptr : L.order,
-                               L.diag_from, m->a, static_cast<unsigned*>(L.rows[0]), (float*)nullptr);
-        if (L.rows[2])
-            hipLaunchKernelGGL((k_lw_rows<double, true>), dim3(g), dim3(256), 0, s, slice, L.n_slices, L.over, L.permuted ? nullptr : L.order,
-                               L.diag_from, m->a, static_cast<unsigned*>(L.rows[2]), L.piv32);
-    }
-    SPT_HIP(hipGetLastError());
-    return SPTRSV_OK;
-}
-
 // Structure of the plan: steps, slices, slots and the entry of each slot.
 static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, LevelPlan& L) {
     const int nl = info->nlevs, n = m->nr;
@@ -757,8 +746,6 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, int kind, hi
     if (!L.n_slices) st = lw_structure(m, info, L);
     if (st == SPTRSV_OK && !L.bad) {
         hipError_t e = lw_alloc_kind(L, kind, m->nr);
-        if (e == hipSuccess) st = lw_values(m, L, kind, nullptr);
-        if (e == hipSuccess && st == SPTRSV_OK) e = hipStreamSynchronize(nullptr);
         if (e != hipSuccess) st = hip_fail(e, "level walk records", __FILE__, __LINE__);
     }
     if (st == SPTRSV_E_ALLOC) {
@@ -773,17 +760,6 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, int kind, hi
     }
     L.ready[kind] = !L.bad;
     *plan = L.bad ? nullptr : &L;
-    return SPTRSV_OK;
-}
-
-// New values on the same structure: the records are made again in place.
-int level_plan_values_changed(sp_mat_t* m) {
-    for (auto& p : priv_of(m)->lw) {
-        LevelPlan& L = p.second;
-        if (L.ready[0] || L.ready[2]) SPT_TRY(lw_values(m, L, 0, nullptr));
-        if (L.ready[1]) SPT_TRY(lw_values(m, L, 1, nullptr));
-    }
-    SPT_HIP(hipDeviceSynchronize());
     return SPTRSV_OK;
 }
 
@@ -825,18 +801,38 @@ static int lw_run(sp_mat_t* m, dfr_analysis_info_t* info, int kind, const void* 
     const KtPair ev = timed ? kernel_timer_pair(s) : KtPair{};
     if (ev) SPT_HIP(hipEventRecord(ev[0], s));
     using T = typename std::conditional<f32, float, double>::type;
-    const unsigned g = lw_grid(m->nr);
-    if (L.permuted) {
-        hipLaunchKernelGGL(k_lw_gather<T>, dim3(g), dim3(256), 0, s, static_cast<const T*>(b), L.order, m->nr,
-                           static_cast<T*>(L.b[kind]));
-        SPT_HIP(hipGetLastError());
-    }
+    LwFill<T> F{};
+    F.slice = static_cast<const int2*>(L.slice);
+    F.n_slices = L.n_slices;
+    F.col = L.col;
+    F.fcol = L.fcol;
+    F.ocol = L.ocol;
+    F.from = L.from;
+    F.ffrom = L.ffrom;
+    F.ofrom = L.ofrom;
+    F.n_over_slots = (long long)L.n_over * kWave;
+    F.over = L.over;
+    F.order = L.order;
+    F.diag_from = L.diag_from;
+    if constexpr (f32) F.a = m->a32;
+    else F.a = m->a;
+    F.rec = L.rec[k];
+    F.frec = L.far ? L.frec[k] : nullptr;
+    F.orec = L.orec[k];
+    F.rowrec = static_cast<unsigned*>(L.rows[kind]);
+    F.piv32 = L.piv32;
+    F.b = static_cast<const T*>(b);
+    F.bp = L.permuted ? static_cast<T*>(L.b[kind]) : nullptr;
+    F.n = m->nr;
+    hipLaunchKernelGGL((k_lw_fill<T, std::is_same<P, PolMixed>::value>), dim3(lw_grid((long long)L.n_slices * kWave)),
+                       dim3(256), 0, s, F);
+    SPT_HIP(hipGetLastError());
     const hipError_t e = L.nw == 1   ? lw_launch<P, 64, 4>(A, L.far, s)
                          : L.nw == 4 ? lw_launch<P, 256, 4>(A, L.far, s)
                                      : lw_launch<P, 512, 4>(A, L.far, s);
     if (e != hipSuccess) return hip_fail(e, "level walk launch", __FILE__, __LINE__);
     if (L.permuted) {
-        hipLaunchKernelGGL(k_lw_scatter<T>, dim3(g), dim3(256), 0, s, static_cast<const T*>(L.x[kind]), L.order, m->nr,
+        hipLaunchKernelGGL(k_lw_scatter<T>, dim3(lw_grid(m->nr)), dim3(256), 0, s, static_cast<const T*>(L.x[kind]), L.order, m->nr,
                            static_cast<T*>(x));
         SPT_HIP(hipGetLastError());
     }

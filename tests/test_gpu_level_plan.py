@@ -1,0 +1,59 @@
+"""GPU tests of what the level walk keeps between solves.
+
+Bars (the repository's): FP64 within 1e-12 relative (max-norm) of the oracle's
+serial substitution, FP32 within 1e-5.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle_py as O
+from sptrsv_amd import _lib as L
+from sptrsv_amd import interface as I
+
+pytestmark = pytest.mark.gpu
+
+BARS = {I.PREC_F64: 1e-12, I.PREC_MIXED: 1e-10, I.PREC_F32: 1e-5}
+
+
+def relerr(x, ref):
+    return float(np.max(np.abs(x - ref)) / max(np.max(np.abs(ref)), 1e-300))
+
+
+def write_device(ptr, array):
+    L.check(L.lib().sptrsv_memcpy_htod(ctypes.c_void_p(ptr), ctypes.c_void_p(array.ctypes.data), array.nbytes))
+
+
+@pytest.mark.parametrize("n", [3000, 20000])
+def test_values_written_in_place(n):
+    """sp_mat_t::a and a32 are the caller's to write: a solve reads them as they
+    are, whether the walk has run before or not, eager and replayed."""
+    print(f"values in place n={n}", flush=True)
+    s = I.generate(2, n)
+    mat = I.allocate_memory(s.ia, s.ja, s.a)
+    info = I.multirow_analysis_base_GPU(mat, I.ALL)
+    cfg = I._cfg(kernel=I.KERNEL_ORDER, lanes=4, variant=4)
+    for scale in (1.0, 1.0 + 2.0 ** -8, 0.75):
+        a = s.a * scale
+        write_device(mat.a, a)
+        write_device(mat.a32, a.astype(np.float32))
+        for prec, bar in BARS.items():
+            dt = np.float32 if prec == I.PREC_F32 else np.float64
+            ref = O.fwd_f64(s.ia, s.ja, a, s.b)
+            db, dx = I.DeviceArray.from_numpy(s.b.astype(dt)), I.DeviceArray(s.n, dt)
+            I.solve(mat, info, prec, db, dx, cfg=cfg)
+            assert relerr(dx.numpy().astype(np.float64), ref) <= bar, (prec, scale)
+            for again in (1.0, 0.5):
+                write_device(mat.a, a * again)
+                write_device(mat.a32, (a * again).astype(np.float32))
+                I.solve_graph(mat, info, prec, db, dx, cfg)
+                I.synchronize()
+                assert relerr(dx.numpy().astype(np.float64), ref / again) <= bar, (prec, scale, again)
+            write_device(mat.a, a)
+            write_device(mat.a32, a.astype(np.float32))
+            db.free()
+            dx.free()
+    I.free_device_analysis(mat, info)
