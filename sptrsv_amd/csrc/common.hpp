@@ -88,13 +88,12 @@ struct TileTable {
 };
 
 // Plan of the level walk (level_walk.hip) for one analysis: steps and slices,
-// their slots (dependency, and the entry the value comes from), and the records
-// of the kinds used so far (0 FP64, 1 FP32, 2 mixed).
+// their slots (dependency, and the entry the value comes from), and room for the
+// records, b and x of one solve, whichever precision it has.
 struct LevelPlan {
     bool bad = false;            // the walk is not taken for this analysis
     bool far = false;            // entries beyond the LDS ring
-    bool permuted = false;       // b and x pass through position order (L.b, L.x)
-    bool ready[3] = {false, false, false};
+    bool permuted = false;       // b and x pass through position order
     int nw = 0, nsteps = 0, n_steps_all = 0, n_slices = 0, n_over = 0;
     void* slice = nullptr;
     void* step = nullptr;
@@ -103,13 +102,13 @@ struct LevelPlan {
     int* over = nullptr;         // first overflow unit of each slice
     int* diag_from = nullptr;    // entry of each position's diagonal
     int* order = nullptr;        // row of each position
-    unsigned *rec[2] = {}, *frec[2] = {}, *orec[2] = {};
-    void* rows[3] = {};
+    // written by every solve
+    unsigned *rec = nullptr, *frec = nullptr, *orec = nullptr, *rows = nullptr;
     float* piv32 = nullptr;
     uint64_t* pub = nullptr;     // published words (mixed, far entries)
-    void *b[3] = {}, *x[3] = {};
+    double *b = nullptr, *x = nullptr;
     // the allocations that hold the arrays above
-    void *structure = nullptr, *shared = nullptr, *kind[3] = {};
+    void *structure = nullptr, *scratch = nullptr;
 };
 
 constexpr int kCounterWords = 16;

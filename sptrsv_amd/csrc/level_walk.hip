@@ -572,7 +572,7 @@ bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
 }
 
 static void free_level_plan(LevelPlan& L) {
-    for (void* p : {L.structure, L.kind[0], L.kind[1], L.kind[2], L.shared})
+    for (void* p : {L.structure, L.scratch})
         if (p) (void)hipFree(p);
     L = LevelPlan{};
 }
@@ -683,6 +683,20 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
         L.bad = f[0] != 0 || f[2] > kLwFarShare * m->nnz;
         L.n_over = f[1];
         L.far = f[2] > 0;
+        if (L.bad) return;
+        // sized for the widest records (mixed), so that solves of every
+        // precision use the same memory and none allocates
+        constexpr size_t rec_words = 3, row_words = 4;
+        Arena sc;
+        sc.add(&L.rec, slots * kLwU * rec_words);
+        sc.add(&L.frec, L.far ? slots * rec_words : 0);
+        sc.add(&L.orec, (size_t)L.n_over * kWave * rec_words);
+        sc.add(&L.rows, slots * row_words);
+        sc.add(&L.piv32, slots);
+        sc.add(&L.pub, L.far ? n : 0);
+        sc.add(&L.b, L.permuted ? n : 0);
+        sc.add(&L.x, L.permuted ? n : 0);
+        chk(sc.get(&L.scratch), "level walk records");
     };
     build();
     if (slices) (void)hipFree(slices);
@@ -693,38 +707,12 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
     return st;
 }
 
-// Memory for the records of one kind.
-static hipError_t lw_alloc_kind(LevelPlan& L, int kind, int n) {
-    const size_t slots = (size_t)L.n_slices * kWave, rb = kind == 1 ? 8 : 12;
-    const int k = kind == 1 ? 1 : 0;  // mixed shares FP64's slot records
-    Arena ar;
-    if (kind != 1 && !L.shared) {
-        Arena sh;
-        sh.add(reinterpret_cast<char**>(&L.rec[0]), slots * kLwU * rb);
-        sh.add(reinterpret_cast<char**>(&L.frec[0]), L.far ? slots * rb : 0);
-        sh.add(reinterpret_cast<char**>(&L.orec[0]), (size_t)L.n_over * kWave * rb);
-        const hipError_t e = sh.get(&L.shared);
-        if (e != hipSuccess) return e;
-    }
-    if (kind == 1) {
-        ar.add(reinterpret_cast<char**>(&L.rec[k]), slots * kLwU * rb);
-        ar.add(reinterpret_cast<char**>(&L.frec[k]), L.far ? slots * rb : 0);
-        ar.add(reinterpret_cast<char**>(&L.orec[k]), (size_t)L.n_over * kWave * rb);
-    }
-    ar.add(reinterpret_cast<char**>(&L.rows[kind]), slots * (kind == 1 ? 12 : 16));
-    if (kind == 2) ar.add(&L.piv32, slots);
-    if (kind == 2 && L.far) ar.add(&L.pub, n);
-    if (L.permuted) {
-        ar.add(reinterpret_cast<char**>(&L.b[kind]), (size_t)n * (kind == 1 ? 4 : 8));
-        ar.add(reinterpret_cast<char**>(&L.x[kind]), (size_t)n * (kind == 1 ? 4 : 8));
-    }
-    return L.kind[kind] ? hipSuccess : ar.get(&L.kind[kind]);
-}
-
-// Makes the plan for `info` and its records of one kind ready.  *plan stays
-// null where the walk cannot be taken: the stream is being captured before the
-// plan exists, there is no memory for the plan, or the analysis does not fit.
-static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, int kind, hipStream_t s, const LevelPlan** plan) {
+// The plan for `info`, made when there is none yet.  *plan stays null where the
+// walk cannot be taken: the stream is being captured before the plan exists,
+// there is no memory for the plan, or the analysis does not fit.  A plan that a
+// solve has used (and a captured solve holds) stays until its analysis or its
+// matrix goes.
+static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, hipStream_t s, const LevelPlan** plan) {
     MatPriv* pv = priv_of(m);
     *plan = nullptr;
     const unsigned long long id = analysis_id(info);
@@ -732,7 +720,7 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, int kind, hi
         info->nlevs < 1 || m->nnz > kLwMaxEntries)
         return SPTRSV_OK;
     const LevelPlan* have = find_level_plan(pv, id, false);
-    if (have && (have->bad || have->ready[kind])) {
+    if (have) {
         *plan = have->bad ? nullptr : have;
         return SPTRSV_OK;
     }
@@ -741,13 +729,8 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, int kind, hi
         (void)hipGetLastError();
         return SPTRSV_OK;
     }
-    int st = SPTRSV_OK;
     LevelPlan& L = *find_level_plan(pv, id, true);
-    if (!L.n_slices) st = lw_structure(m, info, L);
-    if (st == SPTRSV_OK && !L.bad) {
-        hipError_t e = lw_alloc_kind(L, kind, m->nr);
-        if (e != hipSuccess) st = hip_fail(e, "level walk records", __FILE__, __LINE__);
-    }
+    const int st = lw_structure(m, info, L);
     if (st == SPTRSV_E_ALLOC) {
         (void)hipGetLastError();
         free_level_plan(L);
@@ -758,7 +741,6 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, int kind, hi
         drop_level_plan(pv, id);
         return st;
     }
-    L.ready[kind] = !L.bad;
     *plan = L.bad ? nullptr : &L;
     return SPTRSV_OK;
 }
@@ -773,27 +755,25 @@ static hipError_t lw_launch(const LwArgs& A, bool far, hipStream_t s) {
 }
 
 template <class P>
-static int lw_run(sp_mat_t* m, dfr_analysis_info_t* info, int kind, const void* b, void* x, hipStream_t s, bool timed,
-                  bool* done) {
+static int lw_run(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed, bool* done) {
     constexpr bool f32 = std::is_same<P, PolF32>::value;
     const LevelPlan* plan = nullptr;
-    SPT_TRY(lw_prepare(m, info, kind, s, &plan));
+    SPT_TRY(lw_prepare(m, info, s, &plan));
     *done = plan != nullptr;
     if (!plan) return SPTRSV_OK;
     const LevelPlan& L = *plan;
-    const int k = kind == 1 ? 1 : 0;
     LwArgs A{};
     A.nsteps = L.nsteps;
     A.step = static_cast<const unsigned*>(L.step);
-    A.rec = L.rec[k];
-    A.frec = L.frec[k];
-    A.rows = L.rows[kind];
+    A.rec = L.rec;
+    A.frec = L.frec;
+    A.rows = L.rows;
     A.piv32 = L.piv32;
     A.over = L.over;
-    A.orec = L.orec[k];
+    A.orec = L.orec;
     A.ocol = L.ocol;
-    A.b = L.permuted ? L.b[kind] : b;
-    A.x = L.permuted ? L.x[kind] : x;
+    A.b = L.permuted ? L.b : b;
+    A.x = L.permuted ? L.x : x;
     A.pub = L.pub;
     A.n = (unsigned)m->nr;
     A.n_steps_all = (unsigned)L.n_steps_all;
@@ -816,13 +796,13 @@ static int lw_run(sp_mat_t* m, dfr_analysis_info_t* info, int kind, const void* 
     F.diag_from = L.diag_from;
     if constexpr (f32) F.a = m->a32;
     else F.a = m->a;
-    F.rec = L.rec[k];
-    F.frec = L.far ? L.frec[k] : nullptr;
-    F.orec = L.orec[k];
-    F.rowrec = static_cast<unsigned*>(L.rows[kind]);
+    F.rec = L.rec;
+    F.frec = L.far ? L.frec : nullptr;
+    F.orec = L.orec;
+    F.rowrec = L.rows;
     F.piv32 = L.piv32;
     F.b = static_cast<const T*>(b);
-    F.bp = L.permuted ? static_cast<T*>(L.b[kind]) : nullptr;
+    F.bp = L.permuted ? reinterpret_cast<T*>(L.b) : nullptr;
     F.n = m->nr;
     hipLaunchKernelGGL((k_lw_fill<T, std::is_same<P, PolMixed>::value>), dim3(lw_grid((long long)L.n_slices * kWave)),
                        dim3(256), 0, s, F);
@@ -832,7 +812,7 @@ static int lw_run(sp_mat_t* m, dfr_analysis_info_t* info, int kind, const void* 
                                      : lw_launch<P, 512, 4>(A, L.far, s);
     if (e != hipSuccess) return hip_fail(e, "level walk launch", __FILE__, __LINE__);
     if (L.permuted) {
-        hipLaunchKernelGGL(k_lw_scatter<T>, dim3(lw_grid(m->nr)), dim3(256), 0, s, static_cast<const T*>(L.x[kind]), L.order, m->nr,
+        hipLaunchKernelGGL(k_lw_scatter<T>, dim3(lw_grid(m->nr)), dim3(256), 0, s, reinterpret_cast<const T*>(L.x), L.order, m->nr,
                            static_cast<T*>(x));
         SPT_HIP(hipGetLastError());
     }
@@ -841,14 +821,14 @@ static int lw_run(sp_mat_t* m, dfr_analysis_info_t* info, int kind, const void* 
 }
 
 int level_walk_f64(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed, bool* done) {
-    return lw_run<PolF64>(m, info, 0, b, x, s, timed, done);
+    return lw_run<PolF64>(m, info, b, x, s, timed, done);
 }
 int level_walk_f32(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed, bool* done) {
-    return lw_run<PolF32>(m, info, 1, b, x, s, timed, done);
+    return lw_run<PolF32>(m, info, b, x, s, timed, done);
 }
 int level_walk_mixed(sp_mat_t* m, dfr_analysis_info_t* info, const void* b, void* x, hipStream_t s, bool timed,
                      bool* done) {
-    return lw_run<PolMixed>(m, info, 2, b, x, s, timed, done);
+    return lw_run<PolMixed>(m, info, b, x, s, timed, done);
 }
 
 }  // namespace sptrsv

@@ -57,3 +57,34 @@ def test_values_written_in_place(n):
             db.free()
             dx.free()
     I.free_device_analysis(mat, info)
+
+
+def free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert L.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_one_plan_serves_every_precision():
+    """Once the walk has run, a solve of another precision needs no memory (so
+    none can fail for want of it, and take with it what a captured solve holds)."""
+    s = I.generate(1, 500)
+    mat = I.allocate_memory(s.ia, s.ja, s.a)
+    info = I.multirow_analysis_base_GPU(mat, I.ALL)
+    I.reserve(mat, 1)
+    cfg = I._cfg(kernel=I.KERNEL_MULTIROW, lanes=4, variant=4)
+    bufs = {p: (I.DeviceArray.from_numpy(s.b.astype(t)), I.DeviceArray(s.n, t))
+            for p, t in ((I.PREC_F64, np.float64), (I.PREC_MIXED, np.float64), (I.PREC_F32, np.float32))}
+    I.solve_graph(mat, info, I.PREC_F64, *bufs[I.PREC_F64], cfg)
+    I.synchronize()
+    before = free_bytes()
+    for prec in (I.PREC_F32, I.PREC_MIXED):
+        I.solve(mat, info, prec, *bufs[prec], cfg=cfg)
+        I.synchronize()
+        assert free_bytes() == before, prec
+    for prec in (I.PREC_F64, I.PREC_F32, I.PREC_MIXED, I.PREC_F64):
+        bufs[prec][1].fill_bytes(0)
+        I.solve_graph(mat, info, prec, *bufs[prec], cfg)
+        I.synchronize()
+        assert O.validate_x(bufs[prec][1].numpy().astype(np.float64)) == 0, prec
+    I.free_device_analysis(mat, info)
