@@ -88,3 +88,33 @@ def test_one_plan_serves_every_precision():
         I.synchronize()
         assert O.validate_x(bufs[prec][1].numpy().astype(np.float64)) == 0, prec
     I.free_device_analysis(mat, info)
+
+
+def test_analyses_freed_while_values_change():
+    """One thread updates a matrix's values and solves while another releases
+    other analyses of it, whose plans go with them."""
+    import threading
+
+    s = I.generate(1, 40)
+    mat = I.allocate_memory(s.ia, s.ja, s.a)
+    cfg = I._cfg(kernel=I.KERNEL_ORDER, lanes=4, variant=4)
+    db, dx = I.DeviceArray.from_numpy(s.b), I.DeviceArray(s.n, np.float64)
+    keep, others = I.multirow_analysis_base_GPU(mat, I.ORDER), []
+    for _ in range(40):
+        others.append(I.multirow_analysis_base_GPU(mat, I.ORDER))
+        I.solve(mat, others[-1], I.PREC_F64, db, dx, cfg=cfg)
+    I.synchronize()
+
+    def release():
+        for info in others:
+            I.free_device_analysis(None, info)
+
+    t = threading.Thread(target=release)
+    t.start()
+    for i in range(60):
+        scale = 2.0 ** (i % 3 - 1)
+        I.update_values(mat, s.a * scale)
+        I.solve(mat, keep, I.PREC_F64, db, dx, cfg=cfg)
+        assert np.array_equal(dx.numpy(), np.full(s.n, 1.0 / scale))
+    t.join()
+    I.free_device_analysis(mat, keep)
