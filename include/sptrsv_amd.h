@@ -279,11 +279,13 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * the column pattern, then folds its entries exactly as variant 1 does (same
  * results, bit for bit); 4 is the level walk (ORDER/MULTIROW, one right-hand
  * side): one workgroup solves level by level with the results exchanged in
- * LDS, from a plan that is made on first use for the matrix and analysis (20
- * bytes for each of 64 * 5 slots per group of up to 64 rows of a level,
- * released with either; the packed walk runs instead while a stream is captured
- * before the plan exists and where no plan can be made, the lean path while a
- * trace is taken); 5 is the block walk (one right-hand side, natural order whatever the
+ * LDS, from a plan for the matrix and analysis (20 bytes for each of 64 * 5
+ * slots per group of up to 64 rows of a level, released with either).  An
+ * analysis makes the plan where the walk is the default, so that no solve
+ * allocates or waits; for others it is made by the first solve that names the
+ * variant.  The packed walk runs instead where no plan can be made and while
+ * the stream is captured before there is one, the lean path while a trace is
+ * taken; 5 is the block walk (one right-hand side, natural order whatever the
  * kernel): 64 consecutive rows per wave, results of the block's own rows
  * exchanged in registers, for columns at most 63 rows back or rows of at most
  * 8 off-diagonals (other matrices, and a traced solve, take the lean path); 6
@@ -303,8 +305,8 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * shape of the kernel, else from the default shape (SIMPLE: the block walk for
  * banded matrices and grid-like ones, the group walk where rows depend on rows
  * up to some thousands back, else variants 0 or 2; ORDER and MULTIROW: the level
- * walk where a level's share of the matrix is small, else the group or the
- * packed walk; several right-hand sides with an analysis: variant 2 of ORDER);
+ * walk where a level's share of the matrix is small (and the analysis was made
+ * for this handle), else the group or the packed walk; several right-hand sides with an analysis: variant 2 of ORDER);
  * MULTIROW takes its lanes
  * per row from the analysis and ignores a nonzero lanes. */
 typedef struct {

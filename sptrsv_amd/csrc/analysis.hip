@@ -632,29 +632,43 @@ __global__ void k_bucket_counts(const int* __restrict__ bucket_off, int nb, int*
 }
 
 // What solves derive from an analysis: the long-row segments of the wave64
-// layout, and that layout itself where the mode leaves it out.
-static int build_derived(dfr_analysis_info_t* info, sp_mat_t* m) {
+// layout, that layout itself where the mode leaves it out, and the level walk's
+// plan.  All of it is made here, where there is an allocation and a wait
+// anyway: a solve, the first one too, only launches.
+// Working memory: bucket counts, build_warps's and the plan's (null: not at hand).
+struct DerivedWork {
+    const int* bucket_cnt = nullptr;
+    int *wpb = nullptr, *plan = nullptr;
+};
+static int build_derived(dfr_analysis_info_t* info, sp_mat_t* m, bool plan, const DerivedWork& work = {}) {
     if (info->mode == ORDER && info->n > 0 && owns_info(info)) {
         InfoPriv* ip = static_cast<InfoPriv*>(info->priv);
         const int nb = 7 * info->nlevs;
-        int *cnt = nullptr, *wpb = nullptr;
+        int st = SPTRSV_OK;
         void* tmp = nullptr;
-        Arena ar;
-        ar.add(&cnt, nb + 1);
-        ar.add(&wpb, nb + 1 + scan_scratch(nb + 1));
-        SPT_HIP(ar.get(&tmp));
-        hipLaunchKernelGGL(k_bucket_counts, dim3(grid_for(nb)), dim3(256), 0, nullptr, info->bucket_off, nb, cnt);
-        int st = hipGetLastError() == hipSuccess ? SPTRSV_OK : fail(SPTRSV_E_HIP, "bucket counts");
-        if (st == SPTRSV_OK)
-            st = build_warps(cnt, info->bucket_off, nb, 64, info->n, &ip->wbase, &ip->wsize, &ip->n_waves, wpb, nullptr);
+        if (work.bucket_cnt) {
+            st = build_warps(work.bucket_cnt, info->bucket_off, nb, 64, info->n, &ip->wbase, &ip->wsize, &ip->n_waves,
+                             work.wpb, nullptr);
+        } else {
+            int *cnt = nullptr, *wpb = nullptr;
+            Arena ar;
+            ar.add(&cnt, nb + 1);
+            ar.add(&wpb, nb + 1 + scan_scratch(nb + 1));
+            SPT_HIP(ar.get(&tmp));
+            hipLaunchKernelGGL(k_bucket_counts, dim3(grid_for(nb)), dim3(256), 0, nullptr, info->bucket_off, nb, cnt);
+            st = hipGetLastError() == hipSuccess ? SPTRSV_OK : fail(SPTRSV_E_HIP, "bucket counts");
+            if (st == SPTRSV_OK)
+                st = build_warps(cnt, info->bucket_off, nb, 64, info->n, &ip->wbase, &ip->wsize, &ip->n_waves, wpb, nullptr);
+        }
         if (st == SPTRSV_OK && hipStreamSynchronize(nullptr) != hipSuccess) st = fail(SPTRSV_E_HIP, "wave layout");
-        (void)hipFree(tmp);
+        if (tmp) (void)hipFree(tmp);
         if (st != SPTRSV_OK) return st;
     }
-    return build_segments(info, m);
+    SPT_TRY(build_segments(info, m));
+    return plan ? make_level_plan(m, info, work.plan) : SPTRSV_OK;
 }
 
-static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
+static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode, bool plan) {
     hipStream_t s = nullptr;
     MatPriv* pv = priv_of(m);
     const int n = m->nr;
@@ -764,7 +778,7 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
     const int nb = 7 * nlevs;
 
     // 3. keys and histograms
-    int *key = nullptr, *tk = nullptr, *tv = nullptr, *bucket_cnt = nullptr, *scratch = nullptr, *wpb = nullptr;
+    int *key = nullptr, *tk = nullptr, *tv = nullptr, *bucket_cnt = nullptr, *scratch = nullptr, *wpb = nullptr, *work = nullptr;
     struct Temp {
         void* p = nullptr;
         ~Temp() {
@@ -779,6 +793,7 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         ar.add(&bucket_cnt, nb + 1);
         ar.add(&scratch, std::max(sort_scratch(n), scan_scratch(nb + 1)));
         ar.add(&wpb, nb + 1 + scan_scratch(nb + 1));
+        ar.add(&work, level_plan_work(nlevs));
         SPT_HIP(ar.get(&tmp.p));
     }
     SPT_HIP(hipMalloc(&info->bucket_off, sizeof(int) * (size_t)(nb + 1)));
@@ -825,7 +840,7 @@ static int analyse(dfr_analysis_info_t* info, sp_mat_t* m, MODE mode) {
         SPT_HIP(hipGetLastError());
     }
     SPT_HIP(hipStreamSynchronize(s));
-    return build_derived(info, m);
+    return build_derived(info, m, plan && mode != SIMPLE, {bucket_cnt, wpb, work});
 }
 
 // ---- analysis files and copies ------------------------------------------------------
@@ -1007,7 +1022,7 @@ int sptrsv_load_analysis(const char* path, sp_mat_t* mat, dfr_analysis_info_t* i
             hipMemcpy(*a.dev, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
             st = fail(SPTRSV_E_ALLOC, "analysis arrays");
     }
-    if (st == SPTRSV_OK) st = build_derived(info, mat);
+    if (st == SPTRSV_OK) st = build_derived(info, mat, info->mode != SIMPLE);
     if (st != SPTRSV_OK) free_info_arrays(info);
     return st;
 }
@@ -1040,12 +1055,15 @@ int sptrsv_copy_analysis(sp_mat_t* src_mat, dfr_analysis_info_t* src, sp_mat_t* 
             hipMemcpy(*to[i].dev, *from[i].dev, bytes, hipMemcpyDeviceToDevice) != hipSuccess)
             st = fail(SPTRSV_E_ALLOC, "analysis arrays");
     }
-    if (st == SPTRSV_OK) st = build_derived(dst, dst_mat);
+    if (st == SPTRSV_OK) st = build_derived(dst, dst_mat, dst->mode != SIMPLE);
     if (st != SPTRSV_OK) free_info_arrays(dst);
     return st;
 }
 
-int multirow_analysis_base_GPU(dfr_analysis_info_t** info, sp_mat_t* gpu_L, MODE mode) {
+}  // extern "C"
+
+namespace sptrsv {
+int level_analysis(dfr_analysis_info_t** info, sp_mat_t* gpu_L, MODE mode, bool plan) {
     if (!info || !gpu_L || !gpu_L->priv) return fail(SPTRSV_E_INVALID_ARG, "null info or matrix");
     if (mode != ORDER && mode != MULTIROW && mode != ALL && mode != SIMPLE)
         return fail(SPTRSV_E_INVALID_ARG, "unknown MODE");
@@ -1053,9 +1071,16 @@ int multirow_analysis_base_GPU(dfr_analysis_info_t** info, sp_mat_t* gpu_L, MODE
         *info = static_cast<dfr_analysis_info_t*>(calloc(1, sizeof(dfr_analysis_info_t)));
         if (!*info) return fail(SPTRSV_E_ALLOC, "info struct");
     }
-    int st = analyse(*info, gpu_L, mode);
+    int st = analyse(*info, gpu_L, mode, plan);
     if (st != SPTRSV_OK) free_info_arrays(*info);
     return st;
+}
+}  // namespace sptrsv
+
+extern "C" {
+
+int multirow_analysis_base_GPU(dfr_analysis_info_t** info, sp_mat_t* gpu_L, MODE mode) {
+    return level_analysis(info, gpu_L, mode, true);
 }
 
 int sptrsv_analysis_segments(const dfr_analysis_info_t* info, int* n_split_rows, int* n_segments) {

@@ -248,7 +248,7 @@ static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_
     if (kernel == SPTRSV_KERNEL_SIMPLE && k == 1) simple_shape(m, &c);
     if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1) {
         if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;
-        else if (level_walk_fits(m, info)) c.variant = 4;
+        else if (level_plan_made(m, info)) c.variant = 4;
         else if (packed_waves(info).base) c.variant = 6;
         const int lanes = group_walk_lanes(m);
         const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
@@ -287,8 +287,9 @@ int default_config(const sp_mat_t* m, const dfr_analysis_info_t* info, int preci
     // 64-lane layout is made for one (16, 3D grid 128^3: 10.9 ms against 0.98)
     if (k > 1 && has_order(info)) kernel = SPTRSV_KERNEL_ORDER;
     *out = analysed_shape_for(m, info, kernel, k);
-    // an ALL analysis asks for no kernel, and may be there for one solve only:
-    // the packed walk, which needs no plan, or natural order for a chain
+    // an ALL analysis asks for no kernel, and may be there for one solve only
+    // (the spsv-style handle's, which is made without a plan): the packed walk,
+    // or natural order for a chain
     if (k == 1 && info && info->mode == ALL && has_waves(info)) {
         *out = analysed_shape_for(m, info, SPTRSV_KERNEL_MULTIROW, k);
         if (out->variant == 4) out->variant = 6;

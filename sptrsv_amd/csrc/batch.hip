@@ -512,7 +512,7 @@ int build_sub(sptrsv_batch_t* bt) {
     if (st == SPTRSV_OK) chk(hipMemcpy(S.ia + rows, &last, sizeof(int), hipMemcpyHostToDevice), "ia end");
     if (st == SPTRSV_OK) st = convert_values_to_f32(&S);
     if (st == SPTRSV_OK) chk(hipDeviceSynchronize(), "sub build");
-    if (st == SPTRSV_OK) st = multirow_analysis_base_GPU(&bt->sub_info, &S, ALL);
+    if (st == SPTRSV_OK) st = level_analysis(&bt->sub_info, &S, ALL, false);
     if (st == SPTRSV_OK) st = reserve_part(&S, bt->sub_info);  // captured solves allocate nothing
     if (st != SPTRSV_OK) free_sub(bt);
     return st;

@@ -107,8 +107,7 @@ struct LevelPlan {
     float* piv32 = nullptr;
     uint64_t* pub = nullptr;     // published words (mixed, far entries)
     double *b = nullptr, *x = nullptr;
-    // the allocations that hold the arrays above
-    void *structure = nullptr, *scratch = nullptr;
+    void* block = nullptr;       // the allocation that holds the arrays above
 };
 
 constexpr int kCounterWords = 16;
@@ -238,11 +237,18 @@ void drop_graphs(MatPriv* pv);
 void free_mat(sp_mat_t* m);  // device arrays and private state; zeroes *m
 // Releases a matrix's level-ordered copy (if any).
 void drop_level_copy(MatPriv* pv);
-// Level walk: whether it is the default shape of an analysed solve, and its
-// plan's release.
+// Level walk: whether its rule takes this matrix and analysis, whether they have
+// a plan (the walk is then the default shape of an analysed solve), making it
+// where the rule says so, and its release.
 bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info);
+bool level_plan_made(const sp_mat_t* m, const dfr_analysis_info_t* info);
+// (work: level_plan_work words, or null)
+int make_level_plan(sp_mat_t* m, const dfr_analysis_info_t* info, int* work);
+size_t level_plan_work(int nlevs);
 void drop_level_plans(MatPriv* pv);
 void drop_level_plan(MatPriv* pv, unsigned long long id);
+// multirow_analysis_base_GPU, without the level walk's plan unless asked for.
+int level_analysis(dfr_analysis_info_t** info, sp_mat_t* m, MODE mode, bool plan);
 // Releases what the live matrices keep for the analysis with this id.
 void analysis_freed(unsigned long long id);
 // What the rows of a matrix look like, for the choice of a walk.

@@ -15,7 +15,8 @@
 // a step of a wave is about 40 instructions (addresses computed in the kernel
 // made it 450, and the walk five times slower).
 //
-// Plan (built on the device for one matrix and analysis, on first use; its
+// Plan (built on the device for one matrix and analysis, with the analysis where
+// the walk is a default and else on the first solve that names it; its
 // records are written before every walk, see k_lw_fill): slices
 // of 64 / L rows of one level and one row-length group, L lanes per row so
 // that a lane has at most kLwU entries.  A step is NW slices of a level, one
@@ -562,8 +563,8 @@ constexpr double kLwFarShare = 0.01;
 // may take per entry of the matrix and in any case.
 constexpr double kLwSliceBytes = 64.0 * (kLwU * 20 + 20 + 16), kLwPlanShare = 96.0, kLwPlanFree = 32.0 * 1024 * 1024;
 
-// Whether the default shape of an ORDER or MULTIROW solve with one right-hand
-// side is the level walk.
+// Whether an analysis gets a plan, with which the level walk is the default shape
+// of an ORDER or MULTIROW solve with one right-hand side.
 bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     if (!info || !info->iorder || !info->inv_iorder || !info->bucket_off || !info->level || info->nlevs < 1) return false;
     if (!m->priv || info->n != m->nr || m->nr < 1 || m->nnz > kLwMaxEntries || !analysis_id(info)) return false;
@@ -572,8 +573,7 @@ bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
 }
 
 static void free_level_plan(LevelPlan& L) {
-    for (void* p : {L.structure, L.scratch})
-        if (p) (void)hipFree(p);
+    if (L.block) (void)hipFree(L.block);
     L = LevelPlan{};
 }
 
@@ -603,6 +603,12 @@ static LevelPlan* find_level_plan(MatPriv* pv, unsigned long long id, bool make)
     return make ? &pv->lw[id] : nullptr;
 }
 
+bool level_plan_made(const sp_mat_t* m, const dfr_analysis_info_t* info) {
+    const unsigned long long id = analysis_id(info);
+    const LevelPlan* L = id ? find_level_plan(static_cast<MatPriv*>(m->priv), id, false) : nullptr;
+    return L && !L->bad && info->n == m->nr && level_walk_fits(m, info);
+}
+
 static unsigned lw_grid(long long threads) {
     return (unsigned)std::max<long long>(1, std::min<long long>((threads + 255) / 256, 8192));
 }
@@ -621,27 +627,30 @@ static LwShape lw_shape(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     return sh;
 }
 
-// Structure of the plan: steps, slices, slots and the entry of each slot.
-static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, LevelPlan& L) {
+// Words of working memory to make a plan.
+size_t level_plan_work(int nlevs) { return 2 * ((size_t)nlevs + 1) + 3 + scan_scratch((long long)nlevs + 1); }
+
+// The plan: steps, slices, slots and the entry of each slot, with room for one
+// solve's records.  work: level_plan_work words, or null to allocate them.
+static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, LevelPlan& L, int* work) {
     const int nl = info->nlevs, n = m->nr;
     const LwShape sh = lw_shape(m, info);
     L.nw = sh.nw;
     L.permuted = n > kLwInPlace;
     hipStream_t s = nullptr;
-    int *slices = nullptr, *steps = nullptr, *flags = nullptr;
+    int* own = nullptr;
     int st = SPTRSV_OK;
     auto chk = [&](hipError_t e, const char* what) {
         if (e != hipSuccess && st == SPTRSV_OK) st = hip_fail(e, what, __FILE__, __LINE__);
         return st == SPTRSV_OK;
     };
     auto build = [&]() {
-        if (!chk(hipMalloc(&slices, sizeof(int) * (2 * ((size_t)nl + 1) + 3)), "level walk count")) return;
-        steps = slices + nl + 1;
-        flags = steps + nl + 1;
+        if (!work && !chk(hipMalloc(&own, sizeof(int) * level_plan_work(nl)), "level walk count")) return;
+        int *slices = work ? work : own, *steps = slices + nl + 1, *flags = steps + nl + 1, *sums = flags + 3;
         hipLaunchKernelGGL(k_lw_count, dim3(lw_grid(nl + 1)), dim3(256), 0, s, info->bucket_off, nl, sh, slices, steps, flags);
         if (!chk(hipGetLastError(), "level walk count")) return;
-        if ((st = exclusive_scan(slices, slices, (long long)nl + 1, s)) != SPTRSV_OK) return;
-        if ((st = exclusive_scan(steps, steps, (long long)nl + 1, s)) != SPTRSV_OK) return;
+        if ((st = exclusive_scan(slices, slices, (long long)nl + 1, s, sums)) != SPTRSV_OK) return;
+        if ((st = exclusive_scan(steps, steps, (long long)nl + 1, s, sums)) != SPTRSV_OK) return;
         std::vector<int> h((size_t)nl + 2);  // both totals in one copy
         if (!chk(hipMemcpy(h.data(), slices + nl, sizeof(int) * h.size(), hipMemcpyDeviceToHost), "level walk count")) return;
         L.n_slices = h.front();
@@ -668,7 +677,21 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
         ar.add(&L.ofrom, (size_t)over_cap * kWave);
         ar.add(&L.diag_from, n);
         ar.add(&L.order, n);
-        if (!chk(ar.get(&L.structure), "level walk plan")) return;
+        // the records: sized for the widest ones (mixed), so that solves of every
+        // precision use the same memory and none allocates; with all that far
+        // entries and overflow lists can take, which is known only later (one
+        // allocation: each costs an analysis some 20 us, its release as much)
+        constexpr size_t rec_words = 3, row_words = 4;
+        const bool may_far = lw_near(n - 1) > 0;
+        ar.add(&L.rec, slots * kLwU * rec_words);
+        ar.add(&L.frec, may_far ? slots * rec_words : 0);
+        ar.add(&L.orec, (size_t)over_cap * kWave * rec_words);
+        ar.add(&L.rows, slots * row_words);
+        ar.add(&L.piv32, slots);
+        ar.add(&L.pub, may_far ? n : 0);
+        ar.add(&L.b, L.permuted ? n : 0);
+        ar.add(&L.x, L.permuted ? n : 0);
+        if (!chk(ar.get(&L.block), "level walk plan")) return;
         L.slice = slice;
         L.step = step;
         hipLaunchKernelGGL(k_lw_slices, dim3(lw_grid(nl)), dim3(256), 0, s, info->bucket_off, nl, sh, slices, steps,
@@ -683,23 +706,9 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
         L.bad = f[0] != 0 || f[2] > kLwFarShare * m->nnz;
         L.n_over = f[1];
         L.far = f[2] > 0;
-        if (L.bad) return;
-        // sized for the widest records (mixed), so that solves of every
-        // precision use the same memory and none allocates
-        constexpr size_t rec_words = 3, row_words = 4;
-        Arena sc;
-        sc.add(&L.rec, slots * kLwU * rec_words);
-        sc.add(&L.frec, L.far ? slots * rec_words : 0);
-        sc.add(&L.orec, (size_t)L.n_over * kWave * rec_words);
-        sc.add(&L.rows, slots * row_words);
-        sc.add(&L.piv32, slots);
-        sc.add(&L.pub, L.far ? n : 0);
-        sc.add(&L.b, L.permuted ? n : 0);
-        sc.add(&L.x, L.permuted ? n : 0);
-        chk(sc.get(&L.scratch), "level walk records");
     };
     build();
-    if (slices) (void)hipFree(slices);
+    if (own) (void)hipFree(own);
     if (L.bad) {
         free_level_plan(L);
         L.bad = true;
@@ -708,11 +717,13 @@ static int lw_structure(const sp_mat_t* m, const dfr_analysis_info_t* info, Leve
 }
 
 // The plan for `info`, made when there is none yet.  *plan stays null where the
-// walk cannot be taken: the stream is being captured before the plan exists,
-// there is no memory for the plan, or the analysis does not fit.  A plan that a
+// walk cannot be taken: the stream is being captured before the plan exists
+// (a solve that names the walk for a matrix whose analysis made none), there is
+// no memory for the plan, or the analysis does not fit.  A plan that a
 // solve has used (and a captured solve holds) stays until its analysis or its
 // matrix goes.
-static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, hipStream_t s, const LevelPlan** plan) {
+static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, hipStream_t s, const LevelPlan** plan,
+                      int* work = nullptr) {
     MatPriv* pv = priv_of(m);
     *plan = nullptr;
     const unsigned long long id = analysis_id(info);
@@ -730,7 +741,7 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, hipStream_t 
         return SPTRSV_OK;
     }
     LevelPlan& L = *find_level_plan(pv, id, true);
-    const int st = lw_structure(m, info, L);
+    const int st = lw_structure(m, info, L, work);
     if (st == SPTRSV_E_ALLOC) {
         (void)hipGetLastError();
         free_level_plan(L);
@@ -743,6 +754,11 @@ static int lw_prepare(sp_mat_t* m, const dfr_analysis_info_t* info, hipStream_t 
     }
     *plan = L.bad ? nullptr : &L;
     return SPTRSV_OK;
+}
+
+int make_level_plan(sp_mat_t* m, const dfr_analysis_info_t* info, int* work) {
+    const LevelPlan* plan = nullptr;
+    return level_walk_fits(m, info) ? lw_prepare(m, info, nullptr, &plan, work) : SPTRSV_OK;
 }
 
 template <class P, int WG, int D>

@@ -234,7 +234,9 @@ int sptrsv_spsv_analysis(sptrsv_spsv_t* h, int precision, int k, int tune) {
     if (h->analysed) free_device_analysis(nullptr, &h->info);
     h->analysed = false;
     dfr_analysis_info_t* p = &h->info;
-    SPT_TRY(multirow_analysis_base_GPU(&p, &h->mat, ALL));
+    // often for one solve, and solved with the shape an ALL analysis has by
+    // default, which needs no plan (with one, random n = 3000 took 7 % longer)
+    SPT_TRY(level_analysis(&p, &h->mat, ALL, false));
     h->analysed = true;
     if (tune && h->mat.nr > 0) {
         sptrsv_config_t best{};

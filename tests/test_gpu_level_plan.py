@@ -118,3 +118,40 @@ def test_analyses_freed_while_values_change():
         assert np.array_equal(dx.numpy(), np.full(s.n, 1.0 / scale))
     t.join()
     I.free_device_analysis(mat, keep)
+
+
+@pytest.mark.parametrize("mode", [I.ORDER, I.MULTIROW, I.ALL])
+def test_first_solve_beside_a_capture(mode):
+    """The first solve with an analysis allocates nothing and waits for nothing:
+    it runs while another stream is captured in the mode that forbids both."""
+    hip = L.lib()
+    s = I.generate(1, 200)
+    mat = I.allocate_memory(s.ia, s.ja, s.a)
+    info = I.multirow_analysis_base_GPU(mat, mode)
+    db, dx = I.DeviceArray.from_numpy(s.b), I.DeviceArray(s.n, np.float64)
+    b32, x32 = I.DeviceArray.from_numpy(s.b.astype(np.float32)), I.DeviceArray(s.n, np.float32)
+    dx.fill_bytes(0)
+    x32.fill_bytes(0)
+    I.synchronize()
+    streams = [ctypes.c_void_p() for _ in range(2)]
+    for st in streams:
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(st), 1) == 0      # not tied to the null stream
+    graph, errors = ctypes.c_void_p(), []
+    assert hip.hipStreamBeginCapture(streams[0], 0) == 0                   # global mode
+    try:
+        if mode == I.MULTIROW:
+            I.csr_L_solve_multirow(mat, info, db, dx, stream=streams[1])
+            I.csr_L_solve_multirow_f32(mat, info, b32, x32, stream=streams[1])
+        else:
+            I.csr_L_solve_order(mat, info, db, dx, stream=streams[1])
+            I.csr_L_solve_order_f32(mat, info, b32, x32, stream=streams[1])
+    except L.SptrsvError as e:
+        errors.append(str(e))
+    ended = hip.hipStreamEndCapture(streams[0], ctypes.byref(graph))
+    assert not errors and ended == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamSynchronize(streams[1]) == 0
+    assert O.validate_x(dx.numpy()) == 0 and np.all(x32.numpy() == 1.0)
+    for st in streams:
+        assert hip.hipStreamDestroy(st) == 0
+    I.free_device_analysis(mat, info)
