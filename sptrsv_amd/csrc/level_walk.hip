@@ -550,12 +550,19 @@ __global__ __launch_bounds__(WG) void k_level_walk(LwArgs A) {
 
 // ---- host ------------------------------------------------------------------------------
 
-// A level's share of the matrix up to which one CU streaming it all beats the
-// packed walk.  Rows of at most kLwU off-diagonals, a lane each: 0.60 ms against
-// 0.68 at 20 KB (2D grid 600^2), 0.79 against 0.80 at 23.5 (707^2), 1.31 against
-// 1.18 at 33 (1000^2).  Longer rows, spread over lanes with room left over: 55
-// us against 86 at 12 KB (random n = 10000), 114 against 102 at 15 (n = 15000).
-constexpr double kLwLevelBytes = 13.0 * 1024.0, kLwShortLevelBytes = 26.0 * 1024.0;
+// A level's share of the matrix up to which one CU streaming it all, its records
+// written before, beats the walks that need no plan (and is worth one: 50 to 90
+// us of an analysis of 4000 rows).  Level walk against the best of the others,
+// us, FP64 (mixed):
+//  * rows of at most kLwU off-diagonals, a lane each: 131 / 248 (189 / 265) at
+//    8.3 KB (2D grid 250^2), 354 / 397 (418 / 424) at 13.3 KB, 454 / 497 (529 /
+//    533) at 16.6, 624 / 603 (730 / 649) at 19.9 (600^2), 820 / 722 at 23.5;
+//  * rows of up to kLongRow, spread over lanes with room left over: 31 / 45 (42
+//    / 49) at 3.4 KB (random n = 2000), 41 / 54 (54 / 59) at 5.9 KB, 62 / 59
+//    (71 / 64) at 8.1;
+//  * longer ones take a slice each: 50 / 52 (64 / 58) at 4.8 KB (power-law n =
+//    2000), 73 / 58 at 6.8; never.
+constexpr double kLwLevelBytes = 6.0 * 1024.0, kLwShortLevelBytes = 16.0 * 1024.0;
 constexpr long long kLwMaxEntries = 1ll << 27;  // buffer descriptors address 4 GB
 // Share of far entries above which the walk is not taken (their loads wait).
 constexpr double kLwFarShare = 0.01;
@@ -568,7 +575,9 @@ constexpr double kLwSliceBytes = 64.0 * (kLwU * 20 + 20 + 16), kLwPlanShare = 96
 bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     if (!info || !info->iorder || !info->inv_iorder || !info->bucket_off || !info->level || info->nlevs < 1) return false;
     if (!m->priv || info->n != m->nr || m->nr < 1 || m->nnz > kLwMaxEntries || !analysis_id(info)) return false;
-    const bool lane_rows = static_cast<const MatPriv*>(m->priv)->max_row <= kLwU + 1;
+    const int longest = static_cast<const MatPriv*>(m->priv)->max_row - 1;
+    if (longest > kLongRow) return false;
+    const bool lane_rows = longest <= kLwU;
     return (12.0 * m->nnz + 32.0 * m->nr) / info->nlevs <= (lane_rows ? kLwShortLevelBytes : kLwLevelBytes);
 }
 

@@ -155,3 +155,17 @@ def test_first_solve_beside_a_capture(mode):
     for st in streams:
         assert hip.hipStreamDestroy(st) == 0
     I.free_device_analysis(mat, info)
+
+
+@pytest.mark.parametrize("gen,param,walk", [(1, 64, True), (1, 250, True), (1, 600, False), (2, 2000, True),
+                                            (2, 8000, False), (3, 2000, False)])
+def test_walk_is_the_default_where_it_wins(gen, param, walk):
+    """The default shape of an ORDER solve on both sides of each line: levels
+    of the matrix of at most 16 KB with rows of up to 4 off-diagonals (2D grids
+    of 64^2 and 250^2, not of 600^2), 6 KB with longer ones (random), and no rows
+    of more than 64 (power law)."""
+    s = I.generate(gen, param)
+    mat = I.allocate_memory(s.ia, s.ja, s.a)
+    info = I.multirow_analysis_base_GPU(mat, I.ORDER)
+    assert (I.default_config(mat, info, I.PREC_F64, 1).variant == 4) == walk
+    I.free_device_analysis(mat, info)
