@@ -242,12 +242,15 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 // 2.47 ms, n = 3*10^4 109 against 129 us; 20 entries of the last 3000, n =
 // 3*10^5, 2.45 against 2.81 ms).
 constexpr long long kChainRows = 4;
+bool chain_of(const sp_mat_t* m, const dfr_analysis_info_t* info) {
+    return info && static_cast<const MatPriv*>(m->priv)->banded && m->nr < kChainRows * info->nlevs;
+}
 static sptrsv_config_t analysed_shape_for(const sp_mat_t* m, const dfr_analysis_info_t* info, int kernel, int k) {
     sptrsv_config_t c = shape_for(m, kernel, k);
     if (!m->priv) return c;  // a struct that no call has filled: nothing is known of its rows
     if (kernel == SPTRSV_KERNEL_SIMPLE && k == 1) simple_shape(m, &c);
     if ((kernel == SPTRSV_KERNEL_ORDER || kernel == SPTRSV_KERNEL_MULTIROW) && k == 1) {
-        if (priv_of(const_cast<sp_mat_t*>(m))->banded && info && m->nr < kChainRows * info->nlevs) c.variant = 5;
+        if (chain_of(m, info)) c.variant = 5;
         else if (level_plan_made(m, info)) c.variant = 4;
         else if (packed_waves(info).base) c.variant = 6;
         const int lanes = group_walk_lanes(m);

@@ -197,8 +197,8 @@ __global__ __launch_bounds__(64) void k_block_short(SolveArgs A) {
 // Columns at most 63 rows back: only the block before is outside, the rows are
 // taken in order, and both blocks' coefficients are dense in LDS (64 KB in FP64:
 // two waves per CU, 512 blocks ahead of the chain).  A step is a multiply by the
-// reciprocal diagonal, two readlanes and a multiply-add; rows are published
-// eight at a time.  A wave whose predecessor has published nothing yet sleeps
+// reciprocal diagonal, two readlanes, a multiply-add and an add; rows are
+// published eight at a time.  A wave whose predecessor has published nothing yet sleeps
 // between polls: 500 waves spinning made every hand-off slower (n = 50000 3.09
 // -> 2.04 ms).
 // blocks (of several matrices in one): first row and the matrix's end row of
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(64) void k_block_band(SolveArgs A, const int2* __re
         p = A.ia[row];
         dpos = A.ia[row + 1] - 1;
     }
-    Acc acc = live ? P::seed(A, (size_t)row) : P::zero();
+    const Acc seed = live ? P::seed(A, (size_t)row) : P::zero();
     typename P::Diag dg{};
     if (live) dg = P::diag(A, dpos);
     uint64_t bits[2] = {0, 0};  // columns of the two blocks this row depends on
@@ -264,6 +264,20 @@ __global__ __launch_bounds__(64) void k_block_band(SolveArgs A, const int2* __re
     int spins = 0;
     word prev = P::kUnsolved;
     constexpr uint64_t run = (1ull << kBlkRun) - 1;
+    // Four partial sums, by runs of kBlkRun columns, and the right-hand side added
+    // to them: in one accumulator that starts from it, entry after entry, the
+    // error grew with the bandwidth (1.5 times that of the lanes' tree of a row per
+    // wave at bandwidth 17, 2.6 at 63; 0.77 and 0.75 so; a longer step: n = 50000,
+    // bandwidth 17, 2.04 -> 2.14 ms).  Eight sums 2.27 ms and 0.69.  A row's only
+    // entry is folded into the right-hand side, as in that tree.
+    constexpr int kParts = LEVEL ? 1 : 4;
+    const uint64_t deps = bits[0] | bits[1];
+    const bool one = (deps & (deps - 1)) == 0;
+    Acc part[kParts];
+#pragma unroll
+    for (int h = 0; h < kParts; ++h)
+        part[h] = !LEVEL && one && ((deps >> (h * kBlkRun) | deps >> ((h + kParts) * kBlkRun)) & run) ? seed : P::zero();
+    const Acc base_sum = one && deps ? P::zero() : seed;
     auto fold = [&](const Acc& x, typename O::V c, word w, bool mine) {
         Acc f = x;
         P::fold(f, O::unpack(c), w);
@@ -290,11 +304,21 @@ __global__ __launch_bounds__(64) void k_block_band(SolveArgs A, const int2* __re
             }
         }
         const unsigned b8 = (unsigned)(bits[0] >> g);
+        Acc& own = part[g / kBlkRun % kParts];
 #pragma unroll
-        for (int s = 0; s < kBlkRun; ++s) acc = fold(acc, c[s], bcast(prev, g + s), (b8 >> s) & 1);
+        for (int s = 0; s < kBlkRun; ++s) own = fold(own, c[s], bcast(prev, g + s), (b8 >> s) & 1);
     }
 #pragma unroll
     for (int g = 0; g < kWave; g += kBlkRun) {
+        Acc& own = part[g / kBlkRun % kParts];
+        // (the group before's last, as the chain has just come from it)
+        Acc rest = base_sum;
+        if constexpr (!LEVEL) {
+            constexpr int k = kParts;
+            const int h = g / kBlkRun;
+            rest = P::add(P::add(rest, P::add(part[(h + 1) % k], part[(h + 2) % k])), part[(h + 3) % k]);
+        }
+        Acc t = LEVEL ? own : P::add(rest, own);
         if (chain & (run << g)) {
             typename O::V c[kBlkRun] = {};
             if constexpr (!LEVEL) {
@@ -303,14 +327,16 @@ __global__ __launch_bounds__(64) void k_block_band(SolveArgs A, const int2* __re
             }
             const unsigned b8 = (unsigned)(bits[1] >> g);
 #pragma unroll
-            for (int s = 0; s < kBlkRun; ++s)
-                acc = fold(acc, c[s], bcast(blk_word<P>(A, dg, acc), g + s), (b8 >> s) & 1);
+            for (int s = 0; s < kBlkRun; ++s) {
+                own = fold(own, c[s], bcast(blk_word<P>(A, dg, t), g + s), (b8 >> s) & 1);
+                t = LEVEL ? own : P::add(rest, own);
+            }
         }
         if (live && lane >= g && lane < g + kBlkRun) {
-            typename P::Out o{};
-            const word r = P::finish(A, dg, acc, o);
+            typename P::Out x{};
+            const word r = P::finish(A, dg, t, x);
             publish_global(&gpub[row], r);
-            P::emit(A, (size_t)row, o, r);
+            P::emit(A, (size_t)row, x, r);
         }
     }
 }

@@ -276,6 +276,8 @@ int install_row_shape(sp_mat_t* m, int longest);
 // it takes its rows in order (banded kernel).
 bool block_walk_fits(const sp_mat_t* m);
 bool block_walk_in_order(const sp_mat_t* m);
+// Banded with less than four rows per level: the block walk, analysed or not.
+bool chain_of(const sp_mat_t* m, const dfr_analysis_info_t* info);
 // Lanes per row of the group walk where that is the natural-order default, else 0.
 int group_walk_lanes(const sp_mat_t* m);
 // Rows per level below which a banded matrix is taken in order.

@@ -576,7 +576,7 @@ bool level_walk_fits(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     if (!info || !info->iorder || !info->inv_iorder || !info->bucket_off || !info->level || info->nlevs < 1) return false;
     if (!m->priv || info->n != m->nr || m->nr < 1 || m->nnz > kLwMaxEntries || !analysis_id(info)) return false;
     const int longest = static_cast<const MatPriv*>(m->priv)->max_row - 1;
-    if (longest > kLongRow) return false;
+    if (longest > kLongRow || chain_of(m, info)) return false;
     const bool lane_rows = longest <= kLwU;
     return (12.0 * m->nnz + 32.0 * m->nr) / info->nlevs <= (lane_rows ? kLwShortLevelBytes : kLwLevelBytes);
 }

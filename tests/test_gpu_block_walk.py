@@ -201,3 +201,28 @@ def test_batch_members_in_blocks(prec):
     bt.close()
     db.free()
     dx.free()
+
+
+@pytest.mark.parametrize("band", [1, 4, 17, 32, 63])
+@pytest.mark.parametrize("prec", [I.PREC_F64, I.PREC_F32])
+def test_banded_rounding_error(band, prec):
+    """The banded kernel's rounding error (2-norm, against extended precision) is
+    no larger than that of a row per wave, whose lanes' sums meet in a tree."""
+    ia, ja, a, b = matrix(4000, range(1, band + 1), seed=band)
+    if prec == I.PREC_F32:
+        a, b = a.astype(np.float32), b.astype(np.float32)
+    wide, ref = a.astype(np.longdouble), np.zeros(len(b), np.longdouble)
+    for i in range(len(b)):
+        s, d = ia[i], ia[i + 1] - 1
+        ref[i] = (b[i] - wide[s:d] @ ref[ja[s:d]]) / wide[d]
+    mat = (I.allocate_memory_f32 if prec == I.PREC_F32 else I.allocate_memory)(ia, ja, a)
+
+    def error(variant, lanes):
+        db, dx = I.DeviceArray.from_numpy(b), I.DeviceArray(len(b), a.dtype)
+        I.solve(mat, None, prec, db, dx, kernel=I.KERNEL_SIMPLE, lanes=lanes, wg=256, variant=variant)
+        e = dx.numpy() - ref
+        return float(np.sqrt((e @ e) / (ref @ ref)))
+
+    lanes = min(64, max(4, 1 << int(len(ja) // len(b) - 1).bit_length()))     # of a row per wave by default
+    assert error(5, 4) <= error(1, lanes)
+    I.free_device_analysis(mat, None)
