@@ -485,13 +485,15 @@ __global__ __launch_bounds__(WG) void k_level_walk(LwArgs A) {
     };
     auto lds_word = [&](unsigned byte) -> word { return *reinterpret_cast<word*>(reinterpret_cast<char*>(lds) + byte); };
     auto step = [&](int j2, int j) {
-        typename P::Acc acc = O::seed(bv[j]);  // 0 in lanes without a row
+        // a lane's entries after the first in a sum of their own (rounding error
+        // against a row per wave: 0.9, and 1.07 with all in one)
+        typename P::Acc acc = O::seed(bv[j]), rest = P::zero();  // 0 in lanes without a row
         word w[kLwU];
 #pragma unroll
         for (int u = 0; u < kLwU; ++u) w[u] = lds_word(O::at(rec[j][u]));
 #pragma unroll
-        for (int u = 0; u < kLwU; ++u) P::fold(acc, O::val(rec[j][u]), w[u]);
-        if constexpr (FAR) P::fold(acc, O::val(frec[j2]), lw_word(fword[j]));
+        for (int u = 0; u < kLwU; ++u) P::fold(u == 0 ? acc : rest, O::val(rec[j][u]), w[u]);
+        if constexpr (FAR) P::fold(rest, O::val(frec[j2]), lw_word(fword[j]));
         const unsigned z = (unsigned)__builtin_amdgcn_readfirstlane((int)row[j2].x);
         if (z & kLwOverflow) {  // entries beyond the lane's records
             const int at = A.over[slice_of(ent[j2])];
@@ -507,9 +509,10 @@ __global__ __launch_bounds__(WG) void k_level_walk(LwArgs A) {
                     g = lw_word(lw_load<O::V, 16>(r_pub, ((c & ~kLwFar) - 1u) * (unsigned)sizeof(word)));
                 else if (c)
                     g = lds[kLwRing0 + ((c - 1u) & (kLwRing - 1))];
-                P::fold(acc, O::val(r), g);
+                P::fold(rest, O::val(r), g);
             }
         }
+        acc = P::add(acc, rest);
         const int lg = (int)(z >> kLwIndexBits) & 7;
         if (lg) acc = group_reduce<P, 1>(acc, 1 << lg);
         Num xv;
