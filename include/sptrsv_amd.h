@@ -287,8 +287,8 @@ int csr_L_solve_multirow_f32(sp_mat_t* mat, dfr_analysis_info_t* info, const flo
  * the stream is captured before there is one, the lean path while a trace is
  * taken; 5 is the block walk (one right-hand side, natural order whatever the
  * kernel): 64 consecutive rows per wave, results of the block's own rows
- * exchanged in registers, for columns at most 63 rows back or rows of at most
- * 8 off-diagonals (other matrices, and a traced solve, take the lean path); 6
+ * exchanged in registers, for columns at most 63 rows back (none twice in a
+ * row) or rows of at most 8 off-diagonals (other matrices, and a traced solve, take the lean path); 6
  * is the packed walk (ORDER/MULTIROW, one right-hand side): a persistent walk
  * of the analysis's 64-lane layout, by the workgroups of one XCD where a level
  * has few rows, with a workgroup size and wave count of its own (a traced

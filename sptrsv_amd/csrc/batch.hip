@@ -561,7 +561,7 @@ int sptrsv_batch_create(int nmat, const int* n, const int* const* ia, const int*
     }
     bt->band.assign(nmat, 0);
     for (int m = 0; m < nmat; ++m)
-        bt->band[m] = n[m] > 0 && !shapes[m].wide && n[m] < kBandRows * shapes[m].levels;
+        bt->band[m] = n[m] > 0 && shapes[m].banded() && n[m] < kBandRows * shapes[m].levels;
     bt->lanes.resize(nmat);
     bt->avg.resize(nmat);
     bt->delta.resize(nmat);

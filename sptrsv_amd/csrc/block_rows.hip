@@ -251,11 +251,9 @@ __global__ __launch_bounds__(64) void k_block_band(SolveArgs A, const int2* __re
             const int j = c[u] - before;
             if (p + u < dpos && j >= 0 && c[u] < row) {
                 uint64_t& b = j < kWave ? bits[0] : bits[1];
-                const uint64_t bit = 1ull << (j & (kWave - 1));
+                const uint64_t bit = 1ull << (j & (kWave - 1));  // (no column comes twice in a row)
                 if constexpr (!LEVEL) {
-                    auto* at = &coef[j * kWave + lane];
-                    const typename O::V w = O::pack(v[u]);
-                    *at = (b & bit) ? *at + w : w;  // the same column twice: both
+                    coef[j * kWave + lane] = O::pack(v[u]);
                 }
                 b |= bit;
             }

@@ -141,7 +141,7 @@ struct MatPriv {
     double wall_rate_khz = 100000.0;
     int device = 0;
     int max_row = 0;             // longest row (entries incl. diagonal)
-    bool banded = false;         // no column more than 63 rows back
+    bool banded = false;         // no column more than 63 rows back, none twice in a row
     int band_levels = 0;         // banded: number of levels (0: not known)
     bool many_long = false;      // more than one row in 200 has over kLongRow off-diagonals
     double nearest = 0.0;        // mean distance of a row's last off-diagonal
@@ -256,15 +256,18 @@ constexpr int kNear = 8, kLongRow = 64;
 struct RowShape {
     int longest = 0;        // entries, with the diagonal
     bool wide = false;      // a column 64 or more rows back
+    bool twice = false;     // while !wide: a row with the same column twice
     int levels = 0;         // while !wide; 0: not counted
+    // for the banded kernel, which keeps one coefficient per column
+    bool banded() const { return !wide && !twice; }
     long long near = 0;     // rows whose last off-diagonal is at most kNear rows back
     long long long_rows = 0;  // rows of more than kLongRow off-diagonals
     long long dist = 0;     // sum of the rows' distances to their last off-diagonal
     // of the `seen` rows that near, long_rows and dist were counted over
     void install(MatPriv* pv, long long rows, long long seen) const {
         pv->max_row = longest;
-        pv->banded = !wide && rows > 0;
-        pv->band_levels = wide ? 0 : levels;
+        pv->banded = banded() && rows > 0;
+        pv->band_levels = banded() ? levels : 0;
         pv->near_rows = seen > 0 && 2 * near >= seen;
         pv->many_long = 200 * long_rows > seen;
         pv->nearest = seen > 0 ? (double)dist / (double)seen : 0.0;

@@ -149,7 +149,8 @@ void free_mat(sp_mat_t* m) {
     memset(m, 0, sizeof(*m));
 }
 
-// out[0]: a column 64 or more rows back; out[1]: rows whose last off-diagonal
+// out[0] bit 1: a column 64 or more rows back, 2: a row with a column twice (of
+// rows without such a one); out[1]: rows whose last off-diagonal
 // is at most kNear rows back; out[5]: rows of more than kLongRow off-diagonals;
 // dist: the sum of the distances.  A thread leaves a row at its first far column, so long rows of
 // wide matrices cost one load.
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256) void k_row_shape(const int* __restrict__ ia, c
         s_dist = 0;
     }
     __syncthreads();
-    int near = 0, wide = 0, longer = 0;
+    int near = 0, wide = 0, twice = 0, longer = 0;
     unsigned long long far = 0;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         const int lo = ia[i], hi = ia[i + 1] - 1;
@@ -172,15 +173,21 @@ __global__ __launch_bounds__(256) void k_row_shape(const int* __restrict__ ia, c
             far += d;
             longer += hi - lo > kLongRow;
         }
-        for (int p = lo; p < hi && !wide; ++p) wide = (int)i - ja[p] >= kWave;
+        unsigned long long seen = 0;  // distances
+        for (int p = lo; p < hi && !wide; ++p) {
+            const int d = (int)i - ja[p];
+            wide = d >= kWave;
+            twice |= !wide && ((seen >> d) & 1) ? 2 : 0;
+            if (!wide) seen |= 1ull << d;
+        }
     }
     if (near) atomicAdd(&s_near, near);
     if (far) atomicAdd(&s_dist, far);
     if (longer) atomicAdd(&s_long, longer);
-    if (wide) s_wide = 1;
+    if (wide | twice) atomicOr(&s_wide, wide | twice);
     __syncthreads();
     if (threadIdx.x == 0) {
-        if (s_wide) out[0] = 1;
+        if (s_wide) atomicOr(&out[0], s_wide);
         if (s_near) atomicAdd(&out[1], s_near);
         if (s_dist) atomicAdd(dist, s_dist);
         if (s_long) atomicAdd(&out[5], s_long);
@@ -197,7 +204,8 @@ int install_row_shape(sp_mat_t* m, int longest) {
                            m->ja, n, d, reinterpret_cast<unsigned long long*>(d + 2));
         SPT_HIP(hipGetLastError());
         SPT_HIP(hipMemcpy(h, d, sizeof(h), hipMemcpyDeviceToHost));
-        shape.wide = h[0] != 0;
+        shape.wide = (h[0] & 1) != 0;
+        shape.twice = (h[0] & 2) != 0;
         shape.near = h[1];
         shape.long_rows = h[5];
         memcpy(&shape.dist, h + 2, sizeof(shape.dist));
@@ -215,7 +223,8 @@ static int validate_host_csr(const int* ia, const int* ja, int n, RowShape* shap
     const int base = ia[0];
     if (base < 0) return fail(SPTRSV_E_INVALID_CSR, "negative row pointer");
     ja += base;  // rows index ja relative to ia[0]
-    int lev[kWave] = {};  // levels of the last 64 rows, while they are all that is needed
+    int lev[kWave] = {};   // levels of the last 64 rows, while they are all that is needed
+    int seen[kWave] = {};  // row + 1 that last had a column, likewise
     for (int i = 0; i < n; ++i) {
         int level = 1;
         long long s = (long long)ia[i] - base, e = (long long)ia[i + 1] - base;
@@ -230,7 +239,11 @@ static int validate_host_csr(const int* ia, const int* ja, int n, RowShape* shap
                                                       std::to_string(ja[p]) +
                                                       " outside the strict lower triangle");
             shape->wide |= i - ja[p] >= kWave;
-            if (!shape->wide) level = std::max(level, lev[ja[p] % kWave] + 1);
+            if (shape->wide) continue;
+            level = std::max(level, lev[ja[p] % kWave] + 1);
+            int& s = seen[ja[p] % kWave];
+            shape->twice |= s == i + 1;
+            s = i + 1;
         }
         lev[i % kWave] = level;
         shape->levels = std::max(shape->levels, level);
@@ -332,6 +345,7 @@ int upload_concat(const int* n, const int* const* ia, const int* const* ja, cons
         shapes->push_back(own);
         shape.longest = std::max(shape.longest, own.longest);
         shape.wide |= own.wide;
+        shape.twice |= own.twice;
         shape.levels = std::max(shape.levels, own.levels);
         shape.near += own.near;
         shape.long_rows += own.long_rows;

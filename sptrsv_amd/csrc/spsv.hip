@@ -35,18 +35,20 @@ unsigned row_grid(long long count) {
 // Stored-row lengths: kept off-diagonals + 1 (the diagonal) at the stored
 // row (i, or n-1-i for an upper triangle); dpos[i] = the diagonal entry used
 // (-1 for a unit diagonal); out[0] bit 1 = column outside [0, n), bit 2 = a
-// missing diagonal; out[1] = a kept column 64 or more rows away; out[2] of the
+// missing diagonal; out[1] bit 1 = a kept column 64 or more rows
+// away, 2 = one kept twice in a row; out[2] of the
 // out[3] rows of every eighth workgroup have their last kept one within kNear,
 // and out[4..5] is the sum of their distances to it.
 __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, const int* __restrict__ ja, int n,
                                                    int upper, int unit, int* __restrict__ len, int* __restrict__ dpos,
                                                    int* __restrict__ out) {
-    int wide = 0, near = 0, rows = 0;
+    int wide = 0, twice = 0, near = 0, rows = 0;
     unsigned long long dist = 0;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
          t += (long long)gridDim.x * blockDim.x) {
         const int i = (int)t;
         int kept = 0, d = -1, flags = 0, last = 0;
+        unsigned long long seen = 0;  // distances
         for (int p = ia[i]; p < ia[i + 1]; ++p) {
             const int j = ja[p];
             if (j < 0 || j >= n) flags |= 1;
@@ -54,7 +56,12 @@ __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, c
             else if (upper ? j > i : j < i) {
                 ++kept;
                 last = abs(i - j);
-                wide |= last >= kWave;
+                if (last >= kWave) {
+                    wide = 1;
+                } else {
+                    twice |= (seen >> last) & 1 ? 2 : 0;
+                    seen |= 1ull << last;
+                }
             }
         }
         if (!unit && d < 0) flags |= 2;
@@ -65,7 +72,7 @@ __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, c
         dist += last;
         ++rows;
     }
-    if (wide) out[1] = 1;
+    if ((wide | twice) && (out[1] | wide | twice) != out[1]) atomicOr(&out[1], wide | twice);
     if ((blockIdx.x & 7) == 0) {
         __shared__ int s_near, s_rows;
         __shared__ unsigned long long s_dist;
@@ -177,7 +184,8 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
         shape.longest = h_out[6];
         // of all rows, so scaled to the ones seen
         shape.long_rows = n > 0 ? (long long)h_out[7] * h_out[3] / n : 0;
-        shape.wide = h_out[1] != 0;
+        shape.wide = (h_out[1] & 1) != 0;
+        shape.twice = (h_out[1] & 2) != 0;
         shape.near = h_out[2];
         memcpy(&shape.dist, h_out + 4, sizeof(shape.dist));
         shape.install(priv_of(m), n, h_out[3]);

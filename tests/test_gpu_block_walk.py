@@ -226,3 +226,46 @@ def test_banded_rounding_error(band, prec):
     lanes = min(64, max(4, 1 << int(len(ja) // len(b) - 1).bit_length()))     # of a row per wave by default
     assert error(5, 4) <= error(1, lanes)
     I.free_device_analysis(mat, None)
+
+
+@pytest.mark.parametrize("prec,big", [(I.PREC_F64, 1.5e308), (I.PREC_F32, 3.0e38)])
+def test_a_column_twice_keeps_both_products(prec, big):
+    """The entries of a column that a row holds twice are multiplied each by the
+    solution, whose product fits where the entries' sum does not; eager on
+    every kind of handle, and as a batch member."""
+    n = 200
+    ia = np.zeros(n + 1, np.int32)
+    ja, a = [], []
+    for i in range(n):
+        if i % 2:
+            ja += [i - 1, i - 1, i]
+            a += [big, big, 1.0]
+        else:
+            ja += [i - 1, i] if i else [i]          # (a chain, whose rows are taken in order)
+            a += [0.0, 1.0] if i else [1.0]
+        ia[i + 1] = len(ja)
+    ja, a = np.array(ja, np.int32), np.array(a)
+    b = np.where(np.arange(n) % 2 == 0, 1.0 / big, 3.0)
+    if prec == I.PREC_F32:
+        a, b = a.astype(np.float32), b.astype(np.float32)
+    want = np.where(np.arange(n) % 2 == 0, b, 1.0)
+    mats = [(I.allocate_memory_f32 if prec == I.PREC_F32 else I.allocate_memory)(ia, ja, a)]
+    spsv = None
+    if prec == I.PREC_F64:
+        spsv = I.Spsv(n, *(I.DeviceArray.from_numpy(v) for v in (ia, ja, a)))
+        mats.append(spsv.matrix())
+    db, dx = I.DeviceArray.from_numpy(b), I.DeviceArray(n, a.dtype)
+    for mat in mats:
+        for variant, lanes in ((0, 0), (5, 4)):
+            I.solve(mat, None, prec, db, dx, kernel=I.KERNEL_SIMPLE, lanes=lanes, wg=256, variant=variant)
+            assert relerr(dx.numpy(), want) <= 1e-6
+    I.free_device_analysis(mats[0], None)
+    if prec == I.PREC_F64:
+        spsv.close()
+        bt = I.Batch([I.System(n, ia, ja, a, b), I.System(n, ia, ja, a, b)])
+        bt.tune(prec, tune=False)
+        db, dx = I.DeviceArray.from_numpy(np.tile(b, 2)), I.DeviceArray(2 * n, np.float64)
+        bt.solve(prec, db, dx)
+        I.synchronize()
+        assert relerr(dx.numpy(), np.tile(want, 2)) <= 1e-12
+        bt.close()
