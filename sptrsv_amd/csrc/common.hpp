@@ -144,7 +144,7 @@ struct MatPriv {
     bool banded = false;         // no column more than 63 rows back, none twice in a row
     int band_levels = 0;         // banded: number of levels (0: not known)
     bool many_long = false;      // more than one row in 200 has over kLongRow off-diagonals
-    double nearest = 0.0;        // mean distance of a row's last off-diagonal
+    double nearest = 0.0;        // mean distance of a row's nearest off-diagonal
     bool near_rows = false;      // at least half of the rows depend on one of the kNear rows before them
     long long* trace = nullptr;  // per-row timeline (profiling), 3*n*k
     size_t trace_len = 0;
@@ -260,9 +260,9 @@ struct RowShape {
     int levels = 0;         // while !wide; 0: not counted
     // for the banded kernel, which keeps one coefficient per column
     bool banded() const { return !wide && !twice; }
-    long long near = 0;     // rows whose last off-diagonal is at most kNear rows back
+    long long near = 0;     // rows whose nearest off-diagonal is at most kNear rows back
     long long long_rows = 0;  // rows of more than kLongRow off-diagonals
-    long long dist = 0;     // sum of the rows' distances to their last off-diagonal
+    long long dist = 0;     // sum of the rows' distances to their nearest off-diagonal
     // of the `seen` rows that near, long_rows and dist were counted over
     void install(MatPriv* pv, long long rows, long long seen) const {
         pv->max_row = longest;

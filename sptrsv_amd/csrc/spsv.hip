@@ -37,8 +37,9 @@ unsigned row_grid(long long count) {
 // (-1 for a unit diagonal); out[0] bit 1 = column outside [0, n), bit 2 = a
 // missing diagonal; out[1] bit 1 = a kept column 64 or more rows
 // away, 2 = one kept twice in a row; out[2] of the
-// out[3] rows of every eighth workgroup have their last kept one within kNear,
-// and out[4..5] is the sum of their distances to it.
+// out[3] rows of every eighth workgroup have their nearest kept one within kNear,
+// and out[4..5] is the sum of their distances to it (in an upper triangle whose
+// columns ascend that is the first one).
 __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, const int* __restrict__ ja, int n,
                                                    int upper, int unit, int* __restrict__ len, int* __restrict__ dpos,
                                                    int* __restrict__ out) {
@@ -47,20 +48,21 @@ __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, c
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
          t += (long long)gridDim.x * blockDim.x) {
         const int i = (int)t;
-        int kept = 0, d = -1, flags = 0, last = 0;
+        int kept = 0, d = -1, flags = 0, nearest = 0;
         unsigned long long seen = 0;  // distances
         for (int p = ia[i]; p < ia[i + 1]; ++p) {
             const int j = ja[p];
             if (j < 0 || j >= n) flags |= 1;
             else if (j == i) { if (d < 0) d = p; }
             else if (upper ? j > i : j < i) {
+                const int away = abs(i - j);
+                nearest = kept ? min(nearest, away) : away;
                 ++kept;
-                last = abs(i - j);
-                if (last >= kWave) {
+                if (away >= kWave) {
                     wide = 1;
                 } else {
-                    twice |= (seen >> last) & 1 ? 2 : 0;
-                    seen |= 1ull << last;
+                    twice |= (seen >> away) & 1 ? 2 : 0;
+                    seen |= 1ull << away;
                 }
             }
         }
@@ -68,8 +70,8 @@ __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, c
         if (flags) atomicOr(out, flags);
         len[upper ? n - 1 - i : i] = kept + 1;
         dpos[i] = unit ? -1 : d;
-        near += kept > 0 && last <= kNear;
-        dist += last;
+        near += kept > 0 && nearest <= kNear;
+        dist += nearest;
         ++rows;
     }
     if ((wide | twice) && (out[1] | wide | twice) != out[1]) atomicOr(&out[1], wide | twice);
