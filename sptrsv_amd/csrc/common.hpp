@@ -114,7 +114,7 @@ constexpr int kCounterWords = 16;
 
 struct MatPriv {
     void* block = nullptr;       // holds ia, ja, a, a32 and src_perm of a handle made on the device
-    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4] to [7], [9] row shape, [8] XCD of a walk, [10], [11] analysis, [12] batch (device)
+    int* counters = nullptr;     // [0] ticket, [1] watchdog word, [4] to [7], [9], [13] row shape, [8] XCD of a walk, [10], [11] analysis, [12] batch (device)
     uint64_t* pub = nullptr;     // published words, n*k 64-bit (device)
     size_t pub_words = 0;
     uint64_t* part = nullptr;    // published partial sums of long-row segments, 2 per segment (device)
@@ -144,7 +144,7 @@ struct MatPriv {
     bool banded = false;         // no column more than 63 rows back, none twice in a row
     int band_levels = 0;         // banded: number of levels (0: not known)
     bool many_long = false;      // more than one row in 200 has over kLongRow off-diagonals
-    double nearest = 0.0;        // mean distance of a row's nearest off-diagonal
+    double nearest = 0.0;        // mean distance of the nearest off-diagonal, of the rows that have one
     bool near_rows = false;      // at least half of the rows depend on one of the kNear rows before them
     long long* trace = nullptr;  // per-row timeline (profiling), 3*n*k
     size_t trace_len = 0;
@@ -253,6 +253,7 @@ int level_analysis(dfr_analysis_info_t** info, sp_mat_t* m, MODE mode, bool plan
 void analysis_freed(unsigned long long id);
 // What the rows of a matrix look like, for the choice of a walk.
 constexpr int kNear = 8, kLongRow = 64;
+constexpr double kNoneNear = 1e30;  // nearest off-diagonal where no row has one
 struct RowShape {
     int longest = 0;        // entries, with the diagonal
     bool wide = false;      // a column 64 or more rows back
@@ -262,15 +263,16 @@ struct RowShape {
     bool banded() const { return !wide && !twice; }
     long long near = 0;     // rows whose nearest off-diagonal is at most kNear rows back
     long long long_rows = 0;  // rows of more than kLongRow off-diagonals
-    long long dist = 0;     // sum of the rows' distances to their nearest off-diagonal
-    // of the `seen` rows that near, long_rows and dist were counted over
+    long long waiting = 0;  // rows with an off-diagonal
+    long long dist = 0;     // sum of their distances to the nearest
+    // of the `seen` rows that near, long_rows, waiting and dist were counted over
     void install(MatPriv* pv, long long rows, long long seen) const {
         pv->max_row = longest;
         pv->banded = banded() && rows > 0;
         pv->band_levels = banded() ? levels : 0;
         pv->near_rows = seen > 0 && 2 * near >= seen;
         pv->many_long = 200 * long_rows > seen;
-        pv->nearest = seen > 0 ? (double)dist / (double)seen : 0.0;
+        pv->nearest = waiting > 0 ? (double)dist / (double)waiting : kNoneNear;
     }
 };
 // The same of a matrix made on the device (its longest row given; waits).

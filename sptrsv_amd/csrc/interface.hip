@@ -151,21 +151,21 @@ void free_mat(sp_mat_t* m) {
 
 // out[0] bit 1: a column 64 or more rows back, 2: a row with a column twice
 // (counted where bit 1 is not set); out[1]: rows whose nearest off-diagonal is at
-// most kNear rows back; out[5]: rows of more than kLongRow off-diagonals; dist:
-// the sum of the distances.  Columns may come in any order, so all are read,
+// most kNear rows back; out[5]: rows of more than kLongRow off-diagonals; out[9]:
+// rows with an off-diagonal; dist: the sum of their distances.  Columns may come in any order, so all are read,
 // eight lanes a row; few workgroups, large ones, as each adds to the same words
 // (2D grid 250^2 from coordinates: 573 -> 510 us from 2048 workgroups of 256 threads).
 constexpr int kShapeLanes = 8, kShapeThreads = 1024;
 __global__ __launch_bounds__(kShapeThreads) void k_row_shape(const int* __restrict__ ia, const int* __restrict__ ja, int n,
                                                    int* __restrict__ out, unsigned long long* __restrict__ dist) {
-    __shared__ int s_near, s_flags, s_long;
+    __shared__ int s_near, s_flags, s_long, s_waiting;
     __shared__ unsigned long long s_dist;
     if (threadIdx.x == 0) {
-        s_near = s_flags = s_long = 0;
+        s_near = s_flags = s_long = s_waiting = 0;
         s_dist = 0;
     }
     __syncthreads();
-    int near = 0, flags = 0, longer = 0;
+    int near = 0, flags = 0, longer = 0, waiting = 0;
     unsigned long long far = 0;
     const int e = threadIdx.x % kShapeLanes;
     const long long rows = (long long)gridDim.x * blockDim.x / kShapeLanes;
@@ -193,6 +193,7 @@ __global__ __launch_bounds__(kShapeThreads) void k_row_shape(const int* __restri
         if (e == 0 && lo < hi) {
             near += least <= kNear;
             far += least;
+            ++waiting;
             longer += hi - lo > kLongRow;
         }
     }
@@ -200,12 +201,14 @@ __global__ __launch_bounds__(kShapeThreads) void k_row_shape(const int* __restri
     if (far) atomicAdd(&s_dist, far);
     if (longer) atomicAdd(&s_long, longer);
     if (flags) atomicOr(&s_flags, flags);
+    if (waiting) atomicAdd(&s_waiting, waiting);
     __syncthreads();
     if (threadIdx.x == 0) {
         if (s_flags) atomicOr(&out[0], s_flags);
         if (s_near) atomicAdd(&out[1], s_near);
         if (s_dist) atomicAdd(dist, s_dist);
         if (s_long) atomicAdd(&out[5], s_long);
+        if (s_waiting) atomicAdd(&out[9], s_waiting);
     }
 }
 
@@ -214,7 +217,7 @@ int install_row_shape(sp_mat_t* m, int longest) {
     shape.longest = longest;
     const int n = m->nr;
     if (n > 0) {
-        int h[6] = {}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
+        int h[10] = {}, *d = priv_of(m)->counters + 4;  // zero since the handle was made
         hipLaunchKernelGGL(k_row_shape, dim3(std::min<unsigned>(ceil_div((long long)n * kShapeLanes, kShapeThreads), 256)), dim3(kShapeThreads), 0, nullptr, m->ia,
                            m->ja, n, d, reinterpret_cast<unsigned long long*>(d + 2));
         SPT_HIP(hipGetLastError());
@@ -223,6 +226,7 @@ int install_row_shape(sp_mat_t* m, int longest) {
         shape.twice = (h[0] & 2) != 0;
         shape.near = h[1];
         shape.long_rows = h[5];
+        shape.waiting = h[9];
         memcpy(&shape.dist, h + 2, sizeof(shape.dist));
     }
     shape.install(priv_of(m), n, n);
@@ -266,6 +270,7 @@ static int validate_host_csr(const int* ia, const int* ja, int n, RowShape* shap
         if (e - s > 1) {
             shape->near += i - nearest <= kNear;
             shape->dist += i - nearest;
+            ++shape->waiting;
         }
         shape->longest = std::max<int>(shape->longest, (int)(e - s));
         shape->long_rows += e - s > kLongRow + 1;
@@ -366,6 +371,7 @@ int upload_concat(const int* n, const int* const* ia, const int* const* ja, cons
         shape.near += own.near;
         shape.long_rows += own.long_rows;
         shape.dist += own.dist;
+        shape.waiting += own.waiting;
         row_off[q + 1] = row_off[q] + n[q];
         nnz_off[q + 1] = nnz_off[q] + (n[q] > 0 ? (long long)ia[q][n[q]] - ia[q][0] : 0);
     }

@@ -38,12 +38,12 @@ unsigned row_grid(long long count) {
 // missing diagonal; out[1] bit 1 = a kept column 64 or more rows
 // away, 2 = one kept twice in a row; out[2] of the
 // out[3] rows of every eighth workgroup have their nearest kept one within kNear,
-// and out[4..5] is the sum of their distances to it (in an upper triangle whose
-// columns ascend that is the first one).
+// and out[4..5] is the sum of the distances to it of the out[8] rows that have
+// one (in an upper triangle whose columns ascend it is the first one).
 __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, const int* __restrict__ ja, int n,
                                                    int upper, int unit, int* __restrict__ len, int* __restrict__ dpos,
                                                    int* __restrict__ out) {
-    int wide = 0, twice = 0, near = 0, rows = 0;
+    int wide = 0, twice = 0, near = 0, rows = 0, waiting = 0;
     unsigned long long dist = 0;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
          t += (long long)gridDim.x * blockDim.x) {
@@ -72,24 +72,27 @@ __global__ __launch_bounds__(256) void k_tri_count(const int* __restrict__ ia, c
         dpos[i] = unit ? -1 : d;
         near += kept > 0 && nearest <= kNear;
         dist += nearest;
+        waiting += kept > 0;
         ++rows;
     }
     if ((wide | twice) && (out[1] | wide | twice) != out[1]) atomicOr(&out[1], wide | twice);
     if ((blockIdx.x & 7) == 0) {
-        __shared__ int s_near, s_rows;
+        __shared__ int s_near, s_rows, s_waiting;
         __shared__ unsigned long long s_dist;
         if (threadIdx.x == 0) {
-            s_near = s_rows = 0;
+            s_near = s_rows = s_waiting = 0;
             s_dist = 0;
         }
         __syncthreads();
         if (near) atomicAdd(&s_near, near);
         atomicAdd(&s_rows, rows);
+        if (waiting) atomicAdd(&s_waiting, waiting);
         atomicAdd(&s_dist, dist);
         __syncthreads();
         if (threadIdx.x == 0) {
             atomicAdd(&out[2], s_near);
             atomicAdd(&out[3], s_rows);
+            atomicAdd(&out[8], s_waiting);
             atomicAdd(reinterpret_cast<unsigned long long*>(out + 4), s_dist);
         }
     }
@@ -141,13 +144,13 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     Arena work;
     work.add(&len, (size_t)n + 1);
     work.add(&dpos, n);
-    work.add(&bad, 8);
+    work.add(&bad, 9);
     work.add(&ia_s, (size_t)n + 1);
     work.add(&scratch, scan_scratch((long long)n + 1));
     void* tmp = nullptr;
     chk(work.get(&tmp), "hipMalloc triangle work");
     if (st == SPTRSV_OK) chk(hipMemset(len, 0, 4 * ((size_t)n + 1)), "clear lengths");
-    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 32), "clear flag");
+    if (st == SPTRSV_OK) chk(hipMemset(bad, 0, 36), "clear flag");
     if (st == SPTRSV_OK && n > 0) {
         hipLaunchKernelGGL(k_tri_count, dim3(row_grid(n)), dim3(256), 0, nullptr, ia, ja, n, upper ? 1 : 0,
                            unit ? 1 : 0, len, dpos, bad);
@@ -157,9 +160,9 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
     // wait for all
     if (st == SPTRSV_OK) st = exclusive_scan(len, ia_s, (long long)n + 1, nullptr, scratch);
     if (st == SPTRSV_OK && n > 0) st = longest_row(ia_s, n, bad + 6, nullptr);
-    int h_out[8] = {};
+    int h_out[9] = {};
     int total = 0;
-    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 32, hipMemcpyDeviceToHost), "read flag");
+    if (st == SPTRSV_OK) chk(hipMemcpy(h_out, bad, 36, hipMemcpyDeviceToHost), "read flag");
     const int h_bad = h_out[0];
     if (st == SPTRSV_OK && (h_bad & 1)) st = fail(SPTRSV_E_INVALID_CSR, "column index outside [0, n)");
     if (st == SPTRSV_OK && (h_bad & 2)) st = fail(SPTRSV_E_INVALID_CSR, "a row has no diagonal entry (non-unit diagonal)");
@@ -189,6 +192,7 @@ int build_triangle(int n, int nnz, const int* ia, const int* ja, const double* a
         shape.wide = (h_out[1] & 1) != 0;
         shape.twice = (h_out[1] & 2) != 0;
         shape.near = h_out[2];
+        shape.waiting = h_out[8];
         memcpy(&shape.dist, h_out + 4, sizeof(shape.dist));
         shape.install(priv_of(m), n, h_out[3]);
     }

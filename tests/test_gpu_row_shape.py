@@ -109,3 +109,29 @@ def test_order_of_columns_does_not_matter(name):
     h.close()
     for m in [low, mixed] + coo:
         I.free_device_analysis(m, None)
+
+
+def test_rows_without_dependencies_have_no_distance():
+    """Rows that wait for nothing do not bring the others' dependencies nearer:
+    one of five waiting rows and all of them get the same walk."""
+    n, reach = 60000, 20000
+    rng = np.random.default_rng(7)
+
+    def some(share):
+        ia, ja = [0], []
+        for i in range(n):
+            ja += [max(0, i - int(rng.integers(100, reach))), i] if i and rng.random() < share else [i]
+            ia.append(len(ja))
+        ia, ja = np.array(ia, np.int32), np.array(ja, np.int32)
+        return ia, ja, np.where(np.arange(len(ja)) == np.repeat(ia[1:] - 1, np.diff(ia)), 1.0, -0.5)
+
+    dense, sparse = some(1.0), some(0.2)
+    mats = [I.allocate_memory(*dense), I.allocate_memory(*sparse)]
+    h = I.Spsv(n, *device(*sparse))
+    rows = np.repeat(np.arange(n), np.diff(sparse[0])).astype(np.int32)
+    mats.append(I.coo_to_lower(rows, sparse[1], sparse[2], n, False, unit=False))
+    variants = [shapes(m)[1] for m in mats] + [shapes(h.matrix())[1]]
+    assert variants == variants[:1] * 4
+    h.close()
+    for m in mats:
+        I.free_device_analysis(m, None)
