@@ -155,10 +155,21 @@ static sptrsv_config_t shape_for(const sp_mat_t* m, int kernel, int k) {
 // Rows are taken in order (banded kernel) unless a level has 16 rows or more
 // and they are short (2D grid of 50^2: 81 us against 118).
 constexpr long long kWideRows = 1024;
+// Levels of a banded matrix.  They are counted on the host, and by an analysis;
+// of a matrix made on the device, before that, where most rows wait for another,
+// a chain through every row's nearest dependency gives about as many (0: not
+// known).
+static int levels_of_band(const sp_mat_t* m) {
+    const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
+    if (pv->band_levels > 0) return pv->band_levels;
+    if (pv->nearest >= kNoneNear) return 1;
+    return pv->most_wait ? std::max(1, (int)(m->nr / std::max(pv->nearest, 1.0))) : 0;
+}
 bool block_walk_in_order(const sp_mat_t* m) {
     const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
     if (!pv->banded) return false;
-    const bool parallel = pv->band_levels > 0 && m->nr >= kBandRows * pv->band_levels;
+    const int levels = levels_of_band(m);
+    const bool parallel = levels > 0 && m->nr >= kBandRows * levels;
     return !parallel || pv->max_row > kBlockRow + 1;
 }
 
@@ -166,7 +177,9 @@ bool block_walk_fits(const sp_mat_t* m) {
     const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
     // (3D grid 10^3: 34.6 us against 30.0, 14^3: 45.5 against 50.3)
     if (!pv->banded) return pv->near_rows && pv->max_row <= kBlockRow + 1 && m->nr >= 2500;
-    return pv->near_rows || m->nr < kBandRows * std::max(pv->band_levels, 1) || m->nr >= kWideRows * pv->band_levels;
+    const int levels = levels_of_band(m);
+    if (pv->near_rows || !levels) return pv->near_rows;
+    return m->nr < kBandRows * levels || m->nr >= kWideRows * levels;
 }
 
 // Natural order, one right-hand side.

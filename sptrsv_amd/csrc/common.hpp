@@ -142,7 +142,8 @@ struct MatPriv {
     int device = 0;
     int max_row = 0;             // longest row (entries incl. diagonal)
     bool banded = false;         // no column more than 63 rows back, none twice in a row
-    int band_levels = 0;         // banded: number of levels (0: not known)
+    int band_levels = 0;         // banded: number of levels (0: not counted)
+    bool most_wait = false;      // at least half of the rows have an off-diagonal
     bool many_long = false;      // more than one row in 200 has over kLongRow off-diagonals
     double nearest = 0.0;        // mean distance of the nearest off-diagonal, of the rows that have one
     bool near_rows = false;      // at least half of the rows depend on one of the kNear rows before them
@@ -272,6 +273,7 @@ struct RowShape {
         pv->band_levels = banded() ? levels : 0;
         pv->near_rows = seen > 0 && 2 * near >= seen;
         pv->many_long = 200 * long_rows > seen;
+        pv->most_wait = 2 * waiting >= seen;
         pv->nearest = waiting > 0 ? (double)dist / (double)waiting : kNoneNear;
     }
 };

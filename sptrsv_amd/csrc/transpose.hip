@@ -134,6 +134,7 @@ int sptrsv_transpose(sp_mat_t* src, sp_mat_t* dst) {
         // distances and levels are those of the source; near rows as there
         dp->banded = from->banded;
         dp->band_levels = from->band_levels;
+        dp->most_wait = from->most_wait;
         dp->near_rows = from->near_rows;
         dp->nearest = from->nearest;
     }

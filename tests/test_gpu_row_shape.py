@@ -135,3 +135,34 @@ def test_rows_without_dependencies_have_no_distance():
     h.close()
     for m in mats:
         I.free_device_analysis(m, None)
+
+
+def band(n, offsets):
+    ia, ja = [0], []
+    for i in range(n):
+        ja += [i - o for o in sorted(offsets, reverse=True) if o <= i] + [i]
+        ia.append(len(ja))
+    ia, ja = np.array(ia, np.int32), np.array(ja, np.int32)
+    return ia, ja, np.where(np.arange(len(ja)) == np.repeat(ia[1:] - 1, np.diff(ia)), 1.0, -0.1)
+
+
+@pytest.mark.parametrize("offsets", [[32], [17, 40, 63], [10], [1, 2, 17], [], [40]])
+@pytest.mark.parametrize("n", [900, 4000])
+def test_banded_handles_made_on_the_device(offsets, n):
+    """A banded matrix gets the walk that the host's count of its levels gives it
+    when it is made on the device, where they are not counted (only the row 32
+    before, n = 4000: 178 us with the block walk, 112 without)."""
+    ia, ja, a = band(n, offsets)
+    low = I.allocate_memory(ia, ja, a)
+    h = I.Spsv(n, *device(ia, ja, a))
+    rows = np.repeat(np.arange(n), np.diff(ia)).astype(np.int32)
+    coo = I.coo_to_lower(rows, ja, a, n, False, unit=False)
+    assert shapes(h.matrix()) == shapes(low) and shapes(coo) == shapes(low)
+    b = np.random.default_rng(2).uniform(-1.0, 1.0, n)
+    db, dx = device(b, b)
+    for m in (low, coo, h.matrix()):
+        I.csr_L_solve_simple(m, db, dx)
+        assert relerr(dx.numpy(), O.fwd_f64(ia, ja, a, b)) <= 1e-12
+    h.close()
+    I.free_device_analysis(low, None)
+    I.free_device_analysis(coo, None)
