@@ -144,7 +144,7 @@ struct sptrsv_batch {
     hipStream_t aux = nullptr;           // Jacobi half of a MIXED solve
     bool serial = false;                 // MIXED: Jacobi half, then the sync-free half, on one stream
     std::vector<long long> ent_off;      // nmat+1: first entry of each matrix
-    std::vector<int> max_row;            // per matrix: longest row
+    std::vector<RowShape> shape;         // per matrix: what its rows look like
     std::vector<double> chain;           // per matrix: fraction of rows i > 0 that depend on row i - 1
     std::vector<int> pattern;            // per matrix: first matrix with the same structure (n, ia, ja)
     int n_patterns = 0;
@@ -465,19 +465,19 @@ int build_sub(sptrsv_batch_t* bt) {
     free_sub(bt);
     const int nmat = (int)bt->choice.size();
     long long rows = 0, nz = 0;
-    int mr = 0;
+    RowShape shape;
     for (int m = 0; m < nmat; ++m) {
         if (bt->choice[m] == SPTRSV_KERNEL_JACOBI) continue;
         rows += bt->row_off[m + 1] - bt->row_off[m];
         nz += bt->ent_off[m + 1] - bt->ent_off[m];
-        mr = std::max(mr, bt->max_row[m]);
+        shape.add(bt->shape[m]);
     }
     if (rows == 0) return SPTRSV_OK;
     sp_mat_t& S = bt->sub;
     SPT_TRY(ensure_priv(&S));
     S.nr = S.nc = (int)rows;
     S.nnz = (int)nz;
-    priv_of(&S)->max_row = mr;
+    shape.install(priv_of(&S), rows, rows);
     int st = SPTRSV_OK;
     auto chk = [&](hipError_t e, const char* what) {
         if (e != hipSuccess && st == SPTRSV_OK) st = hip_fail(e, what, __FILE__, __LINE__);
@@ -551,8 +551,7 @@ int sptrsv_batch_create(int nmat, const int* n, const int* const* ia, const int*
         std::lock_guard<std::mutex> g(g_batch_mu);
         g_batches.insert(bt);
     }
-    std::vector<RowShape> shapes;
-    int st = upload_concat(n, ia, ja, a, nmat, &bt->mat, bt->row_off, &shapes);
+    int st = upload_concat(n, ia, ja, a, nmat, &bt->mat, bt->row_off, &bt->shape);
     if (st != SPTRSV_OK) {
         std::lock_guard<std::mutex> g(g_batch_mu);
         g_batches.erase(bt);
@@ -561,7 +560,7 @@ int sptrsv_batch_create(int nmat, const int* n, const int* const* ia, const int*
     }
     bt->band.assign(nmat, 0);
     for (int m = 0; m < nmat; ++m)
-        bt->band[m] = n[m] > 0 && shapes[m].banded() && n[m] < kBandRows * shapes[m].levels;
+        bt->band[m] = n[m] > 0 && bt->shape[m].banded() && n[m] < kBandRows * bt->shape[m].levels;
     bt->lanes.resize(nmat);
     bt->avg.resize(nmat);
     bt->delta.resize(nmat);
@@ -570,14 +569,12 @@ int sptrsv_batch_create(int nmat, const int* n, const int* const* ia, const int*
     bt->choice.assign(nmat, SPTRSV_KERNEL_SIMPLE);
     bt->t_sync.assign(nmat, 0.0f);
     bt->ent_off.assign(nmat + 1, 0);
-    bt->max_row.assign(nmat, 0);
     bt->chain.assign(nmat, 0.0);
     long long entry_base = 0;
     for (int m = 0; m < nmat; ++m) {
         long long rows = bt->row_off[m + 1] - bt->row_off[m];
         long long nz = rows > 0 ? (long long)ia[m][n[m]] - ia[m][0] : 0;
         bt->ent_off[m] = entry_base;
-        for (int i = 0; i < n[m]; ++i) bt->max_row[m] = std::max(bt->max_row[m], ia[m][i + 1] - ia[m][i]);
         bt->avg[m] = rows > 0 ? (int)(nz / rows) : 0;
         bt->lanes[m] = lanes_rule(bt->avg[m]);
         double dm = rows > 0 ? 1e300 : 1.0;

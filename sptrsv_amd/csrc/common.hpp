@@ -267,6 +267,17 @@ struct RowShape {
     long long waiting = 0;  // rows with an off-diagonal
     long long dist = 0;     // sum of their distances to the nearest
     // of the `seen` rows that near, long_rows, waiting and dist were counted over
+    // the same of a matrix followed by another, on the diagonal
+    void add(const RowShape& o) {
+        longest = std::max(longest, o.longest);
+        wide |= o.wide;
+        twice |= o.twice;
+        levels = std::max(levels, o.levels);
+        near += o.near;
+        long_rows += o.long_rows;
+        waiting += o.waiting;
+        dist += o.dist;
+    }
     void install(MatPriv* pv, long long rows, long long seen) const {
         pv->max_row = longest;
         pv->banded = banded() && rows > 0;

@@ -364,14 +364,7 @@ int upload_concat(const int* n, const int* const* ia, const int* const* ja, cons
         int st = validate_host_csr(ia[q], ja[q], n[q], &own);
         if (st != SPTRSV_OK) return fail(st, "matrix " + std::to_string(q) + ": " + g_last_error);
         shapes->push_back(own);
-        shape.longest = std::max(shape.longest, own.longest);
-        shape.wide |= own.wide;
-        shape.twice |= own.twice;
-        shape.levels = std::max(shape.levels, own.levels);
-        shape.near += own.near;
-        shape.long_rows += own.long_rows;
-        shape.dist += own.dist;
-        shape.waiting += own.waiting;
+        shape.add(own);
         row_off[q + 1] = row_off[q] + n[q];
         nnz_off[q + 1] = nnz_off[q] + (n[q] > 0 ? (long long)ia[q][n[q]] - ia[q][0] : 0);
     }

@@ -269,3 +269,24 @@ def test_a_column_twice_keeps_both_products(prec, big):
         I.synchronize()
         assert relerr(dx.numpy(), np.tile(want, 2)) <= 1e-12
         bt.close()
+
+
+@pytest.mark.parametrize("offsets", [[1, 40], range(1, 10), [7, 300], [600, 900], []])
+def test_separate_matrix_of_a_tuned_batch(offsets):
+    """The members that stay sync-free, as a matrix of their own, whatever their
+    rows look like (grids, bands, far and no dependencies)."""
+    systems = []
+    for q in range(6):
+        ia, ja, a, b = matrix(1000 + 37 * q, offsets, seed=q)
+        a[ia[1:] - 1] = 0.6 if len(ja) > len(b) else 1.0     # not dominant: no Jacobi
+        systems.append(I.System(len(b), ia, ja, a, b))
+    ref = np.concatenate([O.fwd_f64(s.ia, s.ja, s.a, s.b) for s in systems])
+    bt = I.Batch(systems)
+    bt.tune(I.PREC_MIXED)
+    db, dx = I.DeviceArray.from_numpy(np.concatenate([s.b for s in systems])), I.DeviceArray(len(ref), np.float64)
+    for separate in (0, 1):
+        L.check(L.lib().sptrsv_batch_set_schedule(bt.h, 0, separate))
+        bt.solve(I.PREC_MIXED, db, dx)
+        I.synchronize()
+        assert bt.check() == 0 and relerr(dx.numpy(), ref) <= BARS[I.PREC_MIXED]
+    bt.close()
