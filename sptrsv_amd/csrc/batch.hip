@@ -667,8 +667,11 @@ namespace {
 struct TuneScratch {
     double* b = nullptr;
     double* x = nullptr;
+    int2* blocks = nullptr;  // of one member
+    int nblocks = 0;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     ~TuneScratch() {
+        if (blocks) (void)hipFree(blocks);
         if (b) (void)hipFree(b);
         if (x) (void)hipFree(x);
         if (e0) (void)hipEventDestroy(e0);
@@ -685,11 +688,17 @@ struct TuneScratch {
     }
 };
 
-// Mean time of `reps` sync-free solves of matrix m alone with `lanes`
-// lanes per row (after one untimed solve).
+// Mean time of `reps` sync-free solves of matrix m alone (after one untimed
+// solve), by the walk that solves it in the batch: in blocks, or as tasks with
+// `lanes` lanes per row.
 int time_member(sptrsv_batch_t* bt, TuneScratch& ts, int precision, int m, int lanes, int reps, float* ms) {
     std::vector<Task> tl;
-    matrix_tasks(bt, m, lanes, tl);
+    if (bt->band[m]) {
+        SPT_TRY(upload_blocks(bt, {m}, &ts.blocks, &ts.nblocks));
+    } else {
+        ts.nblocks = 0;
+        matrix_tasks(bt, m, lanes, tl);
+    }
     if ((int)tl.size() > bt->sub_cap) {
         if (bt->d_sub) (void)hipFree(bt->d_sub);
         bt->d_sub = nullptr;
@@ -697,11 +706,13 @@ int time_member(sptrsv_batch_t* bt, TuneScratch& ts, int precision, int m, int l
         SPT_HIP(hipMalloc(&bt->d_sub, sizeof(Task) * tl.size()));
         bt->sub_cap = (int)tl.size();
     }
-    SPT_HIP(hipMemcpy(bt->d_sub, tl.data(), sizeof(Task) * tl.size(), hipMemcpyHostToDevice));
-    SPT_TRY(batch_solve_tasks(bt, precision, bt->d_sub, (int)tl.size(), ts.b, ts.x, nullptr));
+    if (!tl.empty()) SPT_HIP(hipMemcpy(bt->d_sub, tl.data(), sizeof(Task) * tl.size(), hipMemcpyHostToDevice));
+    auto solve = [&]() {
+        return batch_solve_tasks(bt, precision, bt->d_sub, (int)tl.size(), ts.b, ts.x, nullptr, ts.blocks, ts.nblocks);
+    };
+    SPT_TRY(solve());
     SPT_HIP(hipEventRecord(ts.e0, nullptr));
-    for (int r = 0; r < reps; ++r)
-        SPT_TRY(batch_solve_tasks(bt, precision, bt->d_sub, (int)tl.size(), ts.b, ts.x, nullptr));
+    for (int r = 0; r < reps; ++r) SPT_TRY(solve());
     SPT_HIP(hipEventRecord(ts.e1, nullptr));
     SPT_HIP(hipEventSynchronize(ts.e1));
     SPT_HIP(hipEventElapsedTime(ms, ts.e0, ts.e1));
@@ -798,7 +809,7 @@ int tune_mixed(sptrsv_batch_t* bt, TuneScratch& ts) {
         bt->lanes[m] = ref;
         if (jall > 0 && bt->delta[m] > 0 && best > 0.5f * jall) {
             slow.push_back(m);  // Jacobi candidate: lanes do not move a latency-bound chain
-        } else {
+        } else if (!bt->band[m]) {
             for (int L : {std::max(1, ref / 2), std::min(64, ref * 2)}) {
                 if (L == ref) continue;
                 float ms = 0;
@@ -809,6 +820,8 @@ int tune_mixed(sptrsv_batch_t* bt, TuneScratch& ts) {
                 }
             }
             lanes_tuned[m] = 1;
+        } else {
+            lanes_tuned[m] = 1;  // no lanes in blocks
         }
         bt->t_sync[m] = best;
     }
@@ -941,7 +954,8 @@ int sptrsv_batch_tune(sptrsv_batch_t* bt, int precision, int tune) {
         }
         const int ref = lanes_rule(bt->avg[m]);
         float best = 1e30f;
-        for (int L = std::max(1, ref / 2); L <= std::min(64, ref * 2); L <<= 1) {
+        // (members in blocks have no lanes to search)
+        for (int L = bt->band[m] ? ref : std::max(1, ref / 2); L <= (bt->band[m] ? ref : std::min(64, ref * 2)); L <<= 1) {
             float ms = 0;
             SPT_TRY(time_member(bt, ts, precision, m, L, 2, &ms));
             if (ms < best) {

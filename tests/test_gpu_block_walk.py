@@ -290,3 +290,29 @@ def test_separate_matrix_of_a_tuned_batch(offsets):
         I.synchronize()
         assert bt.check() == 0 and relerr(dx.numpy(), ref) <= BARS[I.PREC_MIXED]
     bt.close()
+
+
+@pytest.mark.parametrize("prec", [I.PREC_F64, I.PREC_MIXED])
+def test_batch_tuner_times_the_walk_it_will_use(prec):
+    """A banded member takes some 40 ns a row in blocks and 800 as tasks, and is
+    never solved as tasks: no launch of the FP64 tuner's is as long as those (the
+    mixed one also tries the sync-free members as a matrix of their own, row by
+    row among others)."""
+    n = 20000
+    systems = []
+    for q, offsets in enumerate(([1, 2, 3], [1], [3, 400])):
+        ia, ja, a, b = matrix(n if q < 2 else 500, offsets, seed=q)
+        a[ia[1:] - 1] = 0.9                                  # not dominant: no Jacobi
+        systems.append(I.System(len(b), ia, ja, a, b))
+    ref = np.concatenate([O.fwd_f64(s.ia, s.ja, s.a, s.b) for s in systems])
+    bt = I.Batch(systems)
+    I.kernel_timer(2)
+    bt.tune(prec)
+    ms, launches = I.kernel_timer_read()
+    I.kernel_timer(0)
+    assert launches > 0 and (prec == I.PREC_MIXED or ms / launches < n * 0.2e-3)
+    db, dx = I.DeviceArray.from_numpy(np.concatenate([s.b for s in systems])), I.DeviceArray(len(ref), np.float64)
+    bt.solve(prec, db, dx)
+    I.synchronize()
+    assert bt.check() == 0 and relerr(dx.numpy(), ref) <= BARS[prec]
+    bt.close()
