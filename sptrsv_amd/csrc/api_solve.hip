@@ -697,6 +697,28 @@ static int ensure_level_copy(sp_mat_t* m, dfr_analysis_info_t* info) {
     return st;
 }
 
+// The lean path in place of a walk that cannot be taken, with what the caller
+// asked for in common.
+static sptrsv_config_t lean_instead(const sp_mat_t* m, const sptrsv_config_t& c, int k) {
+    sptrsv_config_t f = shape_for(m, c.kernel, k);
+    f.fused = c.fused;
+    f.window = c.window;
+    f.cu_waves = c.cu_waves;
+    f.split_rows = c.split_rows;
+    return f;
+}
+
+// The configuration that runs: the block walk needs short rows or a band, the
+// packed walk the layout, and a trace is written by the walks row by row.
+// Settled before any workspace is sized (the level walk's plan is not).
+static sptrsv_config_t settled(const sp_mat_t* m, const dfr_analysis_info_t* info, const sptrsv_config_t& c, int k) {
+    const MatPriv* pv = static_cast<const MatPriv*>(m->priv);
+    if ((c.variant >= 5 && pv->trace) || (c.variant == 6 && !packed_waves(info).base) ||
+        (c.variant == 5 && !pv->banded && pv->max_row > kBlockRow + 1))
+        return lean_instead(m, c, k);
+    return c;
+}
+
 struct LevelView {
     const sp_mat_t* mat;
     const int* row_orig;
@@ -721,15 +743,11 @@ static int run_pass(sp_mat_t* m, dfr_analysis_info_t* info, const sptrsv_config_
             if constexpr (std::is_same<P, PolMixed>::value) SPT_TRY(level_walk_mixed(m, info, b, x_out, s, timed, &done));
         }
         if (done) return SPTRSV_OK;
-        c = shape_for(m, c.kernel, k);
+        c = lean_instead(m, c, k);
         c.variant = 6;  // no plan: the packed walk needs none
     }
+    c = settled(m, info, c, k);
     const PackedWaves pw = c.variant == 6 ? packed_waves(info) : PackedWaves{};
-    // a trace is written by the walks row by row
-    if ((c.variant >= 5 && pv->trace) || (c.variant == 6 && !pw.base) ||
-        (c.variant == 5 && !pv->banded && pv->max_row > kBlockRow + 1)) {
-        c = shape_for(m, c.kernel, k);
-    }
     const sp_mat_t* sm = lv ? lv->mat : m;
     const int K = pow2_ceil(k);
     SolveArgs A{};
@@ -1141,7 +1159,7 @@ int sptrsv_solve_mixed_noalloc(sp_mat_t* mat, dfr_analysis_info_t* info, const s
         SPT_TRY(default_config(mat, info, SPTRSV_PREC_MIXED, k, &c));
     }
     c.fused = 1;
-    if (c.variant == 4) c = shape_for(mat, c.kernel, k);  // its plan is a per-analysis workspace
+    if (c.variant == 4) c = lean_instead(mat, c, k);  // its plan is a per-analysis workspace
     if (c.variant == 3)
         return fail(SPTRSV_E_INVALID_ARG, "the allocation-free solve does not run the in-degree walk (its "
                                           "counters are a per-matrix workspace)");
@@ -1152,6 +1170,8 @@ int sptrsv_solve_mixed_noalloc(sp_mat_t* mat, dfr_analysis_info_t* info, const s
                                               "copy is a per-matrix workspace)");
         c.reorder = 0;
     }
+    const bool packed = c.variant == 6;
+    c = settled(mat, info, c, k);
     // the published words, then (split long rows) the segment partials from
     // the next 256-byte boundary
     const size_t pub_words = (size_t)n * k;
@@ -1159,7 +1179,7 @@ int sptrsv_solve_mixed_noalloc(sp_mat_t* mat, dfr_analysis_info_t* info, const s
     const size_t part_at = (pub_words + 31) / 32 * 32;
     // only a solve that names MULTIROW, or an analysis made for it, asks for
     // split rows: others keep theirs whole where the partials find no room
-    if (part_at + part_words > (size_t)SPTRSV_NOALLOC_MAX_WORDS && c.variant == 6 &&
+    if (part_at + part_words > (size_t)SPTRSV_NOALLOC_MAX_WORDS && packed &&
         (c.kernel == SPTRSV_KERNEL_ORDER || (!named && info->mode == ALL))) {
         c.split_rows = -1;
         part_words = 0;
