@@ -961,8 +961,9 @@ __device__ __forceinline__ void fast_segment(const SolveArgs& A, int lane, int g
 // that gives a row fewer lanes than a row per wave has rounds more than that one
 // from more than 3 entries a lane on (8 lanes: 1.06 times its error at 32
 // entries, 1.2 at 64; one lane, 8 entries: 1.27; 3 entries a lane: 1.00).  Added
-// to the sum of the entries it is 0.75 to 0.9 times that, but a further add in
-// every hop (random n = 10^6, 8 lanes and entries: 2.06 -> 2.12 ms).
+// to the sum of the entries it is 0.75 to 0.9 times that.  The walks add it, or 0,
+// at the end of every row: a branch there cost the packed walk 5 % (random n =
+// 10^6 2.51 -> 2.62 ms; the add 0.5 %, 1 % in the group walk, 2.05 -> 2.08 ms).
 template <class P>
 __device__ __forceinline__ bool seed_first(int entries, int lanes) {
     return P::kExact || entries <= 3 * lanes;
@@ -990,6 +991,7 @@ __device__ __forceinline__ void level_rows(const SolveArgs& A, int L, int lane, 
     const Acc seed = lead ? P::seed(A, bi) : P::zero();
     const bool first = seed_first<P>(dpos - rs, L);
     Acc acc = first ? seed : P::zero();
+    const Acc last = first ? P::zero() : seed;
     typename P::Diag dg{};
     if (lead) dg = P::diag(A, dpos);
     const long long t0 = wall_clock64();
@@ -998,7 +1000,7 @@ __device__ __forceinline__ void level_rows(const SolveArgs& A, int L, int lane, 
     fold_entries<P, U, K>(A, L, e, lane, live, rs, dpos, acc, t0, expired, spins, r);
     Acc t = group_reduce<P, K>(acc, G);
     if (lead) {
-        if (!first) t = P::add(seed, t);
+        if (!P::kExact) t = P::add(last, t);
         typename P::Out o{};
         const word w = P::finish(A, dg, t, o);
         if (A.local) publish_near(&gpub[xi], w);
@@ -1168,6 +1170,7 @@ __device__ __forceinline__ void group_rows(const SolveArgs& A, int L, int lane, 
     const Acc seed = lead ? P::seed(A, (size_t)row) : P::zero();
     const bool first = seed_first<P>(dpos - (p - e), L);
     Acc acc = first ? seed : P::zero();
+    const Acc last = first ? P::zero() : seed;
     typename P::Diag dg{};
     if (lead) dg = P::diag(A, dpos);
     bool done = !(live && p < dpos), out = !live;
@@ -1198,7 +1201,7 @@ __device__ __forceinline__ void group_rows(const SolveArgs& A, int L, int lane, 
         if (__ballot(ready)) {
             Acc t = group_reduce<P, 1>(acc, L);
             if (ready && e == 0) {
-                if (!first) t = P::add(seed, t);
+                if (!P::kExact) t = P::add(last, t);
                 typename P::Out o{};
                 const word r = P::finish(A, dg, t, o);
                 publish<word, LOCAL>(&gpub[row], r);
