@@ -186,7 +186,7 @@ bool block_walk_fits(const sp_mat_t* m) {
 //  * Blocks of 64 rows where block_walk_fits says so.
 //  * Where rows depend on rows up to some thousands back, the group walk: a
 //    chain sets the pace, and one XCD's waves hold the rows that can be solved
-//    (nearest dependency 620 rows back, n = 10^6: 5.84 -> 2.04 ms against a row
+//    (nearest dependency 620 rows back, n = 10^6: 5.84 -> 2.08 ms against a row
 //    per wave on the whole device; 1340 back, n = 3*10^5: 875 -> 315 us).  Eight
 //    lanes a row serve rows of 4 to 40 entries within 8 % of the best; long
 //    rows take 32 (power-law n = 6000, 116 -> 80 us, 16 lanes 102; n = 9000, 1600
@@ -225,7 +225,7 @@ int group_walk_lanes(const sp_mat_t* m) {
 
 // Where and how wide the packed walk (variant 6) runs, by the waves of a level.
 // Up to 100 the 32 CUs of one XCD have enough to do: 29 to 46 waves (random, n =
-// 3*10^4 to 10^6) 129 us -> 2.47 ms against 245 us -> 4.93 ms on the whole device,
+// 3*10^4 to 10^6) 127 us -> 2.52 ms against 245 us -> 4.93 ms on the whole device,
 // 58 (power-law, n = 10^5) 199 against 254 us, 75 (3D grid 60^3) 165 against 248
 // us, but 145 (power-law, n = 3*10^5) 412 against 318 us.  With less than 20 waves
 // the fewer pollers hand over sooner (2D grid 1000^2, 17 waves: 1.08 ms with 4
@@ -251,9 +251,9 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 // four rows per level the block walk, which takes about 40 ns a row, the level
 // walk 170 to 200 ns a level (bandwidth 9, n = 5000: 0.21 ms against 1.00); and
 // where the packed walk would stay on one XCD, rows of up to 64 entries, but for a
-// few, the group walk, whose lanes read consecutive rows (random n = 10^6 2.04 against
-// 2.47 ms, n = 3*10^4 109 against 129 us; 20 entries of the last 3000, n =
-// 3*10^5, 2.45 against 2.81 ms).
+// few, the group walk, whose lanes read consecutive rows (random n = 10^6 2.08 against
+// 2.52 ms, n = 3*10^4 108 against 127 us; 20 entries of the last 3000, n =
+// 3*10^5, 2.50 against 2.94 ms).
 constexpr long long kChainRows = 4;
 bool chain_of(const sp_mat_t* m, const dfr_analysis_info_t* info) {
     return info && static_cast<const MatPriv*>(m->priv)->banded && m->nr < kChainRows * info->nlevs;

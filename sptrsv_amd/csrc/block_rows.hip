@@ -5,15 +5,15 @@
 // waits for first.  Through memory that costs 0.65 to 0.8 us a row, and a walk
 // with one row per wave has 8192 rows in flight, less than one plane of a large
 // grid.  Here a solved row reaches the rest of its block with v_readlane, so a
-// row costs 30 ns (banded kernel) or 165 ns (short rows), and 64 times as many
+// row costs 32 ns (banded kernel) or 165 ns (short rows), and 64 times as many
 // rows are in flight.  What bounds it then is the chain of blocks: for a band,
 // 64 steps and one hand-off through memory per block; for a grid, a hand-off
 // per line of the grid.
 //
 // Measured (natural-order solve, before -> now): bandwidth 17, n = 50000 39.3 ->
-// 2.04 ms, bandwidth 60 41 -> 2.36 ms; 3D grid 101^3 FP32 8.7 -> 0.57 ms, 31^3
-// 216 -> 111 us; 2D grid 707^2 19.5 -> 1.40 ms, 200^2 657 -> 354 us, 64^2 130 ->
-// 114 us.
+// 2.13 ms, bandwidth 60 41 -> 2.43 ms; 3D grid 101^3 FP32 8.7 -> 0.57 ms, 31^3
+// 216 -> 107 us; 2D grid 707^2 19.5 -> 1.41 ms, 200^2 657 -> 358 us, 64^2 130 ->
+// 111 us.
 #include <type_traits>
 
 #include "syncfree.hpp"
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(64) void k_block_short(SolveArgs A) {
 // reciprocal diagonal, two readlanes, a multiply-add and an add; rows are
 // published eight at a time.  A wave whose predecessor has published nothing yet sleeps
 // between polls: 500 waves spinning made every hand-off slower (n = 50000 3.09
-// -> 2.04 ms).
+// -> 2.04 ms, with one sum a row).
 // blocks (of several matrices in one): first row and the matrix's end row of
 // each block, else the blocks of one matrix in order.
 template <class P>

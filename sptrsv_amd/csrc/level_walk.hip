@@ -32,15 +32,15 @@
 // The words of at least the last 8192 positions are in an LDS ring (128 KB for
 // 8-byte words).  An entry that reaches further back (far) has a record of its
 // own and reads the words in memory (x itself, or for the fused mixed pass a
-// copy of the words); a full barrier every 4096 positions makes sure that those
-// have been written.  Entries for which a lane has no record left are in an
+// copy of the words), written at least 4096 positions and a full barrier before
+// (see the end of a step).  Entries for which a lane has no record left are in an
 // overflow list of their slice.
 //
 // Measured (default shape of csr_L_solve_order / _multirow before -> now): 2D
-// grid factor of 64^2 (127 levels) 120 -> 27 us, of 250^2 516 -> 125 us, random
-// n = 2000 95 -> 23 us and 15000 203 -> 110 us, bandwidth 9 with one row per
-// level n = 5000 3.74 -> 1.00 ms: 0.15 to 0.2 us a level while a step is one or
-// two slices, 0.55 us with eight (the CU then takes in about 65 GB/s).
+// grid factor of 64^2 (127 levels) 120 -> 27 us, of 250^2 516 -> 130 us, 3D grid
+// 15^3 54 -> 21 us, random n = 2000 95 -> 31 us: 0.15 to 0.2 us a level while a
+// step is one or two slices, 0.55 us with eight (the CU then takes in about 65
+// GB/s), and 5 us for the launch that writes the records.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -521,7 +521,14 @@ __global__ __launch_bounds__(WG) void k_level_walk(LwArgs A) {
         lw_store(r_x, ~row[j2].y, xv);
         if constexpr (FAR && MIXED) lw_store(r_pub, ~row[j2].y, __builtin_bit_cast(Num, res));
         if (FAR && (ent[j2] & kLwStepFlush)) {
-            __syncthreads();  // the words stored so far are in memory, for far entries
+            // A step that enters a new epoch: the words of the epoch before the one
+            // just left are in memory for every wave.  The barrier alone does not
+            // wait for stores; each wave has, in the steps of a whole epoch (at
+            // least eight, of at most 512 rows), waited for loads it issued after
+            // them, and vector memory operations of a wave are counted in order.
+            // A far entry is more than an epoch back when its load goes out, D
+            // steps ahead (lw_near).
+            __syncthreads();
         } else {
             // results reach the other waves through LDS: wait for LDS only
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");

@@ -1150,8 +1150,8 @@ __device__ __forceinline__ int claim_block(int* ctr, int items_per_block, int* s
 // inside the polling loop: a row does not wait for the others of its wave, and
 // may depend on them.  A lane polls one entry at a time, in storage order, which
 // keeps a polling turn to some 20 instructions.  Packed walk on one XCD with the
-// wave's rows published together -> each on its own: random n = 10^6 2.77 -> 2.47
-// ms; in natural order (8 rows a wave) 2.04 ms, 0.52 us a level, of which a
+// wave's rows published together -> each on its own: random n = 10^6 2.77 -> 2.52
+// ms; in natural order (8 rows a wave) 2.08 ms, 0.53 us a level, of which a
 // hand-off through the L2 takes 0.21.
 template <class P, bool LOCAL>
 __device__ __forceinline__ void group_rows(const SolveArgs& A, int L, int lane, int row) {
@@ -1236,7 +1236,7 @@ __device__ __forceinline__ bool on_chosen_xcd(const SolveArgs& A, int* s_slot) {
 // store going to memory and the poll past the L2; inside one XCD a plain store
 // is in the L2 that every CU polls, and it takes 211 ns.  Where the rows of a
 // level keep 32 CUs busy and no more, that is what counts (MULTIROW solve, whole
-// device -> one XCD: random n = 10^6, 253 rows per level, 4.93 -> 2.47 ms; n =
+// device -> one XCD: random n = 10^6, 253 rows per level, 4.93 -> 2.52 ms; n =
 // 30000 245 -> 129 us).  In natural order (MODE 0) an item is the 64 / L rows of
 // a wave.
 template <class P, int WG, int U, int MODE, bool LOCAL = false>
