@@ -186,7 +186,7 @@ bool block_walk_fits(const sp_mat_t* m) {
 //  * Blocks of 64 rows where block_walk_fits says so.
 //  * Where rows depend on rows up to some thousands back, the group walk: a
 //    chain sets the pace, and one XCD's waves hold the rows that can be solved
-//    (nearest dependency 620 rows back, n = 10^6: 5.84 -> 2.08 ms against a row
+//    (nearest dependency 620 rows back, n = 10^6: 5.84 -> 2.07 ms against a row
 //    per wave on the whole device; 1340 back, n = 3*10^5: 875 -> 315 us).  Eight
 //    lanes a row serve rows of 4 to 40 entries within 8 % of the best; long
 //    rows take 32 (power-law n = 6000, 116 -> 80 us, 16 lanes 102; n = 9000, 1600
@@ -251,7 +251,7 @@ static PackedShape packed_shape(int n_waves, int nlevs) {
 // four rows per level the block walk, which takes about 40 ns a row, the level
 // walk 170 to 200 ns a level (bandwidth 9, n = 5000: 0.21 ms against 1.00); and
 // where the packed walk would stay on one XCD, rows of up to 64 entries, but for a
-// few, the group walk, whose lanes read consecutive rows (random n = 10^6 2.08 against
+// few, the group walk, whose lanes read consecutive rows (random n = 10^6 2.07 against
 // 2.52 ms, n = 3*10^4 108 against 127 us; 20 entries of the last 3000, n =
 // 3*10^5, 2.50 against 2.94 ms).
 constexpr long long kChainRows = 4;

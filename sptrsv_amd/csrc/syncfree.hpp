@@ -957,16 +957,17 @@ __device__ __forceinline__ void fast_segment(const SolveArgs& A, int lane, int g
 }
 
 // Where the right-hand side of a row enters its sum.  From the start, in the
-// first lane, it makes every partial sum of that lane as large as itself: a walk
-// that gives a row fewer lanes than a row per wave has rounds more than that one
-// from more than 3 entries a lane on (8 lanes: 1.06 times its error at 32
-// entries, 1.2 at 64; one lane, 8 entries: 1.27; 3 entries a lane: 1.00).  Added
-// to the sum of the entries it is 0.75 to 0.9 times that.  The walks add it, or 0,
+// first lane, it makes every partial sum of that lane and every step of the
+// reduction as large as itself: a walk that gives a row other lanes than a row
+// per wave has then rounds more than that one (8 lanes: 1.06 times its error at
+// 32 entries, 1.2 at 64; one lane, 8 entries: 1.27; 32 lanes for rows of 10: 1.1).
+// Added to the sum of the entries it is 0.7 to 0.9 times that.  A row of one
+// entry has it from the start: one rounding either way.  The walks add it, or 0,
 // at the end of every row: a branch there cost the packed walk 5 % (random n =
-// 10^6 2.51 -> 2.62 ms; the add 0.5 %, 1 % in the group walk, 2.05 -> 2.08 ms).
+// 10^6 2.51 -> 2.62 ms; the add 0.5 %, in the group walk too, 2.06 -> 2.07 ms).
 template <class P>
-__device__ __forceinline__ bool seed_first(int entries, int lanes) {
-    return P::kExact || entries <= 3 * lanes;
+__device__ __forceinline__ bool seed_first(int entries) {
+    return P::kExact || entries <= 1;
 }
 
 // Rows of one level, several right-hand sides: a group of L entry lanes x K
@@ -989,7 +990,7 @@ __device__ __forceinline__ void level_rows(const SolveArgs& A, int L, int lane, 
     const size_t xi = (size_t)(live ? row : 0) * A.k + r;
     const size_t bi = live ? caller_index(A, row, r) : 0;
     const Acc seed = lead ? P::seed(A, bi) : P::zero();
-    const bool first = seed_first<P>(dpos - rs, L);
+    const bool first = seed_first<P>(dpos - rs);
     Acc acc = first ? seed : P::zero();
     const Acc last = first ? P::zero() : seed;
     typename P::Diag dg{};
@@ -1151,7 +1152,7 @@ __device__ __forceinline__ int claim_block(int* ctr, int items_per_block, int* s
 // may depend on them.  A lane polls one entry at a time, in storage order, which
 // keeps a polling turn to some 20 instructions.  Packed walk on one XCD with the
 // wave's rows published together -> each on its own: random n = 10^6 2.77 -> 2.52
-// ms; in natural order (8 rows a wave) 2.08 ms, 0.53 us a level, of which a
+// ms; in natural order (8 rows a wave) 2.07 ms, 0.52 us a level, of which a
 // hand-off through the L2 takes 0.21.
 template <class P, bool LOCAL>
 __device__ __forceinline__ void group_rows(const SolveArgs& A, int L, int lane, int row) {
@@ -1168,7 +1169,7 @@ __device__ __forceinline__ void group_rows(const SolveArgs& A, int L, int lane, 
         dpos = A.ia[row + 1] - 1;
     }
     const Acc seed = lead ? P::seed(A, (size_t)row) : P::zero();
-    const bool first = seed_first<P>(dpos - (p - e), L);
+    const bool first = seed_first<P>(dpos - (p - e));
     Acc acc = first ? seed : P::zero();
     const Acc last = first ? P::zero() : seed;
     typename P::Diag dg{};

@@ -86,3 +86,10 @@ def test_several_right_hand_sides(entries):
     got, bar = errors(ia, ja, a, 16, [dict(kernel=I.KERNEL_ORDER, lanes=1, variant=2, cu_waves=16),
                                       dict(kernel=I.KERNEL_SIMPLE, lanes=4, variant=0)], I.ORDER)
     assert got <= bar
+
+
+def test_group_walk_with_more_lanes_than_entries():
+    ia, ja, a = matrix(10, 1500, False)
+    got, bar = errors(ia, ja, a, 1, [dict(kernel=I.KERNEL_SIMPLE, lanes=32, variant=7),
+                                     dict(kernel=I.KERNEL_SIMPLE, lanes=default_lanes(ia), variant=1)], I.ORDER)
+    assert got <= bar
